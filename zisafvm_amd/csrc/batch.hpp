@@ -109,7 +109,7 @@ ZFV_HD void kb_face_flux_thread(const DevInst *insts, BlockRef b, int t) {
 // the SSP3 stage update of thread t's cell (256 cells per block):
 // K[stage] = L(U_stage), U_next = U0 + dt sum_j c_j K[j]
 // (src/zisa/ode/runge_kutta.cpp:122-165), then the frozen BC
-template <int DIM>
+template <int DIM, bool AOS = false>
 ZFV_HD void kb_update_thread(DevInst *insts, BlockRef b, int t, int stage) {
   constexpr int NV = DIM + 2;
   if (b.inst < 0) return;
@@ -136,41 +136,44 @@ ZFV_HD void kb_update_thread(DevInst *insts, BlockRef b, int t, int stage) {
   double *Un = stage == 2 ? d.U : d.X;
   if (m.steady != nullptr && (m.meta[i] & META_FAR_GHOST) == META_FAR_GHOST) {
     for (int v = 0; v < NV; ++v) {
-      d.K[(int64_t(stage) * NV + v) * n + i] = 0.0;
-      Un[v * n + i] = m.steady[v * n + i];
+      const int64_t at = state_at<AOS, NV>(n, v, i);
+      d.K[int64_t(stage) * NV * n + at] = 0.0;
+      Un[at] = m.steady[at];
     }
     return;
   }
   double L[NV];
-  cell_rate<DIM>(m, i, Us, d.G, d.src, L);
+  cell_rate<DIM, AOS>(m, i, Us, d.G, d.src, L);
   // SSP3 next-state coefficients (src/zisa/ode/runge_kutta.cpp:154-165)
   const double c0 = stage == 0 ? 1.0 : (stage == 1 ? 0.25 : 1.0 / 6);
   const double c1 = stage == 1 ? 0.25 : 1.0 / 6;
   const double c2 = 2.0 / 3;
   const bool ghost = (m.meta[i] & 16) != 0 && m.steady != nullptr;
+  const double *K0 = d.K, *K1 = d.K + int64_t(NV) * n;
   for (int v = 0; v < NV; ++v) {
-    if (stage < 2) d.K[(int64_t(stage) * NV + v) * n + i] = L[v];  // the last stage's is read by no later one
+    const int64_t at = state_at<AOS, NV>(n, v, i);
+    if (stage < 2) d.K[int64_t(stage) * NV * n + at] = L[v];  // the last stage's is read by no later one
     double dudt = 0.0;
     if (stage == 0) {
       dudt += c0 * L[v];
     } else if (stage == 1) {
-      dudt += c0 * d.K[(int64_t(0) * NV + v) * n + i];
+      dudt += c0 * K0[at];
       dudt += c1 * L[v];
     } else {
-      dudt += c0 * d.K[(int64_t(0) * NV + v) * n + i];
-      dudt += c1 * d.K[(int64_t(1) * NV + v) * n + i];
+      dudt += c0 * K0[at];
+      dudt += c1 * K1[at];
       dudt += c2 * L[v];
     }
-    double un = d.U[v * n + i] + dt * dudt;
-    if (ghost) un = m.steady[v * n + i];
-    Un[v * n + i] = un;
+    double un = d.U[at] + dt * dudt;
+    if (ghost) un = m.steady[at];
+    Un[at] = un;
   }
 }
 
 // LocalCFL candidate of thread t's cell, inradius / (|v| + a), or 1e300
 // past the instance's cells; 0 for a NaN or non-positive state
 // (include/zisa/model/local_cfl_condition_impl.hpp:25-40)
-template <int DIM>
+template <int DIM, bool AOS = false>
 ZFV_HD double kb_cfl_thread(const DevInst &d, BlockRef b, int t) {
   constexpr int NV = DIM + 2;
   const int64_t i = int64_t(b.local) * 256 + t;
@@ -179,7 +182,7 @@ ZFV_HD double kb_cfl_thread(const DevInst &d, BlockRef b, int t) {
   if (i < m.n) {
     const int64_t n = m.n;
     double u[NV];
-    for (int v = 0; v < NV; ++v) u[v] = d.U[v * n + i];
+    for (int v = 0; v < NV; ++v) u[v] = d.U[state_at<AOS, NV>(n, v, i)];
     double m2 = u[1] * u[1] + u[2] * u[2];
     if (DIM == 3) m2 += u[3] * u[3];
     double v2 = m2 / (u[0] * u[0]);

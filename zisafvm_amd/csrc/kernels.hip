@@ -1,7 +1,7 @@
 // gfx950 kernels of the rate-of-change hot path and the C-ABI of
 // libzfv_hip.so (declared in include/zfv.h).
 //
-// One SSP3 stage = three launches over SoA arrays in HBM:
+// One SSP3 stage = three launches over arrays in HBM:
 //   k_reconstruct  one group of nvars lanes per cell (lane g: variable g):
 //                  stencil gather, LSQ pseudo-inverse mat-vecs, CWENO/WENO-AO,
 //                  equilibrium solve (well-balanced), point values on the
@@ -55,6 +55,7 @@ __device__ __forceinline__ int64_t xcd_block(unsigned b, unsigned grid) {
 // Cross-lane exchange inside a group of NV consecutive lanes of a wavefront
 // (one cell per group; lane g of the group owns conserved variable g).
 struct WaveGroup {
+  static constexpr bool kAos = true;  // state-shaped arrays keep a cell's values together (state_at)
   int base;       // first lane of the group
   double *slice;  // the group's LDS slice
   double *wave;   // the wavefront's row region
@@ -163,29 +164,29 @@ __global__ __launch_bounds__(256) void k_update(Img m, StageCoeffs sc, int stage
   if (!sc.write_rate_only && m.steady != nullptr && (m.meta[i] & META_FAR_GHOST) == META_FAR_GHOST) {
     // frozen far ghost: its tendency is never used
     for (int v = 0; v < NV; ++v) {
-      K[(int64_t(stage) * NV + v) * n + i] = 0.0;
-      Unext[v * n + i] = m.steady[v * n + i];
+      K[(int64_t(stage) * n + i) * NV + v] = 0.0;
+      Unext[i * NV + v] = m.steady[i * NV + v];
     }
     return;
   }
   double L[NV];
-  cell_rate<DIM>(m, i, Ustage, G, src, L);
+  cell_rate<DIM, true>(m, i, Ustage, G, src, L);
   // the last stage's tendency enters only its own sum (no later stage reads it)
   if (sc.write_rate_only || stage + 1 < 3)
-    for (int v = 0; v < NV; ++v) K[(int64_t(stage) * NV + v) * n + i] = L[v];
+    for (int v = 0; v < NV; ++v) K[(int64_t(stage) * n + i) * NV + v] = L[v];
   if (sc.write_rate_only) return;
   const bool ghost = (m.meta[i] & 16) != 0 && m.steady != nullptr;
   for (int v = 0; v < NV; ++v) {
     double dudt = 0.0;
     for (int j = 0; j < sc.nk; ++j) {
       if (sc.c[j] != 0.0) {
-        const double kj = (j == stage) ? L[v] : K[(int64_t(j) * NV + v) * n + i];
+        const double kj = (j == stage) ? L[v] : K[(int64_t(j) * n + i) * NV + v];
         dudt += sc.c[j] * kj;
       }
     }
-    double un = U0[v * n + i] + dt * dudt;
-    if (ghost) un = m.steady[v * n + i];
-    Unext[v * n + i] = un;
+    double un = U0[i * NV + v] + dt * dudt;
+    if (ghost) un = m.steady[i * NV + v];
+    Unext[i * NV + v] = un;
   }
 }
 
@@ -199,7 +200,7 @@ __global__ __launch_bounds__(256) void k_cfl(Img m, const double *__restrict__ U
   // grid-stride over the cells: few blocks, so few atomics on one word
   for (int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x; i < n; i += int64_t(gridDim.x) * blockDim.x) {
     double u[NV];
-    for (int v = 0; v < NV; ++v) u[v] = U[v * n + i];
+    for (int v = 0; v < NV; ++v) u[v] = U[i * NV + v];
     double m2 = u[1] * u[1] + u[2] * u[2];
     if (DIM == 3) m2 += u[3] * u[3];
     double v2 = m2 / (u[0] * u[0]);
@@ -315,7 +316,7 @@ __global__ __launch_bounds__(256) void kb_face_flux(const DevInst *insts, const 
 
 template <int DIM>
 __global__ __launch_bounds__(256) void kb_update(DevInst *insts, const BlockRef *blk, int stage) {
-  kb_update_thread<DIM>(insts, blk[blockIdx.x], threadIdx.x, stage);
+  kb_update_thread<DIM, true>(insts, blk[blockIdx.x], threadIdx.x, stage);
 }
 
 template <int DIM>
@@ -324,7 +325,7 @@ __global__ __launch_bounds__(256) void kb_cfl(DevInst *insts, const BlockRef *bl
   if (b.inst < 0) return;  // the whole block shares b: it leaves together
   DevInst &d = insts[b.inst];
   if (!d.active) return;
-  double r = kb_cfl_thread<DIM>(d, b, threadIdx.x);
+  double r = kb_cfl_thread<DIM, true>(d, b, threadIdx.x);
   for (int off = 32; off > 0; off >>= 1) r = fmin(r, __shfl_down(r, off, 64));
   __shared__ double wmin[4];
   const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
@@ -374,11 +375,14 @@ __global__ __launch_bounds__(256) void k_adv_backup(const AdvState *a, int64_t c
 }
 
 // RejectLargeDensityChange::check: |rho1 - rho0| > drho_crit rho0 in any cell
-__global__ __launch_bounds__(256) void k_adv_check(AdvState *a, int64_t n, const double *U, const double *Ubk) {
+// (the density is the first of a cell's nv values)
+__global__ __launch_bounds__(256) void k_adv_check(AdvState *a, int64_t n, int nv, const double *U,
+                                                   const double *Ubk) {
   if (!(a->drho_crit > 0.0) || !a->active) return;
   const int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
   if (i >= n) return;
-  if (fabs(Ubk[i] - U[i]) > a->drho_crit * Ubk[i]) atomicOr(&a->bad, 1);
+  const double r0 = Ubk[i * nv], r1 = U[i * nv];
+  if (fabs(r0 - r1) > a->drho_crit * r0) atomicOr(&a->bad, 1);
 }
 
 // a rejected step leaves the state as it was
@@ -791,8 +795,8 @@ static void enqueue_adaptive_step(zfv_handle *h, bool reject, int cfg, AdvState 
     Us = h->X;
   }
   if (reject) {
-    // density is the first SoA plane of U
-    hipLaunchKernelGGL(k_adv_check, dim3(blocks_for(m.n, 256)), dim3(256), 0, h->stream, adv, m.n, h->U, Ubk);
+    hipLaunchKernelGGL(k_adv_check, dim3(blocks_for(m.n, 256)), dim3(256), 0, h->stream, adv, m.n, h->img.s.nvars,
+                       h->U, Ubk);
     hipLaunchKernelGGL(k_adv_restore, dim3(blocks_for(count, 256)), dim3(256), 0, h->stream, adv, count, h->U, Ubk);
   }
   hipLaunchKernelGGL(k_adv_end, dim3(1), dim3(1), 0, h->stream, adv);
@@ -850,12 +854,6 @@ static unsigned char *scratch_on(int dev) {
     g_scratch_dev[dev] = p;
   }
   return static_cast<unsigned char *>(g_scratch_dev[dev]);
-}
-
-static void to_soa(const zfv_handle *h, const double *aos, double *soa) { zfv::to_soa(h->img, aos, soa); }
-
-static void from_soa(const zfv_handle *h, const double *soa, double *aos, bool accumulate) {
-  zfv::from_soa(h->img, soa, aos, accumulate);
 }
 
 // launch configuration named by its threads per block
@@ -1085,7 +1083,7 @@ int zfv_destroy(zfv_handle *h) {
 int zfv_set_state(zfv_handle *h, const double *cvars) {
   ZFV_API_BEGIN
   member_settle(h);
-  to_soa(h, cvars, h->host_stage);
+  to_cells(h->img, cvars, h->host_stage);
   const size_t bytes = sizeof(double) * h->img.s.nvars * h->img.n;
   HIP_CHECK(hipMemcpyAsync(h->U, h->host_stage, bytes, hipMemcpyHostToDevice, h->stream));
   HIP_CHECK(hipStreamSynchronize(h->stream));
@@ -1099,7 +1097,7 @@ int zfv_get_state(zfv_handle *h, double *cvars) {
   const size_t bytes = sizeof(double) * h->img.s.nvars * h->img.n;
   HIP_CHECK(hipMemcpyAsync(h->host_stage, h->U, bytes, hipMemcpyDeviceToHost, h->stream));
   HIP_CHECK(hipStreamSynchronize(h->stream));
-  from_soa(h, h->host_stage, cvars, false);
+  from_cells(h->img, h->host_stage, cvars, false);
   return ZFV_OK;
   ZFV_API_END
 }
@@ -1134,7 +1132,7 @@ int zfv_snapshot_end(zfv_handle *h, double *cvars) {
   if (!h->snap_pending) throw ZfvError(ZFV_ERR_INVALID, "no snapshot pending");
   h->snap_pending = false;
   HIP_CHECK(hipStreamSynchronize(h->copy_stream));
-  from_soa(h, h->snap_host, cvars, false);
+  from_cells(h->img, h->snap_host, cvars, false);
   return ZFV_OK;
   ZFV_API_END
 }
@@ -1145,7 +1143,7 @@ int zfv_set_steady_state(zfv_handle *h, const double *cvars) {
   const int64_t n = h->img.n;
   const int nv = h->img.s.nvars;
   if (!h->steady) h->steady = h->alloc<double>(size_t(nv) * n);
-  to_soa(h, cvars, h->host_stage);
+  to_cells(h->img, cvars, h->host_stage);
   HIP_CHECK(hipMemcpyAsync(h->steady, h->host_stage, sizeof(double) * nv * n, hipMemcpyHostToDevice, h->stream));
   HIP_CHECK(hipStreamSynchronize(h->stream));
   h->dimg.steady = h->steady;
@@ -1161,7 +1159,7 @@ int zfv_rate(zfv_handle *h, const double *u, double *dudt, double t) {
   member_settle(h);
   const int64_t n = h->img.n;
   const int nv = h->img.s.nvars;
-  to_soa(h, u, h->host_stage);
+  to_cells(h->img, u, h->host_stage);
   HIP_CHECK(hipMemcpyAsync(h->X, h->host_stage, sizeof(double) * nv * n, hipMemcpyHostToDevice, h->stream));
   const Img &m = h->dimg;
   h->L.rec[h->ph](m, h->X, h->fpv, h->src, rec_config(h, h->X), 0, h->stream);
@@ -1172,7 +1170,7 @@ int zfv_rate(zfv_handle *h, const double *u, double *dudt, double t) {
   HIP_CHECK(hipGetLastError());
   HIP_CHECK(hipMemcpyAsync(h->host_stage, h->K, sizeof(double) * nv * n, hipMemcpyDeviceToHost, h->stream));
   HIP_CHECK(hipStreamSynchronize(h->stream));
-  from_soa(h, h->host_stage, dudt, true);
+  from_cells(h->img, h->host_stage, dudt, true);
   return ZFV_OK;
   ZFV_API_END
 }

@@ -1180,4 +1180,48 @@ void from_soa(const HostImage &img, const double *soa, double *aos, bool accumul
   }
 }
 
+namespace {
+template <int DIM>
+void to_cells_dim(const HostImage &img, const double *aos, double *cells) {
+  constexpr int NV = DIM + 2;
+  const int64_t n = img.n;
+  const int32_t *perm = img.perm.data();
+#pragma omp parallel for schedule(static)
+  for (int64_t ip = 0; ip < n; ++ip) {
+    const double *u = aos + 5 * int64_t(perm[ip]);
+    double *c = cells + NV * ip;
+    for (int d = 0; d < DIM + 1; ++d) c[d] = u[d];
+    c[NV - 1] = u[4];
+  }
+}
+
+template <int DIM, bool ACCUMULATE>
+void from_cells_dim(const HostImage &img, const double *cells, double *aos) {
+  constexpr int NV = DIM + 2;
+  const int64_t n = img.n;
+  const int32_t *perm = img.perm.data();
+  // perm is a permutation: every iteration writes its own row
+#pragma omp parallel for schedule(static)
+  for (int64_t ip = 0; ip < n; ++ip) {
+    double *u = aos + 5 * int64_t(perm[ip]);
+    const double *c = cells + NV * ip;
+    double w[5] = {c[0], 0.0, 0.0, 0.0, c[NV - 1]};
+    for (int d = 0; d < DIM; ++d) w[1 + d] = c[1 + d];
+    for (int v = 0; v < 5; ++v) u[v] = ACCUMULATE ? u[v] + w[v] : w[v];
+  }
+}
+}  // namespace
+
+void to_cells(const HostImage &img, const double *aos, double *cells) {
+  if (img.s.dim == 2) to_cells_dim<2>(img, aos, cells);
+  else to_cells_dim<3>(img, aos, cells);
+}
+
+void from_cells(const HostImage &img, const double *cells, double *aos, bool accumulate) {
+  if (img.s.dim == 2 && accumulate) from_cells_dim<2, true>(img, cells, aos);
+  else if (img.s.dim == 2) from_cells_dim<2, false>(img, cells, aos);
+  else if (accumulate) from_cells_dim<3, true>(img, cells, aos);
+  else from_cells_dim<3, false>(img, cells, aos);
+}
+
 }  // namespace zfv

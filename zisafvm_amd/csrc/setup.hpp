@@ -101,5 +101,9 @@ bool volume_mean_is_constant_term(const zfv_params &p, const Shape &s);
 // index), on the host's threads.  from_soa adds into aos when accumulate.
 void to_soa(const HostImage &img, const double *aos, double *soa);
 void from_soa(const HostImage &img, const double *soa, double *aos, bool accumulate);
+// The same with the kernels' layout: nvars values per cell in product order
+// (state_at with AOS).
+void to_cells(const HostImage &img, const double *aos, double *cells);
+void from_cells(const HostImage &img, const double *cells, double *aos, bool accumulate);
 
 }  // namespace zfv

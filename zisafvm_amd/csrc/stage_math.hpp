@@ -21,6 +21,7 @@
 // emulation, whatever the surrounding code.
 
 #include <cstdint>
+#include <type_traits>
 
 #if defined(__HIPCC__)
 #include <hip/hip_runtime.h>
@@ -57,7 +58,7 @@ struct Img {
   const int32_t *cface;  // per cell its face words, 4 int32 (one 16-byte load; 2D's fourth unused)
   const int32_t *fslot;  // ne pairs: cell-face slots of each interior face's left and right cell
   const uint32_t *fperm;
-  const double *steady;  // nvars * n (ghost cells only are read)
+  const double *steady;  // as the state (ghost cells only are read)
   const double *phim;    // n pairs: cell mean of phi and of (phi - mean)^2 (one 16-byte load), or null
   const double *pot;     // potential tables of the cell's own points (pot_index), or null
   const double *frm;     // face frames of the cells' local faces (load_face_frame)
@@ -109,6 +110,24 @@ ZFV_HD double sqr(double x) { return x * x; }
 
 ZFV_HD double dmin(double a, double b) { return a < b ? a : b; }
 ZFV_HD double dmax(double a, double b) { return a > b ? a : b; }
+
+// Where variable v of cell i stands in a state-shaped array (state, stage
+// state, tendencies, source, steady state).  The kernels keep the NV values of
+// a cell together (AOS): a stencil member's state is then one 32- or 40-byte
+// piece that its group's lanes fetch side by side, where planes cost one cache
+// line per variable and member.  The planes (v * n + i) are the layout of the
+// host emulation.
+template <bool AOS, int NV>
+ZFV_HD int64_t state_at(int64_t n, int v, int64_t i) {
+  return AOS ? i * NV + v : int64_t(v) * n + i;
+}
+
+// which of the two a lane exchange type's instances use: planes unless the
+// type says otherwise (static constexpr bool kAos)
+template <class X, class = void>
+struct state_is_aos : std::false_type {};
+template <class X>
+struct state_is_aos<X, std::void_t<decltype(X::kAos)>> : std::bool_constant<X::kAos> {};
 
 // two adjacent doubles, one 16-byte load
 struct alignas(16) PPair {
@@ -808,9 +827,9 @@ ZFV_HD void rusanov(const double *uL, const double *uR, double gamma, double *f)
 //   - the face-frame rotation and the gravity source mix momentum components.
 // Every call of bcast sits in control flow that is uniform over the group.
 //
-// U: state, nvars x n SoA.  fpv: per cell-face slot (i * NF + f) its Q x NV
+// U: state (state_at).  fpv: per cell-face slot (i * NF + f) its Q x NV
 // point values, written for interior faces (one group writes its cell's whole
-// block, so cache lines fill within one XCD).  src: nvars x n or null.
+// block, so cache lines fill within one XCD).  src: as the state, or null.
 // LDS of one wavefront: first a row region of wave_lds_doubles holding each
 // group's NV pseudo-inverse rows of NC entries (group c at c NV NC: a stride
 // of NV NC doubles keeps the groups' reads on different banks), then per
@@ -851,12 +870,13 @@ ZFV_HD void reconstruct_lane(const Img &m, int64_t i, const int g, X &xch, const
   constexpr int NC = DOFC - 1;
   constexpr int NBC = DIM;
   constexpr int DEGC = deg_of<DIM>(DOFC);
+  constexpr bool AOS = state_is_aos<X>::value;
   const int64_t n = m.n;
   const double gamma = m.gamma;
 
   // own state and scale (include/zisa/model/characteristic_scale.hpp:23-32)
   double u0[NV];
-  for (int v = 0; v < NV; ++v) u0[v] = U[v * n + i];
+  for (int v = 0; v < NV; ++v) u0[v] = U[state_at<AOS, NV>(n, v, i)];
   double msq = u0[1] * u0[1] + u0[2] * u0[2];
   if (DIM == 3) msq += u0[3] * u0[3];
   const double rho0 = u0[0];
@@ -876,7 +896,7 @@ ZFV_HD void reconstruct_lane(const Img &m, int64_t i, const int g, X &xch, const
   const int32_t rw_pre1 = NV + g < R_ALL ? m.rows[(NV + g) * n + i] : int32_t(0);
   double uk_pre[NV];
   if (DIM == 3)
-    for (int k = 0; k < NV; ++k) uk_pre[k] = U[g * n + (xch.bcast_i(rw_pre0, k) & ROW_CELL_MASK)];
+    for (int k = 0; k < NV; ++k) uk_pre[k] = U[state_at<AOS, NV>(n, g, xch.bcast_i(rw_pre0, k) & ROW_CELL_MASK)];
 
   double vtx[DIM + 1][3];
   load_corners<DIM>(m, i, vtx);
@@ -1234,7 +1254,8 @@ ZFV_HD void reconstruct_lane(const Img &m, int64_t i, const int g, X &xch, const
       const bool mine = my_r < R;
 #pragma unroll
       for (int k = 0; k < NV; ++k)
-        uk[k] = (DIM == 3 && r0 == 0) ? uk_pre[k] : U[g * n + (xch.bcast_i(rw_cur, k) & ROW_CELL_MASK)];
+        uk[k] = (DIM == 3 && r0 == 0) ? uk_pre[k]
+                                      : U[state_at<AOS, NV>(n, g, xch.bcast_i(rw_cur, k) & ROW_CELL_MASK)];
       // a one-sided row whose member is a central row of an earlier chunk
       // takes that row's averages from LDS (the same values: same member,
       // same function) instead of loading the member and averaging again;
@@ -1580,7 +1601,7 @@ ZFV_HD void reconstruct_lane(const Img &m, int64_t i, const int g, X &xch, const
       if (is_E) cs_ = (d == 0) ? bm : cs_ + bm;
     }
     double sum = wb ? (s_acc + 1.0 * cs_) : 1.0 * cs_;
-    src[g * n + i] = sum / vol_i;
+    src[state_at<AOS, NV>(n, g, i)] = sum / vol_i;
   }
 }
 
@@ -1663,7 +1684,7 @@ ZFV_HD void face_flux(const Img &m, int64_t e, const double *__restrict__ fpv, d
 
 // ---- the per-cell rate of change -------------------------------------------------
 // L = -(1/vol) sum_faces (+-) |face| R^T G  (+ source) (+ flux BC)
-template <int DIM>
+template <int DIM, bool AOS = false>
 ZFV_HD void cell_rate(const Img &m, int64_t i, const double *__restrict__ U, const double *__restrict__ G,
                       const double *__restrict__ src, double *L) {
   constexpr int NV = DIM + 2;
@@ -1701,7 +1722,7 @@ ZFV_HD void cell_rate(const Img &m, int64_t i, const double *__restrict__ U, con
     double nn[3], t1[3], t2[3], area;
     load_face_frame<DIM>(m, i, f, nn, t1, t2, area);
     double g[NV], u[NV], r[NV];
-    for (int v = 0; v < NV; ++v) u[v] = U[v * n + i];
+    for (int v = 0; v < NV; ++v) u[v] = U[state_at<AOS, NV>(n, v, i)];
     r[0] = u[0];
     r[NV - 1] = u[NV - 1];
     if (DIM == 2) {
@@ -1721,7 +1742,7 @@ ZFV_HD void cell_rate(const Img &m, int64_t i, const double *__restrict__ U, con
   const double vol = m.vol[i];
   for (int v = 0; v < NV; ++v) L[v] = acc[v] / vol;
   if (m.gravity != 0 && src != nullptr)
-    for (int v = 0; v < NV; ++v) L[v] += src[v * n + i];
+    for (int v = 0; v < NV; ++v) L[v] += src[state_at<AOS, NV>(n, v, i)];
 }
 
 }  // namespace zfv
