@@ -1047,7 +1047,8 @@ void build_image(const zfv_mesh &mesh, const zfv_params &p, HostImage &img) {
 
   // pack SoA in product order
   const size_t N = size_t(n);
-  img.P.assign(size_t(s.m) * N, 0.0);
+  const int gpw = 64 / s.nvars;  // cells of a pseudo-inverse tile (p_central)
+  img.P.assign(size_t(s.m) * gpw * ((N + gpw - 1) / gpw), 0.0);
   img.rows.assign(size_t(s.nrows) * N, 0);
   img.twin.assign(size_t(std::max(s.nrows - s.rc, 1)) * N, int8_t(-1));
   img.crn.assign(size_t(dim == 2 ? 6 : 16) * N, 0.0);  // per cell, each vertex on 16 bytes
@@ -1066,17 +1067,18 @@ void build_image(const zfv_mesh &mesh, const zfv_params &p, HostImage &img) {
     const int i = img.perm[ip];
     // central coefficient a of row r (flat a rc + r) at p_central, one-sided
     // coefficient a of row rr of stencil kb (flat kb nbc rb + a rb + rr after
-    // the central ones) at p_onesided
-    const int nc = s.dofc - 1, nbc = s.dofb - 1;
+    // the central ones) at p_onesided of the cell's tile
+    const int nc = s.dofc - 1, nbc = s.dofb - 1, grp = ip % gpw;
+    double *tile = &img.P[size_t(ip / gpw) * s.m * gpw];
     for (int m = 0; m < s.m; ++m) {
-      size_t at;
+      int at;
       if (m < nc * s.rc) {
-        at = size_t(p_central(nc, s.rc, n, m / s.rc, m % s.rc, ip));
+        at = p_central(s.nvars, gpw, nc, s.rc, m / s.rc, m % s.rc, grp);
       } else {
         const int o = m - nc * s.rc, kb = o / (nbc * s.rb), a = (o % (nbc * s.rb)) / s.rb, rr = o % s.rb;
-        at = size_t(p_onesided(nc, s.rc, nbc, s.nb, s.rb, n, kb, a, rr, ip));
+        at = p_onesided(gpw, nc, s.rc, nbc, s.nb, s.rb, kb, a, rr, grp);
       }
-      img.P[at] = Pc[size_t(i) * s.m + m];
+      tile[at] = Pc[size_t(i) * s.m + m];
     }
     for (int r = 0; r < s.nrows; ++r) {
       const int32_t rc = rows_c[size_t(i) * s.nrows + r];

@@ -45,7 +45,7 @@ struct HostImage {
   Shape s;
   int64_t n = 0;   // cells
   int64_t ne = 0;  // interior faces
-  std::vector<double> P;         // m * n
+  std::vector<double> P;         // m * n in tiles of one wavefront's cells (p_central)
   std::vector<int32_t> rows;     // nrows * n   (product numbering)
   // one-sided row r (rc <= r < nrows) whose member (cell and translation) is
   // also central row twin[(r - rc) * n + i]: its equilibrium average is the

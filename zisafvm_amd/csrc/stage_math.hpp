@@ -129,6 +129,35 @@ struct state_is_aos : std::false_type {};
 template <class X>
 struct state_is_aos<X, std::void_t<decltype(X::kAos)>> : std::bool_constant<X::kAos> {};
 
+// a value that all lanes of a wavefront hold alike, where the compiler cannot
+// see it (the host emulation's exchange has one lane at a time)
+ZFV_HD int wave_uniform(int v) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  return __builtin_amdgcn_readfirstlane(v);
+#else
+  return v;
+#endif
+}
+// no instruction is moved across (keeps later chunks' loads from being pulled
+// forward into registers that the occupancy needs)
+ZFV_HD void schedule_fence() {
+#if defined(__HIP_DEVICE_COMPILE__)
+  __builtin_amdgcn_sched_barrier(0);
+#endif
+}
+
+// the values are formed before this point (the compiler otherwise sinks
+// accumulations to their last use and keeps their operands in registers)
+template <int N>
+ZFV_HD void computed_here(double *v) {
+#if defined(__HIP_DEVICE_COMPILE__)
+#pragma unroll
+  for (int k = 0; k < N; ++k) asm volatile("" : "+v"(v[k]));
+#else
+  (void)v;
+#endif
+}
+
 // two adjacent doubles, one 16-byte load
 struct alignas(16) PPair {
   double lo, hi;
@@ -831,35 +860,41 @@ ZFV_HD void rusanov(const double *uL, const double *uR, double gamma, double *f)
 // point values, written for interior faces (one group writes its cell's whole
 // block, so cache lines fill within one XCD).  src: as the state, or null.
 // LDS of one wavefront: first a row region of wave_lds_doubles holding each
-// group's NV pseudo-inverse rows of NC entries (group c at c NV NC: a stride
-// of NV NC doubles keeps the groups' reads on different banks), then per
+// group's NV rows of row_doubles entries (the NC pseudo-inverse entries, then
+// the member's equilibrium averages; group c at c NV row_doubles, an even
+// stride that puts the groups' 16-byte reads on different banks), then per
 // cell group its central rows' member equilibrium averages (er, eE per row,
 // for the one-sided rows that share their member; group_lds_doubles).
+template <int DOFC>
+constexpr int row_doubles() { return (DOFC + 1 + 1) & ~1; }
 template <int DIM, int DOFC>
-constexpr int wave_lds_doubles() { return (64 / (DIM + 2)) * (DIM + 2) * (DOFC - 1); }
+constexpr int wave_lds_doubles() { return (64 / (DIM + 2)) * (DIM + 2) * row_doubles<DOFC>(); }
 template <int RC>
 constexpr int group_lds_doubles() { return 2 * RC; }
 template <int DIM, int DOFC, int RC>
 constexpr int wave_block_doubles() { return wave_lds_doubles<DIM, DOFC>() + (64 / (DIM + 2)) * group_lds_doubles<RC>(); }
-// the index of central coefficient a of row r of cell i in the pseudo-inverse
-// array (pairs a, a + 1 of one row and cell adjacent, one 16-byte load; an
-// odd last coefficient in its own block); the one-sided rows follow at nc rc n
-// the index of coefficient a of row rr of one-sided stencil kb (nbc
-// coefficients, rb rows each): after the central block, pairs a, a + 1 of a
-// row adjacent as for the central rows, an odd last coefficient in its own
-// block
-ZFV_HD int64_t p_onesided(int nc, int rc, int nbc, int nb, int rb, int64_t n, int kb, int a, int rr, int64_t i) {
-  const int64_t base = int64_t(nc) * rc * n;
-  const int npair = nbc / 2;
-  const int64_t row = int64_t(kb) * rb + rr;
-  if (a < 2 * npair) return base + ((row * npair + (a >> 1)) * n + i) * 2 + (a & 1);
-  return base + int64_t(2 * npair) * nb * rb * n + row * n + i;
+
+// The pseudo-inverses are stored in tiles of one wavefront's cells (gpw =
+// 64 / nv consecutive cells; m gpw doubles a tile, m entries a cell), in the
+// order the wavefront reads them: rows in chunks of nv (lane g of a group
+// takes row g of the chunk), and within a chunk coefficient pairs (a, a + 1),
+// each pair of all the tile's lanes contiguous, so that a load instruction
+// reads one piece of 16 bytes a lane and a wavefront streams one contiguous
+// tile.  Central rows come first (all pairs, then an odd last coefficient),
+// then the one-sided stencils, whose rb rows form a chunk each.  These are
+// the places inside a tile of coefficient a of central row r and of row rr of
+// one-sided stencil kb, for the tile's cell grp.
+ZFV_HD int p_central(int nv, int gpw, int nc, int rc, int a, int r, int grp) {
+  const int c = r / nv, g = r - c * nv, np = nc / 2;
+  const int vc = rc - c * nv < nv ? rc - c * nv : nv;  // rows of this chunk
+  if (a < 2 * np) return 2 * ((c * nv * np + (a >> 1) * vc) * gpw + grp * vc + g) + (a & 1);
+  return 2 * np * rc * gpw + c * nv * gpw + grp * vc + g;
 }
 
-ZFV_HD int64_t p_central(int nc, int rc, int64_t n, int a, int r, int64_t i) {
-  const int ncp = nc / 2;
-  if (a < 2 * ncp) return ((int64_t(a >> 1) * rc + r) * n + i) * 2 + (a & 1);
-  return int64_t(2 * ncp) * rc * n + int64_t(r) * n + i;
+ZFV_HD int p_onesided(int gpw, int nc, int rc, int nbc, int nb, int rb, int kb, int a, int rr, int grp) {
+  const int base = nc * rc * gpw, np = nbc / 2;
+  if (a < 2 * np) return base + 2 * ((kb * np + (a >> 1)) * rb * gpw + grp * rb + rr) + (a & 1);
+  return base + 2 * np * nb * rb * gpw + (kb * gpw + grp) * rb + rr;
 }
 
 template <int DIM, int DOFC, int RC, int NB, int RB, int Q, int PH, class X>
@@ -887,16 +922,40 @@ ZFV_HD void reconstruct_lane(const Img &m, int64_t i, const int g, X &xch, const
   double sc_rho = rho0, sc_E = Eint0, sc_a = sqrt(gamma * (Eint0 * (gamma - 1.0)) / rho0);
   if (m.scaling == 1) sc_rho = sc_E = sc_a = 1.0;
   const bool is_rho = g == 0, is_E = g == NV - 1;
-  // The first two chunks' stencil row entries (and in 3D the first chunk's
-  // member states) are loaded before the equilibrium solve, whose arithmetic
-  // then covers their latency (every row entry names a cell, first-order
-  // cells included)
-  constexpr int R_ALL = RC + NB * RB;
-  const int32_t rw_pre0 = g < R_ALL ? m.rows[g * n + i] : int32_t(0);
-  const int32_t rw_pre1 = NV + g < R_ALL ? m.rows[(NV + g) * n + i] : int32_t(0);
-  double uk_pre[NV];
-  if (DIM == 3)
-    for (int k = 0; k < NV; ++k) uk_pre[k] = U[state_at<AOS, NV>(n, g, xch.bcast_i(rw_pre0, k) & ROW_CELL_MASK)];
+  // Stencil rows in chunks: lane g owns row c NV + g of central chunk c and
+  // row g of each one-sided stencil's chunk.  All row entries and the first
+  // chunk's member states are loaded before the equilibrium solve, whose
+  // arithmetic then covers their latency (every row entry names a cell,
+  // first-order cells included).
+  static_assert(RB <= NV, "a one-sided stencil's rows form one chunk");
+  constexpr int CCH = (RC + NV - 1) / NV;  // central chunks
+  constexpr int NCH = CCH + NB;
+  auto chunk_rows = [](int ch) { return ch < CCH ? (RC - ch * NV < NV ? RC - ch * NV : NV) : RB; };
+  auto chunk_row0 = [](int ch) { return ch < CCH ? ch * NV : RC + (ch - CCH) * RB; };
+  int32_t rw[NCH];
+#pragma unroll
+  for (int ch = 0; ch < NCH; ++ch) {
+    // (a lane past the chunk's rows reads the chunk's last)
+    const int rg = g < chunk_rows(ch) ? g : chunk_rows(ch) - 1;
+    rw[ch] = m.rows[(chunk_row0(ch) + rg) * n + i];
+  }
+  // this lane's variable of the members of chunk ch.  (Byte offsets of 32
+  // bits: the state of the largest instance that fits is under 4 GiB.)
+  auto gather = [&](int ch, double *uk) {
+    const int32_t j = rw[ch] & ROW_CELL_MASK;
+#pragma unroll
+    for (int k = 0; k < NV; ++k) {
+      if (k >= chunk_rows(ch)) break;
+      if (AOS) {
+        const uint32_t at = uint32_t(xch.bcast_i(int32_t(uint32_t(j) * uint32_t(NV * 8)), k)) + uint32_t(g) * 8u;
+        uk[k] = *reinterpret_cast<const double *>(reinterpret_cast<const char *>(U) + at);
+      } else {
+        uk[k] = U[state_at<AOS, NV>(n, g, xch.bcast_i(j, k))];
+      }
+    }
+  };
+  double uk[NV];
+  gather(0, uk);
 
   double vtx[DIM + 1][3];
   load_corners<DIM>(m, i, vtx);
@@ -1157,21 +1216,51 @@ ZFV_HD void reconstruct_lane(const Img &m, int64_t i, const int g, X &xch, const
   // this variable's coefficients: central c[alpha] (alpha = 1..DOFC-1),
   // one-sided b[k][alpha] (alpha = 1..DIM)
   double c[NC];
-  // (b is zeroed after the central rows, where it starts to be used, so it
-  // holds no registers during them)
   double b[NB > 0 ? NB : 1][NBC];
   for (int a = 0; a < NC; ++a) c[a] = 0.0;
 
   if (!first_order) {
-    // Rows in chunks of NV: lane k of the group owns row r0 + k of a chunk.
-    // It computes that row's member equilibrium average (member data loaded
-    // one chunk ahead, row entries two chunks ahead, so memory latency
-    // overlaps arithmetic), then loads the row of the pseudo-inverse, which
-    // reaches every lane through the group's LDS slice; the averages reach
-    // the lanes by wavefront shuffles.
-    double *pl = xch.wave_lds() + xch.lane0() * NC;  // this group's NV rows x NC coefficients
-    double *ceq = xch.lds();                         // central rows' member averages (er, eE)
-    constexpr int NCP = NC / 2;                      // coefficient pairs of a central row
+    // Per chunk each lane computes its row's member equilibrium average, and
+    // its row of the pseudo-inverse and that average reach the group's lanes
+    // through LDS.  The next chunk's pseudo-inverse rows, member states and
+    // member data are loaded as soon as this chunk's have left their
+    // registers, so that they are in flight during its arithmetic.
+    constexpr int ROWW = row_doubles<DOFC>();
+    double *pl = xch.wave_lds() + xch.lane0() * ROWW;  // this group's NV rows
+    double *ceq = xch.lds();                           // central rows' member averages (er, eE)
+    constexpr int NCP = NC / 2;                        // coefficient pairs of a central row
+    constexpr int GPW = 64 / NV;
+    // the tile of pseudo-inverses of this wavefront's cells
+    const int64_t tile = wave_uniform(int(uint32_t(i) / uint32_t(GPW)));
+    const int grp = int(i - tile * GPW);
+    const double *Pt = m.P + tile * (int64_t(NC) * RC + NB * RB * NBC) * GPW;
+    // this lane's row of chunk ch: NC entries (central) or NBC (one-sided);
+    // lanes past the chunk's rows read nothing
+    auto load_P = [&](int ch, double *pr) {
+      const PPair *pp = reinterpret_cast<const PPair *>(Pt);
+      if (g >= chunk_rows(ch)) return;
+      if (ch < CCH) {
+#pragma unroll
+        for (int p = 0; p < NCP; ++p) {
+          const PPair v = pp[uint32_t(p_central(NV, GPW, NC, RC, 2 * p, ch * NV, 0) / 2) +
+                             uint32_t(grp * chunk_rows(ch) + g)];
+          pr[2 * p] = v.lo;
+          pr[2 * p + 1] = v.hi;
+        }
+        if (NC & 1)
+          pr[NC - 1] = Pt[uint32_t(p_central(NV, GPW, NC, RC, NC - 1, ch * NV, 0)) + uint32_t(grp * chunk_rows(ch) + g)];
+      } else {
+#pragma unroll
+        for (int p = 0; p < NBC / 2; ++p) {
+          const PPair v = pp[uint32_t(p_onesided(GPW, NC, RC, NBC, NB, RB, ch - CCH, 2 * p, 0, 0) / 2) +
+                             uint32_t(grp * RB + g)];
+          pr[2 * p] = v.lo;
+          pr[2 * p + 1] = v.hi;
+        }
+        if (NBC & 1)
+          pr[NBC - 1] = Pt[uint32_t(p_onesided(GPW, NC, RC, NBC, NB, RB, ch - CCH, NBC - 1, 0, 0)) + uint32_t(grp * RB + g)];
+      }
+    };
     // scaled deviation of row k of the chunk in this lane's variable
     // (the equilibrium parts enter with factors 1 or 0: u - 1 er = u - er
     // and x - 0 eE = x exactly, so this equals the branchy form bit for bit)
@@ -1180,15 +1269,6 @@ ZFV_HD void reconstruct_lane(const Img &m, int64_t i, const int g, X &xch, const
       const double d = fma(-f_E, eE, fma(-f_rho, er, u));
       return fma(d, inv_g, -q0);
     };
-    // a member's equilibrium averages as lane k computed them; in the light
-    // set the energy average is the density average times the cell constant
-    // b (member_avg), formed here from the broadcast density average
-    auto member_eq = [&](double my_er, double my_eE, int k, double &er, double &eE) {
-      er = xch.bcast(my_er, k);
-      if (PH == PH_LIGHT) eE = eq_sub ? er * thc.b : 0.0;
-      else eE = xch.bcast(my_eE, k);
-    };
-
     // what the equilibrium average over a member (row entry rw) needs: its potential
     // moments (linear isentropic equilibrium, untranslated member) or its
     // translated corners and volume
@@ -1199,9 +1279,9 @@ ZFV_HD void reconstruct_lane(const Img &m, int64_t i, const int g, X &xch, const
       double sphi;  // light set: the translation's potential, added at use
       int lin;
     };
-    auto load_member = [&](int32_t rw, Member &mb) {
-      const int64_t j = rw & ROW_CELL_MASK;
-      const int code = rw >> ROW_CELL_BITS;
+    auto load_member = [&](int32_t entry, Member &mb) {
+      const int64_t j = entry & ROW_CELL_MASK;
+      const int code = entry >> ROW_CELL_BITS;
       if (PH == PH_LIGHT) {
         // the member's corner potentials in w3[k][0] and its translation's
         // potential, added where they are used (so that the loads stay in
@@ -1233,133 +1313,78 @@ ZFV_HD void reconstruct_lane(const Img &m, int64_t i, const int g, X &xch, const
         member_avg(mb.w3, mb.vol, er, eE);
       }
     };
-    // All rows R = RC + NB RB (central rows, then the one-sided stencils'
-    // rows kb RB + rr) in one stream of chunks: the row entries run two chunks
-    // ahead and lane g's member one chunk ahead of the chunk being
-    // accumulated.  Chunks of central rows only run in a first rolled loop,
-    // the rest (the last central rows and the one-sided ones) in a second, so
-    // the one-sided coefficients b hold registers only there.
-    constexpr int R = RC + NB * RB;
-    int32_t rw_cur = rw_pre0;
-    int32_t rw_nxt = rw_pre1;
-    Member mb_cur{};
-    if (eq_sub && g < R) load_member(rw_cur, mb_cur);
-    // stages chunk r0: loads the chunk's member states, advances the
-    // member/row pipeline, computes this lane's member average, then loads
-    // this lane's row of the pseudo-inverse (central: NC entries; one-sided:
-    // NBC, the rest 0; loaded after the average so that they hold no
-    // registers during it) and shares the rows through the LDS slice
-    auto chunk = [&](int r0, double *uk, double &my_er, double &my_eE) {
-      const int my_r = r0 + g;
-      const bool mine = my_r < R;
-#pragma unroll
-      for (int k = 0; k < NV; ++k)
-        uk[k] = (DIM == 3 && r0 == 0) ? uk_pre[k]
-                                      : U[state_at<AOS, NV>(n, g, xch.bcast_i(rw_cur, k) & ROW_CELL_MASK)];
-      // a one-sided row whose member is a central row of an earlier chunk
-      // takes that row's averages from LDS (the same values: same member,
-      // same function) instead of loading the member and averaging again;
-      // not in PH_LIN, whose member averages cost less than the lookup
-      auto twin_before = [&](int r, int chunk0) {
-        if (PH == PH_LIN || !eq_sub || r < RC || r >= R) return -1;
-        const int t = m.twin[(r - RC) * n + i];
-        return t < chunk0 ? t : -1;
-      };
-      const int tw = twin_before(my_r, r0);
-      Member mb_nxt{};
-      if (eq_sub && my_r + NV < R && twin_before(my_r + NV, r0 + NV) < 0) load_member(rw_nxt, mb_nxt);
-      const int32_t rw_far = my_r + 2 * NV < R ? m.rows[(my_r + 2 * NV) * n + i] : int32_t(0);
-      my_er = 0.0;
-      my_eE = 0.0;
-      if (eq_sub && mine) {
-        if (tw >= 0) {
-          my_er = ceq[2 * tw];
-          my_eE = ceq[2 * tw + 1];
-        } else {
-          member_avg_of(mb_cur, my_er, my_eE);
-        }
-        if (PH != PH_LIN && my_r < RC) {
-          ceq[2 * my_r] = my_er;
-          ceq[2 * my_r + 1] = my_eE;
-        }
-      }
-      double pr[NC];
-      if (my_r < RC) {
-        // coefficient pairs in one 16-byte load each
-        const PPair *pp = reinterpret_cast<const PPair *>(m.P);
-#pragma unroll
-        for (int p = 0; p < NCP; ++p) {
-          const PPair v = pp[p_central(NC, RC, n, 2 * p, my_r, i) >> 1];
-          pr[2 * p] = v.lo;
-          pr[2 * p + 1] = v.hi;
-        }
-        if (NC & 1) pr[NC - 1] = m.P[p_central(NC, RC, n, NC - 1, my_r, i)];
-      } else {
-        const int kb = (my_r - RC) / RB, rr = (my_r - RC) - kb * RB;
-#pragma unroll
-        for (int a = 0; a < NC; ++a) pr[a] = 0.0;
-        if (mine) {
-          const PPair *pp = reinterpret_cast<const PPair *>(m.P);
-#pragma unroll
-          for (int p = 0; p < NBC / 2; ++p) {
-            const PPair v = pp[p_onesided(NC, RC, NBC, NB, RB, n, kb, 2 * p, rr, i) >> 1];
-            pr[2 * p] = v.lo;
-            pr[2 * p + 1] = v.hi;
-          }
-          if (NBC & 1) pr[NBC - 1] = m.P[p_onesided(NC, RC, NBC, NB, RB, n, kb, NBC - 1, rr, i)];
-        }
-      }
-      xch.sync();
-#pragma unroll
-      for (int a = 0; a < NC; ++a) pl[g * NC + a] = pr[a];
-      xch.sync();
-      rw_cur = rw_nxt;
-      rw_nxt = rw_far;
-      mb_cur = mb_nxt;
+    // a one-sided row whose member is also a central row takes that row's
+    // averages from LDS (the same values: same member, same function)
+    // instead of loading the member and averaging again; not in PH_LIN,
+    // whose member averages cost less than the lookup
+    auto twin_of = [&](int ch) {
+      if (PH == PH_LIN || !eq_sub || ch < CCH || g >= RB) return -1;
+      return int(m.twin[(chunk_row0(ch) + g - RC) * n + i]);
     };
-    // Rows are accumulated in a rolled loop over the chunk (one row's
-    // entries in registers at a time).  Central rows past the last of a
-    // chunk would add exact zeros; rows past R are skipped.
-    constexpr int R0 = (RC / NV) * NV;  // central rows in whole chunks
-#pragma unroll 1
-    for (int r0 = 0; r0 < R0; r0 += NV) {
-      double uk[NV], my_er, my_eE;
-      chunk(r0, uk, my_er, my_eE);
-#pragma unroll 1
-      for (int k = 0; k < NV; ++k) {
-        double er = 0.0, eE = 0.0;
-        if (wb) member_eq(my_er, my_eE, k, er, eE);
-        const double d = deviation(uk[k], er, eE);
-#pragma unroll
-        for (int a = 0; a < NC; ++a) c[a] = fma(pl[k * NC + a], d, c[a]);
-      }
-    }
     for (int k = 0; k < NB; ++k)
       for (int a = 0; a < NBC; ++a) b[k][a] = 0.0;
-#pragma unroll 1
-    for (int r0 = R0; r0 < R; r0 += NV) {
-      double uk[NV], my_er, my_eE;
-      chunk(r0, uk, my_er, my_eE);
-#pragma unroll 1
-      for (int k = 0; k < NV; ++k) {
-        const int r = r0 + k;  // uniform over the group
-        if (r >= R) break;
+    double pr[NC];
+    for (int a = 0; a < NC; ++a) pr[a] = 0.0;
+    Member mb{};
+    int tw = -1;
+    load_P(0, pr);
+    if (eq_sub && g < chunk_rows(0)) load_member(rw[0], mb);
+#pragma unroll
+    for (int ch = 0; ch < NCH; ++ch) {
+      const int cnt = chunk_rows(ch);
+      xch.sync();  // the previous chunk's reads are done
+#pragma unroll
+      for (int a = 0; a < (ch < CCH ? NC : NBC); ++a) pl[g * ROWW + a] = pr[a];
+      const Member mc = mb;
+      const int tc = tw;
+      double uc[NV];
+#pragma unroll
+      for (int k = 0; k < NV; ++k) uc[k] = uk[k];
+      if (ch + 1 < NCH) {
+        load_P(ch + 1, pr);
+        gather(ch + 1, uk);
+        tw = twin_of(ch + 1);
+        if (eq_sub && g < chunk_rows(ch + 1) && tw < 0) load_member(rw[ch + 1], mb);
+      }
+      if (eq_sub) {
         double er = 0.0, eE = 0.0;
-        if (wb) member_eq(my_er, my_eE, k, er, eE);
-        const double d = deviation(uk[k], er, eE);
-        if (r < RC) {
-#pragma unroll
-          for (int a = 0; a < NC; ++a) c[a] = fma(pl[k * NC + a], d, c[a]);
-        } else {
-          const int kb = (r - RC) / RB;
-#pragma unroll
-          for (int a = 0; a < NBC; ++a) {
-            const double p = pl[k * NC + a];
-#pragma unroll
-            for (int kk = 0; kk < NB; ++kk)
-              if (kk == kb) b[kk][a] = fma(p, d, b[kk][a]);
-          }
+        if (tc >= 0) {
+          er = ceq[2 * tc];
+          eE = ceq[2 * tc + 1];
+        } else if (g < cnt) {
+          member_avg_of(mc, er, eE);
         }
+        if (PH != PH_LIN && ch < CCH && g < cnt) {
+          ceq[2 * (ch * NV + g)] = er;
+          ceq[2 * (ch * NV + g) + 1] = eE;
+        }
+        pl[g * ROWW + NC] = er;
+        if (PH != PH_LIGHT) pl[g * ROWW + NC + 1] = eE;
+      }
+      xch.sync();
+#pragma unroll
+      for (int k = 0; k < NV; ++k) {
+        if (k >= cnt) break;
+        // in the light set the energy average is the density average times
+        // the cell constant b (member_avg)
+        const double *row = pl + k * ROWW;
+        double er = 0.0, eE = 0.0;
+        if (eq_sub) {
+          er = row[NC];
+          eE = PH == PH_LIGHT ? er * thc.b : row[NC + 1];
+        }
+        const double d = deviation(uc[k], er, eE);
+        if (ch < CCH) {
+#pragma unroll
+          for (int a = 0; a < NC; ++a) c[a] = fma(row[a], d, c[a]);
+        } else {
+#pragma unroll
+          for (int a = 0; a < NBC; ++a) b[ch < CCH ? 0 : ch - CCH][a] = fma(row[a], d, b[ch < CCH ? 0 : ch - CCH][a]);
+        }
+        // one row's entries in registers at a time
+        if (ch < CCH) computed_here<NC>(c);
+        else computed_here<NBC>(b[ch < CCH ? 0 : ch - CCH]);
+        schedule_fence();
       }
     }
   }
