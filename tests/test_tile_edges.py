@@ -13,13 +13,13 @@ from conftest import rel_err, wb_err
 TOL = 1e-12  # the parity tolerance of a rate of change
 
 # (cells modulo the tile size: 162 % 16 = 2, 242 % 16 = 2, 338 % 16 = 2; the
-# atmosphere's 9 x (9 + 6) x 2 = 270 % 16 = 14)
+# atmosphere's 9 x (9 + 6) x 2 = 270 % 16 = 14; 3135 % 12 = 3)
 CASES = {
     "order2_162": lambda: (W.vortex_2d(n=9), dict(order=2, edge_deg=2)),
     "order3_242": lambda: (W.vortex_2d(n=11), dict(order=3)),
     "order4_338": lambda: (W.vortex_2d(n=13), dict(order=4)),
     "isothermal_order4_270": lambda: (W.isothermal_2d(n=9, amplitude=1e-3), None),
-    "polytrope3d": lambda: (W.polytrope_3d(n=9, amplitude=1e-3), None),
+    "polytrope3d_3135": lambda: (W.polytrope_3d(n=10, amplitude=1e-3), None),
 }
 
 
