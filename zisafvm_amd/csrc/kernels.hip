@@ -243,6 +243,13 @@ __global__ __launch_bounds__(256) void k_face_table(Img m, double *tab) {
   store_face_table<DIM>(m, e, tab);
 }
 
+// per-cell outward area normals of the faces (3D)
+__global__ __launch_bounds__(256) void k_face_normals(Img m, double *tab) {
+  const int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
+  if (i >= m.n) return;
+  store_face_normals(m, i, tab);
+}
+
 // the gravity source moments of every cell
 template <int DIM, int DOFC>
 __global__ __launch_bounds__(256) void k_source_moments(Img m, double *tab) {
@@ -1019,6 +1026,14 @@ int create_device(zfv_handle *h) {
     }
     m.ffr = tab;
   }
+  m.fan = nullptr;
+  if (s.dim == 3 && params->equilibrium != ZFV_EQ_NONE) {
+    double *tab = h->alloc<double>(size_t(12) * n);
+    hipLaunchKernelGGL(k_face_normals, dim3(blocks_for(n, 256)), dim3(256), 0, h->stream, m, tab);
+    HIP_CHECK(hipGetLastError());
+    HIP_CHECK(hipStreamSynchronize(h->stream));
+    m.fan = tab;
+  }
   h->ph = physics_set(m);
   if (params->gravity != ZFV_GRAVITY_NONE) {
     double *tab = h->alloc<double>(size_t(s.dofc) * s.dim * n);
@@ -1327,11 +1342,11 @@ int zfv_get_info(zfv_handle *h, zfv_info *info) {
   const double nv = s.nvars;
   const double frame = s.dim == 2 ? frame_words<2>() : frame_words<3>();
   const Img &dm = h->dimg;
-  // tables: the potential at the cell's own volume and face points (its
-  // gradient rows are not read: the source moments hold the volume terms),
-  // the potential moments, the source moments (read outside the light set)
+  // tables: the potential at the cell's own volume and face points, the
+  // potential moments, the source moments (read outside the light set), the
+  // outward area normals
   const double tables = (dm.pot ? 8.0 * (dm.qv + s.nfaces * s.q) : 0.0) + (dm.phim ? 16.0 : 0.0) +
-                        (dm.smom && h->ph != PH_LIGHT ? 8.0 * s.dofc * s.dim : 0.0);
+                        (dm.smom && h->ph != PH_LIGHT ? 8.0 * s.dofc * s.dim : 0.0) + (dm.fan ? 8.0 * 12 : 0.0);
   const double rec = 8.0 * s.m + 4.0 * s.nrows + 8.0 * nv + 8.0 * (s.nfaces * s.dim + s.dim + 2 + s.nmom) +
                      4.0 * (1 + s.nfaces + 1) + tables +
                      8.0 * (2.0 * ne / n) * s.q * nv + (h->src ? 8.0 * nv : 0.0);
@@ -1435,12 +1450,13 @@ int zfv_estimate_device_bytes(const zfv_mesh *mesh, const zfv_params *params, in
   if (params->gravity != ZFV_GRAVITY_NONE) {
     per_cell += 8.0 * nv;                       // source
     per_cell += 8.0 * 2;                        // potential moments
-    per_cell += 8.0 * (16 * (1 + s.dim) + s.nfaces * s.q);  // potential tables (at most)
+    per_cell += 8.0 * (16 + s.nfaces * s.q);    // potential tables (at most)
   }
   if (mesh->ghost_mask) per_cell += 8.0 * nv;                          // steady state
   if (params->steps_per_recompute > 1) per_cell += 8.0 * 8 + 4.0;       // kept equilibria
   per_cell += 8.0 * s.nfaces * ((s.q * s.nvars + 1) & ~1);            // face-point values per cell-face slot
   if (params->equilibrium != ZFV_EQ_NONE) per_cell += 8.0 * s.nfaces;  // corner potentials (light set)
+  if (params->equilibrium != ZFV_EQ_NONE && s.dim == 3) per_cell += 8.0 * 12;  // outward area normals
   if (params->gravity != ZFV_GRAVITY_NONE) per_cell += 8.0 * s.dofc * s.dim;  // source moments
   double per_face = 8.0 * nv + 4.0 * 2 + 8.0 * frame;  // fluxes, the two slots, the frame and area
   *bytes = int64_t(n * per_cell + ne * per_face) + (1 << 20);

@@ -63,6 +63,9 @@ struct Img {
   const double *pot;     // potential tables of the cell's own points (pot_index), or null
   const double *frm;     // face frames of the cells' local faces (load_face_frame)
   const double *ffr;     // per interior face its frame and area, t1, area (2D) or n, t1, area (3D), x ne
+  // 3D with an equilibrium: per cell its faces' outward normals times their
+  // areas, n x (face 3 + d) (store_face_normals), or null
+  const double *fan;
   // gravity: per cell vol sum_q vw_q b_alpha(x_q) d_d phi(x_q) over its volume
   // points, n x (alpha DIM + d), each cell's DOFC x DIM values contiguous
   // (store_source_moments), or null
@@ -293,7 +296,7 @@ ZFV_HD void eq_at_phi(const Img &m, const EqC &c, double ph, double &rho, double
     // PH_LIN has gamma = 2: the exponents are 1 and 2, as ipow takes them
     rho = PH == PH_LIN ? c.a * h : ipow(c.a * h, c.b);
     double p = c.th1 * (PH == PH_LIN ? rho * rho : ipow(rho, m.gamma));
-    E = p / (m.gamma - 1.0);
+    E = PH == PH_LIN ? p : p / (m.gamma - 1.0);
   } else {
     rho = c.th0 * exp((ph - c.phi_ref) * c.a);
     E = rho * c.b;
@@ -404,11 +407,28 @@ ZFV_HD void face_vertices(uint32_t fperm, int f, const double (*v)[3], double (*
   }
 }
 
-// the same vertices read from the cell's corner arrays (cache hits) instead
-// of selected from registers
+// Corner t of a cell's local face f, in the cell's own order (the GMSH tables;
+// outward by the right-hand rule for the cells' standard vertex order)
 template <int DIM>
-ZFV_HD void load_face_vertices(const Img &m, int64_t i, uint32_t fperm, int f, double (*w)[3]) {
-  for (int r = 0; r < DIM; ++r) load_corner<DIM>(m, i, int((fperm >> (2 * (f * 3 + r))) & 3u), w[r]);
+ZFV_HD constexpr int face_corner(int f, int t) {
+  if (DIM == 2) return (f + t) % 3;
+  constexpr int tab[4][3] = {{0, 1, 3}, {0, 2, 1}, {0, 3, 2}, {1, 2, 3}};
+  return tab[f][t];
+}
+
+// A face's quadrature points numbered along the cell's own vertex order of the
+// face, and the number of the same point in the face's left cell's order
+// (fperm): the rules are symmetric, so an edge's points run backwards in the
+// other direction, and a triangle's points beyond the Q mod 3 central ones
+// each belong to one vertex.
+template <int DIM, int Q>
+ZFV_HD int face_point_in_left_order(uint32_t fperm, int f, int q) {
+  if (DIM == 2) return int((fperm >> (6 * f)) & 3u) == f ? q : Q - 1 - q;
+  constexpr int C = Q % 3;
+  if (q < C) return q;
+  const int t = (q - C) % 3, own = face_corner<3>(f, t);
+  const int pos = int((fperm >> (6 * f + 2)) & 3u) == own ? 1 : (int((fperm >> (6 * f + 4)) & 3u) == own ? 2 : 0);
+  return q - t + pos;
 }
 
 // Face frame (src/zisa/math/face_factory.cpp:11-34): n, t1, t2 and the face
@@ -457,9 +477,7 @@ ZFV_HD void face_frame(const double (*w)[3], double *n, double *t1, double *t2, 
 // faces' frames (the left cell's view) are copied into a table in face order
 // for the face kernel (store_face_table); the flux BC of the cell update
 // reads a cell's own.  n (2D) and t2 follow from the stored values with
-// face_frame's own formulas, so every value equals face_frame's.  (The
-// reconstruction, which loads the face vertices for its quadrature points
-// anyway, rebuilds them: measured faster.)
+// face_frame's own formulas, so every value equals face_frame's.
 template <int DIM>
 constexpr int frame_words() { return DIM == 2 ? 3 : 7; }
 // doubles of one cell-face slot of face-point values: Q x NV rounded up to
@@ -519,6 +537,29 @@ ZFV_HD void load_face_frame(const Img &m, int64_t i, int f, double *n, double *t
   t2[0] = n[1] * t1[2] - n[2] * t1[1];
   t2[1] = n[2] * t1[0] - n[0] * t1[2];
   t2[2] = n[0] * t1[1] - n[1] * t1[0];
+}
+
+// the outward normal of cell i's face f times its area (3D; the area and the
+// normal of its frame table entry, so that the well-balanced source's face
+// term and the fluxes see the same values)
+ZFV_HD void face_normal_out(const Img &m, int64_t i, int f, double *an) {
+  double n[3], t1[3], t2[3], area, c[4][3], xc[3] = {0.0, 0.0, 0.0};
+  load_face_frame<3>(m, i, f, n, t1, t2, area);
+  load_corners<3>(m, i, c);
+  // (the sign against the vector from the cell's mean corner to the face's)
+  for (int k = 0; k < 4; ++k)
+    for (int d = 0; d < 3; ++d) xc[d] += 0.25 * c[k][d];
+  double dd = 0.0;
+  for (int d = 0; d < 3; ++d) {
+    const double fc = (c[face_corner<3>(f, 0)][d] + c[face_corner<3>(f, 1)][d] + c[face_corner<3>(f, 2)][d]) / 3.0;
+    dd += n[d] * (fc - xc[d]);
+  }
+  for (int d = 0; d < 3; ++d) an[d] = (dd < 0.0 ? -area : area) * n[d];
+}
+
+// writes the outward area normals of cell i's faces (tab: 12 n)
+ZFV_HD void store_face_normals(const Img &m, int64_t i, double *tab) {
+  for (int f = 0; f < 4; ++f) face_normal_out(m, i, f, tab + 12 * i + 3 * f);
 }
 
 // Per interior face its frame in face order (the face kernel reads it
@@ -611,21 +652,20 @@ ZFV_HD void phi_moments(const Img &m, int64_t i, double &mean, double &var) {
 }
 
 // Potential tables.  Radial and polytrope gravity have no affine closed form,
-// and the potential and its gradient at a cell's own quadrature points do not
-// change in time, so instances of the full physics sets with gravity keep
-// them per cell (SoA, n cells), computed once with the functions below:
-//   pot[q n + i]                       phi at volume point q      (q < qv)
-//   pot[(qv + q DIM + d) n + i]        d-th component of grad phi there
-//   pot[(qv (1 + DIM) + f Q + q) n + i] phi at point q of local face f
+// and the potential at a cell's own quadrature points does not change in time,
+// so instances of the full physics sets with gravity keep it per cell,
+// computed once with the functions above:
+//   pot[i (DIM + 1) Q + f Q + q]         phi at point q of local face f (the
+//                                        cell's own vertex order), each cell's
+//                                        contiguous
+//   pot[((DIM + 1) Q + q) n + i]         phi at volume point q (q < qv)
 // The reconstruction then evaluates no transcendental function at its own
 // points; the values are those the functions give at the same points.
 template <int DIM>
-ZFV_HD int64_t pot_index_grad(const Img &m, int q, int d) { return int64_t(m.qv + q * DIM + d) * m.n; }
-template <int DIM>
-ZFV_HD int64_t pot_index_face(const Img &m, int nqf, int f, int q) { return int64_t(m.qv * (1 + DIM) + f * nqf + q) * m.n; }
+ZFV_HD int64_t pot_index_vol(const Img &m, int nqf, int q) { return (int64_t(DIM + 1) * nqf + q) * m.n; }
 // rows of the tables for nqf face points
 template <int DIM>
-ZFV_HD int pot_rows(int qv, int nqf) { return qv * (1 + DIM) + (DIM + 1) * nqf; }
+ZFV_HD int pot_rows(int qv, int nqf) { return qv + (DIM + 1) * nqf; }
 
 // fills the potential tables of cell i (tab has pot_rows * n entries)
 template <int DIM>
@@ -633,20 +673,18 @@ ZFV_HD void potential_points(const Img &m, int nqf, int64_t i, double *tab) {
   double vtx[DIM + 1][3];
   load_corners<DIM>(m, i, vtx);
   for (int q = 0; q < m.qv; ++q) {
-    double x[3], gp[3];
+    double x[3];
     volume_point<DIM>(m, q, vtx, x);
-    tab[int64_t(q) * m.n + i] = phi<DIM, PH_FULL>(m, x);
-    grad_phi<DIM, PH_FULL>(m, x, gp);
-    for (int d = 0; d < DIM; ++d) tab[pot_index_grad<DIM>(m, q, d) + i] = gp[d];
+    tab[pot_index_vol<DIM>(m, nqf, q) + i] = phi<DIM, PH_FULL>(m, x);
   }
-  const uint32_t fperm = m.fperm[i];
   for (int f = 0; f < DIM + 1; ++f) {
     double w3[3][3];
-    face_vertices<DIM>(fperm, f, vtx, w3);
+    for (int t = 0; t < DIM; ++t)
+      for (int d = 0; d < 3; ++d) w3[t][d] = vtx[face_corner<DIM>(f, t)][d];
     for (int q = 0; q < nqf; ++q) {
       double x[3];
       face_point<DIM>(m, q, w3, x);
-      tab[pot_index_face<DIM>(m, nqf, f, q) + i] = phi<DIM, PH_FULL>(m, x);
+      tab[i * int64_t((DIM + 1) * nqf) + f * nqf + q] = phi<DIM, PH_FULL>(m, x);
     }
   }
 }
@@ -686,6 +724,38 @@ ZFV_HD void poly_eval(const double (*a)[NV], const double *c, const double *X, d
     }
     pxk *= X[0];
   }
+}
+
+// sum_alpha a[alpha] X^alpha in nested form (one multiply-add per
+// coefficient past the first)
+template <int DIM, int DEG>
+ZFV_HD double poly_nested(const double *a, const double *X) {
+  double rx = 0.0;
+#pragma unroll
+  for (int kx = DEG; kx >= 0; --kx) {
+    double ry = 0.0;
+#pragma unroll
+    for (int ky = DEG - kx; ky >= 0; --ky) {
+      if (DIM == 2) {
+        const int n = kx + ky;
+        const double c = a[(n + 1) * n / 2 + ky];
+        ry = ky == DEG - kx ? c : fma(ry, X[1], c);
+      } else {
+        double rz = 0.0;
+#pragma unroll
+        for (int kz = DEG - kx - ky; kz >= 0; --kz) {
+          const int n3 = kx + ky + kz - 1;
+          const int d3 = n3 < 0 ? 0 : (n3 + 1) * (n3 + 2) * (n3 + 3) / 6;
+          const int n2 = ky + kz;
+          const double c = a[d3 + (n2 + 1) * n2 / 2 + kz];
+          rz = kz == DEG - kx - ky ? c : fma(rz, X[2], c);
+        }
+        ry = ky == DEG - kx ? rz : fma(ry, X[1], rz);
+      }
+    }
+    rx = kx == DEG ? ry : fma(rx, X[0], ry);
+  }
+  return rx;
 }
 
 // the basis of poly_eval at X, in its order: b[i] = X^alpha_i - c[i]
@@ -862,11 +932,12 @@ ZFV_HD void rusanov(const double *uL, const double *uR, double gamma, double *f)
 // LDS of one wavefront: first a row region of wave_lds_doubles holding each
 // group's NV rows of row_doubles entries (the NC pseudo-inverse entries, then
 // the member's equilibrium averages; group c at c NV row_doubles, an even
-// stride that puts the groups' 16-byte reads on different banks), then per
+// stride that puts the groups' 16-byte reads on different banks; at least 6,
+// which holds the exchange of the nonlinear weights), then per
 // cell group its central rows' member equilibrium averages (er, eE per row,
 // for the one-sided rows that share their member; group_lds_doubles).
 template <int DOFC>
-constexpr int row_doubles() { return (DOFC + 1 + 1) & ~1; }
+constexpr int row_doubles() { return ((DOFC + 1 + 1) & ~1) > 6 ? ((DOFC + 1 + 1) & ~1) : 6; }
 template <int DIM, int DOFC>
 constexpr int wave_lds_doubles() { return (64 / (DIM + 2)) * (DIM + 2) * row_doubles<DOFC>(); }
 template <int RC>
@@ -963,7 +1034,9 @@ ZFV_HD void reconstruct_lane(const Img &m, int64_t i, const int g, X &xch, const
   // The potential at the cell's own quadrature points: from the instance's
   // tables in the full sets (always present in PH_LIN), else evaluated.
   const bool tab = PH == PH_LIN || (PH == PH_FULL && m.pot != nullptr);
-  auto vol_phi = [&](int q, const double *x) { return tab ? m.pot[int64_t(q) * n + i] : phi<DIM, PH>(m, x); };
+  auto vol_phi = [&](int q, const double *x) {
+    return tab ? m.pot[pot_index_vol<DIM>(m, Q, q) + i] : phi<DIM, PH>(m, x);
+  };
 
   // Average of an equilibrium over this cell with the quadrature points split
   // over the group's lanes: lane k sums the points q = k (mod NV) in order,
@@ -998,7 +1071,7 @@ ZFV_HD void reconstruct_lane(const Img &m, int64_t i, const int g, X &xch, const
   double th[2] = {0.0, 0.0};
   double phi_ref = 0.0;
   double ar1 = -1.0;  // isothermal: the average of exp(a (phi - phi_ref)) over the cell, once solved
-  const bool wb = m.eq != 0;
+  const bool wb = PH == PH_LIN || m.eq != 0;
   bool eq_found = false;
   if (wb) {
     double xref[3];
@@ -1128,7 +1201,11 @@ ZFV_HD void reconstruct_lane(const Img &m, int64_t i, const int g, X &xch, const
   const double scale_g = g == 0 ? sc_rho : (g == NV - 1 ? sc_E : sc_a);
   const double inv_g = 1.0 / scale_g;
 
-  const EqC thc = eq_consts<PH>(m, th, phi_ref);
+  // (without an equilibrium, constants that evaluate to zero everywhere, so
+  // that its evaluations need no branch)
+  const bool eq_sub = wb && eq_found;
+  EqC thc = eq_consts<PH>(m, th, phi_ref);
+  if (!eq_sub) thc.th0 = thc.th1 = thc.phi_ref = thc.a = thc.b = 0.0;
 
   // equilibrium average of this cell's equilibrium over a member cell given
   // its (translated) corners and volume
@@ -1179,7 +1256,6 @@ ZFV_HD void reconstruct_lane(const Img &m, int64_t i, const int g, X &xch, const
     er = (1.0 * sr) / vol_j;
     eE = (1.0 * sE) / vol_j;
   };
-  const bool eq_sub = wb && eq_found;
   // this cell's equilibrium averaged over the cell itself, the points split
   // over the group's lanes
   auto own_eq = [&](double &er, double &eE) { group_avg(thc, er, eE); };
@@ -1235,30 +1311,30 @@ ZFV_HD void reconstruct_lane(const Img &m, int64_t i, const int g, X &xch, const
     const int grp = int(i - tile * GPW);
     const double *Pt = m.P + tile * (int64_t(NC) * RC + NB * RB * NBC) * GPW;
     // this lane's row of chunk ch: NC entries (central) or NBC (one-sided);
-    // lanes past the chunk's rows read nothing
+    // lanes past the chunk's rows read its last
     auto load_P = [&](int ch, double *pr) {
       const PPair *pp = reinterpret_cast<const PPair *>(Pt);
-      if (g >= chunk_rows(ch)) return;
+      const int gr = g < chunk_rows(ch) ? g : chunk_rows(ch) - 1;
       if (ch < CCH) {
 #pragma unroll
         for (int p = 0; p < NCP; ++p) {
           const PPair v = pp[uint32_t(p_central(NV, GPW, NC, RC, 2 * p, ch * NV, 0) / 2) +
-                             uint32_t(grp * chunk_rows(ch) + g)];
+                             uint32_t(grp * chunk_rows(ch) + gr)];
           pr[2 * p] = v.lo;
           pr[2 * p + 1] = v.hi;
         }
         if (NC & 1)
-          pr[NC - 1] = Pt[uint32_t(p_central(NV, GPW, NC, RC, NC - 1, ch * NV, 0)) + uint32_t(grp * chunk_rows(ch) + g)];
+          pr[NC - 1] = Pt[uint32_t(p_central(NV, GPW, NC, RC, NC - 1, ch * NV, 0)) + uint32_t(grp * chunk_rows(ch) + gr)];
       } else {
 #pragma unroll
         for (int p = 0; p < NBC / 2; ++p) {
           const PPair v = pp[uint32_t(p_onesided(GPW, NC, RC, NBC, NB, RB, ch - CCH, 2 * p, 0, 0) / 2) +
-                             uint32_t(grp * RB + g)];
+                             uint32_t(grp * RB + gr)];
           pr[2 * p] = v.lo;
           pr[2 * p + 1] = v.hi;
         }
         if (NBC & 1)
-          pr[NBC - 1] = Pt[uint32_t(p_onesided(GPW, NC, RC, NBC, NB, RB, ch - CCH, NBC - 1, 0, 0)) + uint32_t(grp * RB + g)];
+          pr[NBC - 1] = Pt[uint32_t(p_onesided(GPW, NC, RC, NBC, NB, RB, ch - CCH, NBC - 1, 0, 0)) + uint32_t(grp * RB + gr)];
       }
     };
     // scaled deviation of row k of the chunk in this lane's variable
@@ -1328,7 +1404,7 @@ ZFV_HD void reconstruct_lane(const Img &m, int64_t i, const int g, X &xch, const
     Member mb{};
     int tw = -1;
     load_P(0, pr);
-    if (eq_sub && g < chunk_rows(0)) load_member(rw[0], mb);
+    if (wb) load_member(rw[0], mb);
 #pragma unroll
     for (int ch = 0; ch < NCH; ++ch) {
       const int cnt = chunk_rows(ch);
@@ -1344,14 +1420,14 @@ ZFV_HD void reconstruct_lane(const Img &m, int64_t i, const int g, X &xch, const
         load_P(ch + 1, pr);
         gather(ch + 1, uk);
         tw = twin_of(ch + 1);
-        if (eq_sub && g < chunk_rows(ch + 1) && tw < 0) load_member(rw[ch + 1], mb);
+        if (wb && tw < 0) load_member(rw[ch + 1], mb);
       }
-      if (eq_sub) {
+      if (wb) {
         double er = 0.0, eE = 0.0;
         if (tc >= 0) {
           er = ceq[2 * tc];
           eE = ceq[2 * tc + 1];
-        } else if (g < cnt) {
+        } else {
           member_avg_of(mc, er, eE);
         }
         if (PH != PH_LIN && ch < CCH && g < cnt) {
@@ -1369,7 +1445,7 @@ ZFV_HD void reconstruct_lane(const Img &m, int64_t i, const int g, X &xch, const
         // the cell constant b (member_avg)
         const double *row = pl + k * ROWW;
         double er = 0.0, eE = 0.0;
-        if (eq_sub) {
+        if (wb) {
           er = row[NC];
           eE = PH == PH_LIGHT ? er * thc.b : row[NC + 1];
         }
@@ -1431,31 +1507,48 @@ ZFV_HD void reconstruct_lane(const Img &m, int64_t i, const int g, X &xch, const
         }
       }
     }
-    // smoothness indicators (maximum over the variables, in variable order)
-    // and nonlinear weights (src/zisa/reconstruction/hybrid_weno.cpp:110-127)
+    // Smoothness indicators (maximum over the variables, in variable order) and
+    // nonlinear weights (src/zisa/reconstruction/hybrid_weno.cpp:110-127).  The
+    // lanes exchange their sums of squares through LDS; lane k then forms
+    // stencil k's weight, so that its power and division run once a cell
+    // instead of once a lane.
+    static_assert(NB + 1 <= NV, "one lane per stencil");
+    static_assert((NB + 1) * (NV + 1) <= NV * row_doubles<DOFC>(), "the exchange fits the group's rows");
+    double *sq = xch.wave_lds() + xch.lane0() * row_doubles<DOFC>();  // [stencil][variable], then the weights
+    double *wk = sq + (NB + 1) * NV;
+    xch.sync();
+#pragma unroll
+    for (int k = 0; k <= NB; ++k) {
+      double t = 0.0;
+      if (k == 0) {
+        for (int al = 0; al < NC; ++al) t += c[al] * c[al];
+      } else {
+        for (int al = 0; al < NBC; ++al) t += b[k - 1][al] * b[k - 1][al];
+      }
+      sq[k * NV + g] = t;
+    }
+    xch.sync();
+    const int my_k = g <= NB ? g : NB;
+    double IS = sq[my_k * NV];
+#pragma unroll
+    for (int v = 1; v < NV; ++v) IS = dmax(IS, sq[my_k * NV + v]);
+    const double isp = m.exponent == 4.0 ? sqr(sqr(IS)) : pow(IS, m.exponent);
+    wk[my_k] = m.lw[my_k] / (m.eps + isp);
+    xch.sync();
     double alpha[NB + 1];
     double al_tot = 0.0;
 #pragma unroll
     for (int k = 0; k <= NB; ++k) {
-      double s = 0.0;
-      if (k == 0) {
-        for (int al = 0; al < NC; ++al) s += c[al] * c[al];
-      } else {
-        for (int al = 0; al < NBC; ++al) s += b[k - 1][al] * b[k - 1][al];
-      }
-      double IS = xch.bcast(s, 0);
-#pragma unroll
-      for (int v = 1; v < NV; ++v) IS = dmax(IS, xch.bcast(s, v));
-      double isp = m.exponent == 4.0 ? sqr(sqr(IS)) : pow(IS, m.exponent);
-      alpha[k] = m.lw[k] / (m.eps + isp);
+      alpha[k] = wk[k];
       al_tot += alpha[k];
     }
-    const double w0 = alpha[0] / al_tot;
+    const double inv_tot = 1.0 / al_tot;
+    const double w0 = alpha[0] * inv_tot;
     a[0] = 0.0 + w0 * a0[0];
     for (int al = 1; al < DOFC; ++al) a[al] = 0.0 + w0 * c[al - 1];
 #pragma unroll
     for (int k = 0; k < NB; ++k) {
-      const double w = alpha[k + 1] / al_tot;
+      const double w = alpha[k + 1] * inv_tot;
       a[0] = a[0] + w * a0[k + 1];
       for (int al = 1; al <= NBC; ++al) a[al] = a[al] + w * b[k][al - 1];
     }
@@ -1468,18 +1561,14 @@ ZFV_HD void reconstruct_lane(const Img &m, int64_t i, const int g, X &xch, const
   load_centre<DIM>(m, i, xc);
   const double len = m.len[i];
   const uint32_t fperm = m.fperm[i];
-
-  // this variable of the scaled reconstruction at x, given the equilibrium
-  // point values (r_eq, E_eq) there; delta is the scaled deviation
   const double inv_len = 1.0 / len;
-  auto eval = [&](const double *x, double r_eq, double E_eq, double &u, double &delta) {
-    double Xs[3] = {(x[0] - xc[0]) * inv_len, (x[1] - xc[1]) * inv_len, DIM == 3 ? (x[2] - xc[2]) * inv_len : 0.0};
-    double px;
-    poly_eval<DIM, DEGC, 1>(reinterpret_cast<const double(*)[1]>(a), cm, Xs, &px);
-    delta = scale_g * px;
-    u = delta;
-    if (eq_sub) u = is_rho ? r_eq + delta : (is_E ? E_eq + delta : 0.0 + delta);
-  };
+
+  // The deviation of this variable, sum_alpha a_alpha (X^alpha - c_alpha): the
+  // variable's scale goes into the coefficients and the moments into the
+  // constant one, so that a point costs one nested evaluation.
+  for (int al = 0; al < DOFC; ++al) a[al] = scale_g * a[al];
+  const double mean = a[0];  // the coefficient of the basis function 1
+  for (int al = 3; al < DOFC; ++al) a[0] = fma(-a[al], cm[al], a[0]);
 
   double s_acc = 0.0;
   const bool gravity_src = (m.gravity != 0) && (src != nullptr);
@@ -1488,42 +1577,78 @@ ZFV_HD void reconstruct_lane(const Img &m, int64_t i, const int g, X &xch, const
   // (this cell's own, solved above: the same solve_exact from the same
   // average) as a state at rest, (0, p_eq n, 0), integrated with the face
   // rule and subtracted.  It has the form of the well-balanced source's face
-  // term, w p_eq (sgn n), so it enters that sum as w p_eq ((sgn - 1) n): the
-  // two cancel at a face whose frame normal points out of the cell.  An
-  // equilibrium that was not found gives NaN, as the reference's zero
-  // extrapolation does.  (Isentropic only: never in the light physics set.)
+  // term, w p_eq n out of the cell, and cancels it there.  An equilibrium that
+  // was not found gives NaN, as the reference's zero extrapolation does.
+  // (Isentropic only: never in the light physics set.)
   const bool eq_flux_bc = PH != PH_LIGHT && m.flux_bc == 2 && gravity_src;
 
+  // The face points along the cell's own vertex order, so that every corner
+  // index is known at compile time; a point's values go to the place of the
+  // same point in the left cell's order, which the face kernel reads.
   const FaceWords cfw = load_face_words(m, i);
+  double V[DIM + 1][3];
+  load_corners<DIM>(m, i, V);
+  // this lane's component of a face's outward normal times the area (momentum
+  // lanes; zero for the others): 2D the turned edge, 3D from the table
+  const bool mom_lane = g >= 1 && g <= DIM;
+  double an2[DIM == 2 ? NF : 1];
+  if (DIM == 2) {
+#pragma unroll
+    for (int f = 0; f < NF; ++f) {
+      const double *p0 = V[face_corner<DIM>(f, 0)], *p1 = V[face_corner<DIM>(f, 1)];
+      an2[DIM == 2 ? f : 0] = g == 1 ? p1[1] - p0[1] : p0[0] - p1[0];
+    }
+  }
+  auto face_normal = [&](int f) -> double {
+    if (!mom_lane || (eq_flux_bc && cfw.w[f] == 2)) return 0.0;
+    if (DIM == 2) return an2[DIM == 2 ? f : 0];
+#if defined(__HIP_DEVICE_COMPILE__)
+    return m.fan[uint32_t(i) * 12u + uint32_t(3 * f + g - 1)];
+#else
+    double v[3];
+    face_normal_out(m, i, f, v);
+    return v[g - 1];
+#endif
+  };
+#pragma unroll
+  for (int k = 0; k < DIM + 1; ++k)
+    for (int d = 0; d < DIM; ++d) V[k][d] = (V[k][d] - xc[d]) * inv_len;
+  const double eq_rho = is_rho ? 1.0 : 0.0, eq_E = is_E ? 1.0 : 0.0;
 #pragma unroll
   for (int f = 0; f < NF; ++f) {
     const int32_t cf = cfw.w[f];
-    double w3[3][3];
-    load_face_vertices<DIM>(m, i, fperm, f, w3);
-    double nn[3], t1[3], t2[3], area;
-    face_frame<DIM>(w3, nn, t1, t2, area);  // (the vertices are needed here anyway)
     const bool exterior = (cf & 2) != 0;
-    // outward normal sign for the source term (src/zisa/math/face.cpp:24-27)
-    double x0f[3];
-    face_point<DIM>(m, 0, w3, x0f);
-    double sgn = 0.0;
-    if (gravity_src && wb) {
-      double dd = nn[0] * (x0f[0] - xc[0]) + nn[1] * (x0f[1] - xc[1]) + (DIM == 3 ? nn[2] * (x0f[2] - xc[2]) : 0.0);
-      sgn = double((0.0 < dd) - (dd < 0.0));
-    }
-    // equilibrium point values of this face: lane k evaluates point q = k
-    // (mod NV), every lane receives all of them
+    // the face's corners in scaled coordinates, then its points
+    double w3[3][3];
+#pragma unroll
+    for (int t = 0; t < DIM; ++t)
+      for (int d = 0; d < 3; ++d) w3[t][d] = d < DIM ? V[face_corner<DIM>(f, t)][d] : 0.0;
+    // equilibrium point values: every lane forms all of them where that is
+    // cheap (PH_LIN); else lane k evaluates point k (mod NV) and every lane
+    // receives them
     double eqr[Q], eqE[Q];
     for (int q = 0; q < Q; ++q) eqr[q] = eqE[q] = 0.0;
-    const bool need_eq = eq_sub && (!exterior || gravity_src);
-    if (need_eq) {
+    const double *pf = m.pot + i * int64_t(NF * Q) + f * Q;
+    if (PH == PH_LIN) {
+      double ph[Q];
+#pragma unroll
+      for (int q = 0; q < Q; ++q) ph[q] = pf[q];
+#pragma unroll
+      for (int q = 0; q < Q; ++q) eq_at_phi<PH>(m, thc, ph[q], eqr[q], eqE[q]);
+    } else if (wb) {
 #pragma unroll
       for (int q0 = 0; q0 < Q; q0 += NV) {
         double my_r = 0.0, my_E = 0.0;
         if (q0 + g < Q) {
-          double x[3];
-          face_point<DIM>(m, q0 + g, w3, x);
-          const double ph = tab ? m.pot[pot_index_face<DIM>(m, Q, f, q0 + g) + i] : phi<DIM, PH>(m, x);
+          double ph;
+          if (tab) {
+            ph = pf[q0 + g];
+          } else {
+            double x[3];
+            face_point<DIM>(m, q0 + g, w3, x);
+            for (int d = 0; d < DIM; ++d) x[d] = fma(x[d], len, xc[d]);
+            ph = phi<DIM, PH>(m, x);
+          }
           eq_at_phi<PH>(m, thc, ph, my_r, my_E);
         }
 #pragma unroll
@@ -1536,28 +1661,28 @@ ZFV_HD void reconstruct_lane(const Img &m, int64_t i, const int g, X &xch, const
         }
       }
     }
-    double fs = 0.0;
-    const double bc_sub = (eq_flux_bc && cf == 2) ? 1.0 : 0.0;
+    double fs = 0.0, u[Q];
 #pragma unroll
     for (int q = 0; q < Q; ++q) {
-      if (!exterior) {
-        double x[3];
-        face_point<DIM>(m, q, w3, x);
-        double u, dl;
-        eval(x, eqr[q], eqE[q], u, dl);
-        // in the global frame: the face kernel rotates the momentum into the
-        // face frame, with every component in one thread
-        fpv[(int64_t(i) * NF + f) * slot_doubles<DIM, Q>() + q * NV + g] = u;
-      }
-      if (gravity_src && eq_sub && g >= 1 && g <= DIM) {
-        double p_eq = eqE[q] * (gamma - 1.0);
-        double w = area * m.fw[q];
-        double t = p_eq * ((sgn - bc_sub) * nn[g - 1]);
-        fs = (q == 0) ? w * t : fma(w, t, fs);
+      double Xs[3];
+      face_point<DIM>(m, q, w3, Xs);
+      u[q] = poly_nested<DIM, DEGC>(a, Xs);
+      if (wb) {
+        u[q] = fma(eq_rho, eqr[q], fma(eq_E, eqE[q], u[q]));
+        fs = fma(m.fw[q], eqE[q], fs);
       }
     }
-    if (gravity_src && wb) s_acc += 1.0 * fs;
+    computed_here<Q>(u);
+    // in the global frame: the face kernel rotates the momentum into the
+    // face frame, with every component in one thread
+    if (!exterior) {
+      double *slot = fpv + (int64_t(i) * NF + f) * slot_doubles<DIM, Q>() + g;
+#pragma unroll
+      for (int q = 0; q < Q; ++q) slot[face_point_in_left_order<DIM, Q>(fperm, f, q) * NV] = u[q];
+    }
+    if (gravity_src && wb) s_acc = fma((gamma - 1.0) * fs, face_normal(f), s_acc);
     if (eq_flux_bc && cf == 2 && !eq_sub) s_acc = __builtin_nan("");
+    schedule_fence();
   }
 
   if (gravity_src) {
@@ -1576,7 +1701,7 @@ ZFV_HD void reconstruct_lane(const Img &m, int64_t i, const int g, X &xch, const
       // other basis function, X^alpha - c_alpha, to zero)
       double gp[3];
       grad_phi<DIM, PH>(m, xc, gp);
-      const double s0 = vol_i * (scale_g * a[0]);
+      const double s0 = vol_i * mean;
 #pragma unroll
       for (int d = 0; d < DIM; ++d) acc[d] = -s0 * gp[d];
     } else if (PH == PH_LIGHT) {
@@ -1585,10 +1710,10 @@ ZFV_HD void reconstruct_lane(const Img &m, int64_t i, const int g, X &xch, const
       load_corners<DIM>(m, i, vtx);
 #pragma unroll 1
       for (int q = 0; q < m.qv; ++q) {
-        double x[3];
+        double x[3], Xs[3] = {0.0, 0.0, 0.0};
         volume_point<DIM>(m, q, vtx, x);
-        double u, dl;
-        eval(x, 0.0, 0.0, u, dl);
+        for (int d = 0; d < DIM; ++d) Xs[d] = (x[d] - xc[d]) * inv_len;
+        const double dl = poly_nested<DIM, DEGC>(a, Xs);
         double gp[3];
         grad_phi<DIM, PH>(m, x, gp);
         const double w = vol_i * m.vw[q];
@@ -1610,12 +1735,11 @@ ZFV_HD void reconstruct_lane(const Img &m, int64_t i, const int g, X &xch, const
           sm[2 * k + 1] = v.hi;
         }
       }
+      // (a[0] holds the constant of the nested form; the basis's is mean)
 #pragma unroll
       for (int al = 0; al < DOFC; ++al)
 #pragma unroll
-        for (int d = 0; d < DIM; ++d) acc[d] = fma(a[al], sm[al * DIM + d], acc[d]);
-#pragma unroll
-      for (int d = 0; d < DIM; ++d) acc[d] = -scale_g * acc[d];
+        for (int d = 0; d < DIM; ++d) acc[d] = fma(al == 0 ? -mean : -a[al], sm[al * DIM + d], acc[d]);
     }
     double cs_ = 0.0;
 #pragma unroll
