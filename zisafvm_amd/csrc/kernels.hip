@@ -103,9 +103,14 @@ struct QuadGroup : WaveGroup {
   }
 };
 
+// Wavefronts per SIMD the reconstruction is compiled for: three leave 168
+// registers, which hold the next chunk's data in flight.  (Four in 2D order 4
+// spill 56 bytes: 20 steps of 263,520 triangles take 13.1 instead of 12.3 ms.)
+constexpr int rec_min_waves(int ph) { return ph == PH_FULL ? 1 : 3; }
+
 // k_reconstruct: blocks of `blockDim.x / 64` waves, 64 / NV cells per wave
 template <int DIM, int DOFC, int RC, int NB, int RB, int Q, int PH>
-__global__ __launch_bounds__(256) void k_reconstruct(
+__global__ __launch_bounds__(256, rec_min_waves(PH)) void k_reconstruct(
     Img m, const double *__restrict__ U, double *__restrict__ fpv, double *__restrict__ src, int skip_far_ghosts) {
   constexpr int NV = DIM + 2;
   constexpr int GPW = groups_per_wave<NV>();
@@ -258,12 +263,34 @@ __global__ __launch_bounds__(256) void k_source_moments(Img m, double *tab) {
   store_source_moments<DIM, DOFC>(m, i, tab);
 }
 
-// the light set's corner potentials
+// the light set's potential values of the cells
 template <int DIM>
-__global__ __launch_bounds__(256) void k_corner_phi(Img m, double *tab) {
+__global__ __launch_bounds__(256) void k_cell_phi(Img m, double *tab) {
   const int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
   if (i >= m.n) return;
-  store_corner_phi<DIM>(m, i, tab);
+  store_cell_phi<DIM>(m, i, tab);
+}
+
+// 2D light set: the instance's bounds on what the series of its equilibrium
+// averages is asked for (Img::es_dist, es_p2), as bits of doubles >= 0
+__global__ __launch_bounds__(256) void k_series_bounds(Img m, int nrows, unsigned long long *out) {
+  const int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
+  double dist = 0.0, p2 = 0.0;
+  if (i < m.n) {
+    p2 = m.cphi[3 * i + 1];
+    for (int r = 0; r < nrows; ++r) {
+      const int32_t e = m.rows[r * m.n + i];
+      dist = fmax(dist, fabs(m.cphi[3 * int64_t(e & ROW_CELL_MASK)] + m.shift_phi[e >> ROW_CELL_BITS] - m.cphi[3 * i]));
+    }
+  }
+  for (int off = 32; off > 0; off >>= 1) {
+    dist = fmax(dist, __shfl_down(dist, off, 64));
+    p2 = fmax(p2, __shfl_down(p2, off, 64));
+  }
+  if ((threadIdx.x & 63) == 0) {
+    atomicMax(out, (unsigned long long)__double_as_longlong(dist));
+    atomicMax(out + 1, (unsigned long long)__double_as_longlong(p2));
+  }
 }
 
 // per-cell potential tables of the cells' own quadrature points
@@ -302,7 +329,7 @@ constexpr int32_t kBatchMaxMembers = 8;
 // one XCD, so the kernels index them by blockIdx directly.
 
 template <int DIM, int DOFC, int RC, int NB, int RB, int Q, int PH>
-__global__ __launch_bounds__(256) void kb_reconstruct(const DevInst *insts, const BlockRef *blk, int stage) {
+__global__ __launch_bounds__(256, rec_min_waves(PH)) void kb_reconstruct(const DevInst *insts, const BlockRef *blk, int stage) {
   constexpr int NV = DIM + 2;
   constexpr int GPW = groups_per_wave<NV>();
   extern __shared__ double slices[];  // as in k_reconstruct
@@ -1034,6 +1061,7 @@ int create_device(zfv_handle *h) {
     HIP_CHECK(hipStreamSynchronize(h->stream));
     m.fan = tab;
   }
+  m.es_dist = m.es_p2 = 0.0;
   h->ph = physics_set(m);
   if (params->gravity != ZFV_GRAVITY_NONE) {
     double *tab = h->alloc<double>(size_t(s.dofc) * s.dim * n);
@@ -1043,16 +1071,30 @@ int create_device(zfv_handle *h) {
     m.smom = tab;
   }
   for (int c = 0; c < 16; ++c) m.shift_phi[c] = s.dim == 2 ? phi<2, PH_LIGHT>(m, m.shift[c]) : phi<3, PH_LIGHT>(m, m.shift[c]);
+  m.phi_unshifted = 1;
+  for (int c = 0; c < 16; ++c)
+    if (m.shift_phi[c] != 0.0) m.phi_unshifted = 0;
   if (h->ph == PH_LIGHT && m.eq != 0) {
-    // member equilibrium averages read the members' corner potentials
+    // member equilibrium averages read the members' potential values
     double *tab = h->alloc<double>(size_t(s.dim + 1) * n);
     if (s.dim == 2)
-      hipLaunchKernelGGL(k_corner_phi<2>, dim3(blocks_for(n, 256)), dim3(256), 0, h->stream, m, tab);
+      hipLaunchKernelGGL(k_cell_phi<2>, dim3(blocks_for(n, 256)), dim3(256), 0, h->stream, m, tab);
     else
-      hipLaunchKernelGGL(k_corner_phi<3>, dim3(blocks_for(n, 256)), dim3(256), 0, h->stream, m, tab);
+      hipLaunchKernelGGL(k_cell_phi<3>, dim3(blocks_for(n, 256)), dim3(256), 0, h->stream, m, tab);
     HIP_CHECK(hipGetLastError());
-    HIP_CHECK(hipStreamSynchronize(h->stream));
     m.cphi = tab;
+    if (s.dim == 2 && exp_average_constants(m, m.es)) {
+      unsigned long long *b = h->alloc<unsigned long long>(2), got[2];
+      hipLaunchKernelGGL(k_fill_u64, dim3(1), dim3(1), 0, h->stream, b, 0ull);
+      hipLaunchKernelGGL(k_fill_u64, dim3(1), dim3(1), 0, h->stream, b + 1, 0ull);
+      hipLaunchKernelGGL(k_series_bounds, dim3(blocks_for(n, 256)), dim3(256), 0, h->stream, m, s.nrows, b);
+      HIP_CHECK(hipGetLastError());
+      HIP_CHECK(hipMemcpyAsync(got, b, sizeof(got), hipMemcpyDeviceToHost, h->stream));
+      HIP_CHECK(hipStreamSynchronize(h->stream));
+      std::memcpy(&m.es_dist, &got[0], sizeof(double));
+      std::memcpy(&m.es_p2, &got[1], sizeof(double));
+    }
+    HIP_CHECK(hipStreamSynchronize(h->stream));
   }
   if (h->ph != PH_LIGHT && params->gravity != ZFV_GRAVITY_NONE) {
     // potential tables of the cells' own quadrature points

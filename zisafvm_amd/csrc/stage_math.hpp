@@ -70,9 +70,18 @@ struct Img {
   // points, n x (alpha DIM + d), each cell's DOFC x DIM values contiguous
   // (store_source_moments), or null
   const double *smom;
-  // the potential at every cell's corners ((d + 1) x n; the light set with an
-  // equilibrium, whose axial potential is affine), or null
+  // the light set with an equilibrium, whose axial potential is affine, or
+  // null; each cell's values contiguous (store_cell_phi).  3D: the potential
+  // at its corners.  2D: the corners' mean and the sums of the squares and
+  // cubes of their deviations from it.
   const double *cphi;
+  // 2D light set: the equilibrium averages in series form (exp_average), used
+  // while the exponents of a cell's stencil stay within its range: bounds over
+  // the instance of |mean of a member - mean of the cell| and of the sums of
+  // squares; 0: not available
+  double es_dist, es_p2;
+  double es[12];
+  int phi_unshifted;  // 1: no translation changes the axial potential (shift_phi all zero)
   // stateful equilibria (steps_per_recompute > 1), or null: per cell theta
   // (2), found flag, EulerScaling (rho, a, E_int) and the equilibrium's own
   // cell average (rho, E) of the last recompute (8 x n), and calls since it
@@ -95,7 +104,7 @@ struct Img {
   double g, axis[3], rhoC, K, G;
   int flux_bc;
   double shift[16][3];  // periodic translations addressed by the row shift code
-  double shift_phi[16];  // axial potential of each translation (added to cphi)
+  double shift_phi[16];  // axial potential of each translation (added to cphi's potentials)
   // normalized quadrature rules
   int qv;                   // points of the volume rule
   double fw[8], fx[8][3];   // face rule: weights, GL abscissa (2D) or barycentric (3D)
@@ -137,6 +146,14 @@ struct state_is_aos<X, std::void_t<decltype(X::kAos)>> : std::bool_constant<X::k
 ZFV_HD int wave_uniform(int v) {
 #if defined(__HIP_DEVICE_COMPILE__)
   return __builtin_amdgcn_readfirstlane(v);
+#else
+  return v;
+#endif
+}
+// true on every active lane of the wavefront if it is on all of them
+ZFV_HD bool wave_all(bool v) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  return __all(v);
 #else
   return v;
 #endif
@@ -195,13 +212,17 @@ constexpr int PH_LIGHT = 0;
 constexpr int PH_FULL = 1;
 constexpr int PH_LIN = 2;
 
+// (an equilibrium of the light set has axial gravity)
+template <int DIM>
+ZFV_HD double axial_phi(const Img &m, const double *x) {
+  double d = x[0] * m.axis[0] + x[1] * m.axis[1];
+  if (DIM == 3) d += x[2] * m.axis[2];
+  return m.g * d;
+}
+
 template <int DIM, int PH = PH_FULL>
 ZFV_HD double phi(const Img &m, const double *x) {
-  if (m.gravity == 1) {
-    double d = x[0] * m.axis[0] + x[1] * m.axis[1];
-    if (DIM == 3) d += x[2] * m.axis[2];
-    return m.g * d;
-  }
+  if (m.gravity == 1) return axial_phi<DIM>(m, x);
   if (PH == PH_LIGHT) return 0.0;
   double r2 = x[0] * x[0] + x[1] * x[1];
   if (DIM == 3) r2 += x[2] * x[2];
@@ -485,12 +506,92 @@ constexpr int frame_words() { return DIM == 2 ? 3 : 7; }
 template <int DIM, int Q>
 constexpr int slot_doubles() { return (Q * (DIM + 2) + 1) & ~1; }
 
-// writes the light set's potential at cell i's corners (tab: (d + 1) n)
+// writes the light set's potential values of cell i (Img::cphi; tab: (d + 1) n)
 template <int DIM>
-ZFV_HD void store_corner_phi(const Img &m, int64_t i, double *tab) {
-  double v[DIM + 1][3];
+ZFV_HD void store_cell_phi(const Img &m, int64_t i, double *tab) {
+  double v[DIM + 1][3], p[DIM + 1];
   load_corners<DIM>(m, i, v);
-  for (int k = 0; k < DIM + 1; ++k) tab[k * m.n + i] = phi<DIM, PH_LIGHT>(m, v[k]);
+  for (int k = 0; k < DIM + 1; ++k) p[k] = phi<DIM, PH_LIGHT>(m, v[k]);
+  if (DIM == 2) {
+    const double mean = (p[0] + p[1] + p[2]) / 3.0;
+    double p2 = 0.0, p3 = 0.0;
+    for (int k = 0; k < 3; ++k) {
+      const double d = p[k] - mean;
+      p2 = fma(d, d, p2);
+      p3 = fma(d * d, d, p3);
+    }
+    p[0] = mean;
+    p[1] = p2;
+    p[2] = p3;
+  }
+  for (int k = 0; k < DIM + 1; ++k) tab[i * (DIM + 1) + k] = p[k];
+}
+template <int DIM>
+ZFV_HD void store_corner_phi(const Img &m, int64_t i, double *tab) { store_cell_phi<DIM>(m, i, tab); }
+
+// ---- the isothermal average over a triangle as a series ----------------------
+// With an affine potential the average of exp(a (phi - mean)) over a cell,
+// sum_q w_q exp(a d_q), depends on the three corner deviations d_k (sum zero)
+// only.  The rules' points come in classes (alpha, beta, beta) of three, at
+// d = (alpha - beta) d_k, and single centroids at d = 0, so
+//   sum_q w_q exp(a d_q) = W + sum_{k >= 2} C_k y_k,
+//   C_k = sum_q w_q (alpha_q - beta_q)^k / (3 k!),   y_k = a^k sum_j d_j^k,
+// and, the sum of the d_j being zero, Newton's identities give every power sum
+// from y_2 and y_3: twelve multiply-adds up to the ninth order instead of an
+// exponential a point.  For y_2 <= kSeriesMaxY2 (|a d| <= 0.125, of which the
+// rules' points reach at most 0.73) the terms left out are below 1e-17.
+constexpr double kSeriesMaxY2 = 0.0234;
+// exp_near reaches full accuracy to this argument
+constexpr double kSeriesMaxArg = 0.25;
+
+// the constants (es) of the instance's volume rule; false: not of that form
+inline bool exp_average_constants(const Img &m, double *es) {
+  double W = 0.0, C[10] = {0};
+  for (int q = 0; q < m.qv; ++q) {
+    const double *x = m.vx[q];
+    double s;
+    if (x[0] == x[1] && x[1] == x[2]) s = 0.0;
+    else if (x[1] == x[2]) s = x[0] - x[1];
+    else if (x[0] == x[2]) s = x[1] - x[0];
+    else if (x[0] == x[1]) s = x[2] - x[0];
+    else return false;
+    W = q == 0 ? m.vw[q] : W + m.vw[q];
+    double t = m.vw[q] / 3.0;
+    for (int k = 1; k < 10; ++k) {
+      t = t * s / k;
+      C[k] += t;
+    }
+  }
+  const double v[12] = {W,        C[2],          C[3],          C[4] / 2,      5 * C[5] / 6, C[6] / 4,
+                        C[6] / 3, 7 * C[7] / 12, C[8] / 8,      4 * C[8] / 9,  3 * C[9] / 8, C[9] / 9};
+  for (int k = 0; k < 12; ++k) es[k] = v[k];
+  return true;
+}
+
+ZFV_HD double exp_average(const Img &m, double y2, double y3) {
+  const double *e = m.es;
+  const double s0 = fma(y2, fma(y2, fma(y2, fma(y2, e[8], e[5]), e[3]), e[1]), e[0]);
+  const double s2 = fma(y3, e[11], fma(y2, e[9], e[6]));
+  const double s1 = fma(y3, s2, fma(y2, fma(y2, fma(y2, e[10], e[7]), e[4]), e[2]));
+  return fma(y3, s1, s0);
+}
+
+// exp(z) for |z| <= kSeriesMaxArg, to the last place or so: its Taylor
+// polynomial of degree 12 (the first term left out is below 3e-18)
+ZFV_HD double exp_near(double z) {
+  double r = 1.0 / 479001600;
+  r = fma(r, z, 1.0 / 39916800);
+  r = fma(r, z, 1.0 / 3628800);
+  r = fma(r, z, 1.0 / 362880);
+  r = fma(r, z, 1.0 / 40320);
+  r = fma(r, z, 1.0 / 5040);
+  r = fma(r, z, 1.0 / 720);
+  r = fma(r, z, 1.0 / 120);
+  r = fma(r, z, 1.0 / 24);
+  r = fma(r, z, 1.0 / 6);
+  r = fma(r, z, 0.5);
+  r = fma(r, z, 1.0);
+  return fma(r, z, 1.0);
 }
 
 // writes the frames of cell i's local faces (tab has frame_words (d+1) n entries)
@@ -1028,13 +1129,16 @@ ZFV_HD void reconstruct_lane(const Img &m, int64_t i, const int g, X &xch, const
   double uk[NV];
   gather(0, uk);
 
-  double vtx[DIM + 1][3];
-  load_corners<DIM>(m, i, vtx);
+  // The 2D light set's averages in series form (exp_average) where the
+  // exponents over every member of every cell of this wavefront are in range
+  constexpr bool SERIES = DIM == 2 && PH == PH_LIGHT;
+  const bool wb = PH == PH_LIN || m.eq != 0;
 
   // The potential at the cell's own quadrature points: from the instance's
   // tables in the full sets (always present in PH_LIN), else evaluated.
   const bool tab = PH == PH_LIN || (PH == PH_FULL && m.pot != nullptr);
   auto vol_phi = [&](int q, const double *x) {
+    if (PH == PH_LIGHT) return axial_phi<DIM>(m, x);  // (asked for with an equilibrium only)
     return tab ? m.pot[pot_index_vol<DIM>(m, Q, q) + i] : phi<DIM, PH>(m, x);
   };
 
@@ -1048,6 +1152,8 @@ ZFV_HD void reconstruct_lane(const Img &m, int64_t i, const int g, X &xch, const
       return;
     }
     const double vol_i = m.vol[i];
+    double vtx[DIM + 1][3];
+    load_corners<DIM>(m, i, vtx);
     double pr = 0.0, pE = 0.0;
     for (int q = g; q < m.qv; q += NV) {
       double x[3];
@@ -1071,12 +1177,21 @@ ZFV_HD void reconstruct_lane(const Img &m, int64_t i, const int g, X &xch, const
   double th[2] = {0.0, 0.0};
   double phi_ref = 0.0;
   double ar1 = -1.0;  // isothermal: the average of exp(a (phi - phi_ref)) over the cell, once solved
-  const bool wb = PH == PH_LIN || m.eq != 0;
   bool eq_found = false;
+  double y_p2 = 0.0, y_p3 = 0.0;  // the cell's own power sums (SERIES)
   if (wb) {
-    double xref[3];
-    volume_point<DIM>(m, 0, vtx, xref);
-    phi_ref = vol_phi(0, xref);
+    // the potential the equilibrium is written against: the first volume
+    // point's, in the 2D light set the corners' mean
+    if (SERIES) {
+      phi_ref = m.cphi[3 * i];
+      y_p2 = m.cphi[3 * i + 1];
+      y_p3 = m.cphi[3 * i + 2];
+    } else {
+      double xref[3], vtx[DIM + 1][3];
+      load_corners<DIM>(m, i, vtx);
+      volume_point<DIM>(m, 0, vtx, xref);
+      phi_ref = vol_phi(0, xref);
+    }
   }
   // Stateful equilibria (LocalReconstruction::recompute_equilibrium,
   // include/zisa/reconstruction/local_reconstruction.hpp:87-100): between
@@ -1106,8 +1221,12 @@ ZFV_HD void reconstruct_lane(const Img &m, int64_t i, const int g, X &xch, const
       }
     }
   }
+  // the series is in range at temperature RT for every cell of the wavefront
+  auto series_ok = [&](double RT) {
+    const bool ok = m.es_dist > 0.0 && m.es_dist <= kSeriesMaxArg * RT && m.es_p2 <= kSeriesMaxY2 * (RT * RT);
+    return wave_all(ok);
+  };
   if (wb && !reuse) {
-    double vol_i = m.vol[i];
     // cell average of the equilibrium with parameters t over this cell
     auto cell_avg = [&](const double *t, double &ar, double &aE) {
       group_avg(eq_consts<PH>(m, t, phi_ref), ar, aE);
@@ -1116,7 +1235,12 @@ ZFV_HD void reconstruct_lane(const Img &m, int64_t i, const int g, X &xch, const
       double RT = (gamma - 1.0) * Eint0 / rho0;
       double t1[2] = {1.0, RT};
       double ar, aE;
-      cell_avg(t1, ar, aE);
+      if (SERIES && series_ok(RT)) {
+        const double a1 = -1.0 / RT;
+        ar = exp_average(m, a1 * a1 * y_p2, a1 * a1 * a1 * y_p3);
+      } else {
+        cell_avg(t1, ar, aE);
+      }
       ar1 = ar;
       th[0] = rho0 / ar;
       th[1] = RT;
@@ -1207,6 +1331,8 @@ ZFV_HD void reconstruct_lane(const Img &m, int64_t i, const int g, X &xch, const
   EqC thc = eq_consts<PH>(m, th, phi_ref);
   if (!eq_sub) thc.th0 = thc.th1 = thc.phi_ref = thc.a = thc.b = 0.0;
 
+  const bool series = SERIES && wb && series_ok(eq_sub ? th[1] : 1.0e300);
+  const double aa = thc.a * thc.a;
   // equilibrium average of this cell's equilibrium over a member cell given
   // its (translated) corners and volume
   auto member_avg = [&](const double (*w3)[3], double vol_j, double &er, double &eE) {
@@ -1268,6 +1394,9 @@ ZFV_HD void reconstruct_lane(const Img &m, int64_t i, const int g, X &xch, const
       // average is th0 ar1 (to rounding), with E = b rho pointwise
       if (ar1 > 0.0) {
         er = th[0] * ar1;
+        eE = er * thc.b;
+      } else if (series) {
+        er = th[0] * exp_average(m, aa * y_p2, aa * thc.a * y_p3);
         eE = er * thc.b;
       } else {
         own_eq(er, eE);
@@ -1340,9 +1469,13 @@ ZFV_HD void reconstruct_lane(const Img &m, int64_t i, const int g, X &xch, const
     // scaled deviation of row k of the chunk in this lane's variable
     // (the equilibrium parts enter with factors 1 or 0: u - 1 er = u - er
     // and x - 0 eE = x exactly, so this equals the branchy form bit for bit)
-    const double f_rho = (wb && is_rho) ? 1.0 : 0.0, f_E = (wb && is_E) ? 1.0 : 0.0;
+    // In the light set the energy average is the density average times the
+    // cell constant b, so one factor serves each lane.
+    const double f_rho = (wb && is_rho) ? 1.0 : ((PH == PH_LIGHT && wb && is_E) ? thc.b : 0.0);
+    const double f_E = (PH != PH_LIGHT && wb && is_E) ? 1.0 : 0.0;
     auto deviation = [&](double u, double er, double eE) {
-      const double d = fma(-f_E, eE, fma(-f_rho, er, u));
+      double d = fma(-f_rho, er, u);
+      if (PH != PH_LIGHT) d = fma(-f_E, eE, d);
       return fma(d, inv_g, -q0);
     };
     // what the equilibrium average over a member (row entry rw) needs: its potential
@@ -1354,16 +1487,19 @@ ZFV_HD void reconstruct_lane(const Img &m, int64_t i, const int g, X &xch, const
       double pm, pv;
       double sphi;  // light set: the translation's potential, added at use
       int lin;
+      int32_t cell;  // 2D light set: the member, for averages out of the series' range
     };
     auto load_member = [&](int32_t entry, Member &mb) {
       const int64_t j = entry & ROW_CELL_MASK;
       const int code = entry >> ROW_CELL_BITS;
       if (PH == PH_LIGHT) {
-        // the member's corner potentials in w3[k][0] and its translation's
-        // potential, added where they are used (so that the loads stay in
-        // flight until then)
-        for (int k = 0; k < DIM + 1; ++k) mb.w3[k][0] = m.cphi[k * n + j];
-        mb.sphi = m.shift_phi[code];
+        // the member's potential values (cphi) in w3[k][0] and its
+        // translation's potential, added where they are used (so that the
+        // loads stay in flight until then)
+        const double *cp = m.cphi + uint32_t(j) * uint32_t(DIM + 1);
+        for (int k = 0; k < DIM + 1; ++k) mb.w3[k][0] = cp[k];
+        mb.sphi = m.phi_unshifted ? 0.0 : m.shift_phi[code];
+        mb.cell = int32_t(j);
         return;
       }
       mb.lin = PH == PH_LIN || (PH == PH_FULL && linear_isentropic(m) && code == 0) ? 1 : 0;
@@ -1383,6 +1519,28 @@ ZFV_HD void reconstruct_lane(const Img &m, int64_t i, const int g, X &xch, const
         linear_isentropic_avg(thc, mb.pm, mb.pv, er, eE);
       } else if (PH == PH_LIGHT) {
         double w3[DIM + 1][3];
+        if (SERIES) {
+          if (series) {
+            // th0 exp(a (mean - phi_ref)) times the average about the mean
+            const double z = (mb.w3[0][0] + (mb.sphi - thc.phi_ref)) * thc.a;
+            er = thc.th0 * (exp_near(z) * exp_average(m, aa * mb.w3[1][0], aa * thc.a * mb.w3[2][0]));
+            eE = er * thc.b;
+            return;
+          }
+          // out of the series' range: the rule's points one by one
+          load_corners<DIM>(m, mb.cell, w3);
+          for (int k = 0; k < DIM + 1; ++k) w3[k][0] = axial_phi<DIM>(m, w3[k]) + (mb.sphi - thc.phi_ref);
+          double se = 0.0;
+#pragma unroll 1
+          for (int q = 0; q < m.qv; ++q) {
+            double ph = m.vx[q][0] * w3[0][0];
+            for (int k = 1; k < DIM + 1; ++k) ph = fma(m.vx[q][k], w3[k][0], ph);
+            se = fma(m.vw[q], exp(ph * thc.a), se);
+          }
+          er = thc.th0 * se;
+          eE = er * thc.b;
+          return;
+        }
         for (int k = 0; k < DIM + 1; ++k) w3[k][0] = mb.w3[k][0] + mb.sphi;
         member_avg(w3, mb.vol, er, eE);
       } else {
@@ -1391,10 +1549,10 @@ ZFV_HD void reconstruct_lane(const Img &m, int64_t i, const int g, X &xch, const
     };
     // a one-sided row whose member is also a central row takes that row's
     // averages from LDS (the same values: same member, same function)
-    // instead of loading the member and averaging again; not in PH_LIN,
-    // whose member averages cost less than the lookup
+    // instead of loading the member and averaging again; not in PH_LIN and
+    // in series form, where a member average costs less than the lookup
     auto twin_of = [&](int ch) {
-      if (PH == PH_LIN || !eq_sub || ch < CCH || g >= RB) return -1;
+      if (PH == PH_LIN || series || !eq_sub || ch < CCH || g >= RB) return -1;
       return int(m.twin[(chunk_row0(ch) + g - RC) * n + i]);
     };
     for (int k = 0; k < NB; ++k)
@@ -1430,7 +1588,7 @@ ZFV_HD void reconstruct_lane(const Img &m, int64_t i, const int g, X &xch, const
         } else {
           member_avg_of(mc, er, eE);
         }
-        if (PH != PH_LIN && ch < CCH && g < cnt) {
+        if (PH != PH_LIN && !series && ch < CCH && g < cnt) {
           ceq[2 * (ch * NV + g)] = er;
           ceq[2 * (ch * NV + g) + 1] = eE;
         }
@@ -1441,13 +1599,11 @@ ZFV_HD void reconstruct_lane(const Img &m, int64_t i, const int g, X &xch, const
 #pragma unroll
       for (int k = 0; k < NV; ++k) {
         if (k >= cnt) break;
-        // in the light set the energy average is the density average times
-        // the cell constant b (member_avg)
         const double *row = pl + k * ROWW;
         double er = 0.0, eE = 0.0;
         if (wb) {
           er = row[NC];
-          eE = PH == PH_LIGHT ? er * thc.b : row[NC + 1];
+          if (PH != PH_LIGHT) eE = row[NC + 1];
         }
         const double d = deviation(uc[k], er, eE);
         if (ch < CCH) {
@@ -1610,6 +1766,13 @@ ZFV_HD void reconstruct_lane(const Img &m, int64_t i, const int g, X &xch, const
     return v[g - 1];
 #endif
   };
+  // in series form: the exponents a (phi - phi_ref) at the corners
+  double zc[DIM + 1];
+  for (int k = 0; k < DIM + 1; ++k) zc[k] = 0.0;
+  if (series) {
+#pragma unroll
+    for (int k = 0; k < DIM + 1; ++k) zc[k] = (axial_phi<DIM>(m, V[k]) - thc.phi_ref) * thc.a;
+  }
 #pragma unroll
   for (int k = 0; k < DIM + 1; ++k)
     for (int d = 0; d < DIM; ++d) V[k][d] = (V[k][d] - xc[d]) * inv_len;
@@ -1635,6 +1798,14 @@ ZFV_HD void reconstruct_lane(const Img &m, int64_t i, const int g, X &xch, const
       for (int q = 0; q < Q; ++q) ph[q] = pf[q];
 #pragma unroll
       for (int q = 0; q < Q; ++q) eq_at_phi<PH>(m, thc, ph[q], eqr[q], eqE[q]);
+    } else if (series) {
+      // (within an exponent of 0.125: exp_near)
+#pragma unroll
+      for (int q = 0; q < Q; ++q) {
+        const double xi = m.fx[q][0], z0 = zc[face_corner<DIM>(f, 0)], z1 = zc[face_corner<DIM>(f, 1)];
+        eqr[q] = thc.th0 * exp_near(fma(0.5 + 0.5 * xi, z1, (0.5 - 0.5 * xi) * z0));
+        eqE[q] = eqr[q] * thc.b;
+      }
     } else if (wb) {
 #pragma unroll
       for (int q0 = 0; q0 < Q; q0 += NV) {
@@ -1647,7 +1818,7 @@ ZFV_HD void reconstruct_lane(const Img &m, int64_t i, const int g, X &xch, const
             double x[3];
             face_point<DIM>(m, q0 + g, w3, x);
             for (int d = 0; d < DIM; ++d) x[d] = fma(x[d], len, xc[d]);
-            ph = phi<DIM, PH>(m, x);
+            ph = PH == PH_LIGHT ? axial_phi<DIM>(m, x) : phi<DIM, PH>(m, x);
           }
           eq_at_phi<PH>(m, thc, ph, my_r, my_E);
         }
@@ -1707,6 +1878,7 @@ ZFV_HD void reconstruct_lane(const Img &m, int64_t i, const int g, X &xch, const
     } else if (PH == PH_LIGHT) {
       // constant gradient, rules that do not integrate the basis exactly:
       // the quadrature over the points
+      double vtx[DIM + 1][3];
       load_corners<DIM>(m, i, vtx);
 #pragma unroll 1
       for (int q = 0; q < m.qv; ++q) {
