@@ -993,6 +993,7 @@ int create_device(zfv_handle *h) {
   m.rhoC = params->polytrope_rhoC;
   m.K = params->polytrope_K;
   m.G = params->polytrope_G;
+  eq_pow_constants(params->gamma, m.eq_half, m.eq_db);
   m.flux_bc = params->flux_bc;
   m.spr = params->steps_per_recompute;
   m.eq_threshold = params->recompute_threshold;

@@ -102,6 +102,10 @@ struct Img {
   int eq;        // 0 none, 1 isentropic, 2 isothermal
   int gravity;   // 0 none, 1 axial, 2 radial, 3 polytrope
   double g, axis[3], rhoC, K, G;
+  // isentropic equilibrium: 1/(gamma - 1) = eq_half / 2 + eq_db to the last
+  // place, where it is a multiple of 1/2 up to rounding (eq_pow); eq_half 0: not
+  int eq_half;
+  double eq_db;
   int flux_bc;
   double shift[16][3];  // periodic translations addressed by the row shift code
   double shift_phi[16];  // axial potential of each translation (added to cphi's potentials)
@@ -220,6 +224,18 @@ ZFV_HD double axial_phi(const Img &m, const double *x) {
   return m.g * d;
 }
 
+// the n = 1 polytrope's potential at radius r.  (A call on the device: the
+// member averages' point loops are unrolled many times, and as many copies of
+// the sine overflow the instruction cache.)
+#if defined(__HIP_DEVICE_COMPILE__)
+__device__ __attribute__((noinline))
+#endif
+inline double polytrope_phi(double rhoC, double K, double G, double r) {
+  const double alpha = sqrt(2.0 * 3.14159265358979323846 * G / K);
+  const double ce = alpha * (r + 2.2250738585072014e-308);
+  return -2.0 * K * rhoC * sin(ce) / ce;
+}
+
 template <int DIM, int PH = PH_FULL>
 ZFV_HD double phi(const Img &m, const double *x) {
   if (m.gravity == 1) return axial_phi<DIM>(m, x);
@@ -228,11 +244,7 @@ ZFV_HD double phi(const Img &m, const double *x) {
   if (DIM == 3) r2 += x[2] * x[2];
   double r = sqrt(r2);
   if (m.gravity == 2) return m.g * r;
-  if (m.gravity == 3) {
-    double alpha = sqrt(2.0 * 3.14159265358979323846 * m.G / m.K);
-    double ce = alpha * (r + 2.2250738585072014e-308);
-    return -2.0 * m.K * m.rhoC * sin(ce) / ce;
-  }
+  if (m.gravity == 3) return polytrope_phi(m.rhoC, m.K, m.G, r);
   return 0.0;
 }
 
@@ -258,28 +270,9 @@ ZFV_HD void grad_phi(const Img &m, const double *x, double *gp) {
 }
 
 // ---- local equilibrium: theta -> (rho, E) at x ------------------------------
-template <int DIM, int PH = PH_FULL>
-ZFV_HD void eq_eval(const Img &m, const double *th, double phi_ref, const double *x, double &rho, double &E) {
-  const double gamma = m.gamma;
-  if (PH != PH_LIGHT && m.eq == 1) {
-    double h = th[0] + phi_ref - phi<DIM, PH>(m, x);
-    double K = th[1];
-    double base = 1.0 / K * (gamma - 1.0) / gamma * h;
-    rho = pow(base, 1.0 / (gamma - 1.0));
-    double p = K * pow(rho, gamma);
-    E = p / (gamma - 1.0);
-  } else {
-    double RT = th[1];
-    rho = th[0] * exp(-(phi<DIM, PH>(m, x) - phi_ref) / RT);
-    E = rho * RT / (gamma - 1.0);
-  }
-}
-
-// The same equilibrium with its per-cell constants hoisted out of the point
-// loops: isentropic (the reference's): a = (1/K)(gamma-1)/gamma and
-// b = 1/(gamma-1), the very subexpressions eq_eval forms at every point, so
-// the values are identical; isothermal (an extension): a = -1/RT and
-// b = RT/(gamma-1), which replace two divisions per point by products.
+// With the per-cell constants taken out of the point loops: isentropic (the
+// reference's) a = (1/K)(gamma-1)/gamma and b = 1/(gamma-1); isothermal (an
+// extension) a = -1/RT and b = RT/(gamma-1).
 struct EqC {
   double th0, th1, phi_ref, a, b;
 };
@@ -302,11 +295,52 @@ ZFV_HD EqC eq_consts(const Img &m, const double *th, double phi_ref) {
 
 // x^y with the exponents an ideal gas of gamma = 2 (the n = 1 polytrope)
 // produces, 1 and 2, done exactly (x^1 = x; x^2 is one correctly rounded
-// product); any other exponent goes to pow
+// product); any other exponent goes to pow.  (A call: the equilibrium's point
+// loops are unrolled many times, and as many copies of pow overflow the
+// instruction cache.)
+#if defined(__HIP_DEVICE_COMPILE__)
+__device__ __attribute__((noinline)) inline double pow_call(double x, double y) { return pow(x, y); }
+#else
+inline double pow_call(double x, double y) { return pow(x, y); }
+#endif
 ZFV_HD double ipow(double x, double y) {
   if (y == 1.0) return x;
   if (y == 2.0) return x * x;
-  return pow(x, y);
+  return pow_call(x, y);
+}
+
+// x^(1/(gamma-1)).  For the common gases (gamma = 7/5, 5/3, 4/3, 3/2, 2 ...)
+// the exponent is a half of a small whole number up to its last place: a
+// product of a few factors and a square root, and the last place as a first
+// order correction (a single precision logarithm is enough for that).  The
+// exponents of double precision's pow cost about twenty times as much.
+ZFV_HD double eq_pow(const Img &m, double x, double b) {
+  if (m.eq_half > 0 && x > 1.0e-30 && x < 1.0e30) {
+    double r = (m.eq_half & 1) ? sqrt(x) : 1.0, f = x;
+    for (int k = m.eq_half >> 1; k > 0; k >>= 1) {
+      if (k & 1) r = r * f;
+      f = f * f;
+    }
+#if defined(__HIP_DEVICE_COMPILE__)
+    const double l = double(__logf(float(x)));
+#else
+    const double l = double(logf(float(x)));
+#endif
+    return fma(r, m.eq_db * l, r);
+  }
+  return ipow(x, b);
+}
+
+// eq_half and eq_db of a gas (host)
+inline void eq_pow_constants(double gamma, int &half, double &db) {
+  const double b = 1.0 / (gamma - 1.0);
+  const double k = nearbyint(2.0 * b);
+  half = 0;
+  db = 0.0;
+  if (k >= 1.0 && k <= 30.0 && fabs(b - 0.5 * k) <= 8.0 * 2.220446049250313e-16 * b) {
+    half = int(k);
+    db = b - 0.5 * k;
+  }
 }
 
 // the equilibrium at a point of potential ph
@@ -314,10 +348,11 @@ template <int PH>
 ZFV_HD void eq_at_phi(const Img &m, const EqC &c, double ph, double &rho, double &E) {
   if (PH != PH_LIGHT && m.eq == 1) {
     double h = c.th0 + c.phi_ref - ph;
-    // PH_LIN has gamma = 2: the exponents are 1 and 2, as ipow takes them
-    rho = PH == PH_LIN ? c.a * h : ipow(c.a * h, c.b);
-    double p = c.th1 * (PH == PH_LIN ? rho * rho : ipow(rho, m.gamma));
-    E = PH == PH_LIN ? p : p / (m.gamma - 1.0);
+    // PH_LIN has gamma = 2: the exponents are 1 and 2.  Else, with base =
+    // a h and rho = base^b: p = K rho^gamma = K rho base, which is
+    // (gamma - 1)/gamma rho h, so that E needs no power of its own
+    rho = PH == PH_LIN ? c.a * h : eq_pow(m, c.a * h, c.b);
+    E = PH == PH_LIN ? c.th1 * (rho * rho) : rho * h / m.gamma;
   } else {
     rho = c.th0 * exp((ph - c.phi_ref) * c.a);
     E = rho * c.b;
@@ -1176,7 +1211,9 @@ ZFV_HD void reconstruct_lane(const Img &m, int64_t i, const int g, X &xch, const
   // local equilibrium of this cell: every lane solves it (identical results)
   double th[2] = {0.0, 0.0};
   double phi_ref = 0.0;
-  double ar1 = -1.0;  // isothermal: the average of exp(a (phi - phi_ref)) over the cell, once solved
+  // once solved, the equilibrium's average over the cell as the solve has it
+  // (isothermal: in ar1 that of exp(a (phi - phi_ref)))
+  double ar1 = -1.0, aE1 = 0.0;
   bool eq_found = false;
   double y_p2 = 0.0, y_p3 = 0.0;  // the cell's own power sums (SERIES)
   if (wb) {
@@ -1246,49 +1283,80 @@ ZFV_HD void reconstruct_lane(const Img &m, int64_t i, const int g, X &xch, const
       th[1] = RT;
       eq_found = true;
     } else {
-      // quasi-Newton with a central finite-difference Jacobian
-      // (include/zisa/math/quasi_newton.hpp:12-50)
-      double p = Eint0 * (gamma - 1.0);
-      double guess[2] = {gamma / (gamma - 1.0) * p / rho0, p / (PH == PH_LIN ? rho0 * rho0 : ipow(rho0, gamma))};
-      double atol[2] = {1e-13 * guess[0], 1e-13 * guess[1]};
+      // The reference's quasi-Newton iteration (its guess, tolerance, limits
+      // and convergence test: include/zisa/math/quasi_newton.hpp:12-50) with
+      // the Jacobian in closed form instead of by central differences, one
+      // evaluation an iteration instead of five.  With rho = (a h)^b, E = rho
+      // h / gamma, averages R, Eavg and D = avg(rho / h):
+      //   dR/dh = b D, dEavg/dh = b R, dR/dK = -b R / K, dEavg/dK = -b Eavg / K
+      const double p = Eint0 * (gamma - 1.0);
+      const double guess[2] = {gamma / (gamma - 1.0) * p / rho0, p / (PH == PH_LIN ? rho0 * rho0 : ipow(rho0, gamma))};
+      const double atol[2] = {1e-13 * guess[0], 1e-13 * guess[1]};
       double x0 = guess[0], x1 = guess[1];
-      auto f = [&](double a, double b, double &f0, double &f1) {
-        double t[2] = {a, b};
-        double ar, aE;
-        cell_avg(t, ar, aE);
-        f0 = rho0 - ar;
-        f1 = Eint0 - aE;
+      const double bexp = PH == PH_LIN ? 1.0 : 1.0 / (gamma - 1.0);
+      const bool linear = PH == PH_LIN || linear_isentropic(m);
+      // the potential at this lane's volume points q = g (mod NV)
+      constexpr int QL = (16 + NV - 1) / NV;
+      double phq[PH == PH_LIN ? 1 : QL];
+      if (!linear) {
+        double vtx[DIM + 1][3];
+        load_corners<DIM>(m, i, vtx);
+#pragma unroll
+        for (int k = 0; k < (PH == PH_LIN ? 1 : QL); ++k) {
+          phq[k] = 0.0;
+          if (g + k * NV >= m.qv) continue;
+          double x[3];
+          volume_point<DIM>(m, g + k * NV, vtx, x);
+          phq[k] = vol_phi(g + k * NV, x);
+        }
+      }
+      double R, E, D;  // averages of the equilibrium of (x0, x1)
+      auto average = [&]() {
+        const double t[2] = {x0, x1};
+        const EqC tc = eq_consts<PH>(m, t, phi_ref);
+        if (linear) {
+          linear_isentropic_avg(tc, m.phim[2 * i], m.phim[2 * i + 1], R, E);
+          D = tc.a;
+          return;
+        }
+        double pr = 0.0, pE = 0.0, pD = 0.0;
+#pragma unroll
+        for (int k = 0; k < (PH == PH_LIN ? 1 : QL); ++k) {
+          if (g + k * NV >= m.qv) continue;
+          double r, e;
+          eq_at_phi<PH>(m, tc, phq[k], r, e);
+          const double w = m.vw[g + k * NV];
+          pr = fma(w, r, pr);
+          pE = fma(w, e, pE);
+          pD = fma(w, r / (tc.th0 + tc.phi_ref - phq[k]), pD);
+        }
+        R = xch.bcast(pr, 0);
+        E = xch.bcast(pE, 0);
+        D = xch.bcast(pD, 0);
+#pragma unroll
+        for (int k = 1; k < NV; ++k) {
+          R = R + xch.bcast(pr, k);
+          E = E + xch.bcast(pE, k);
+          D = D + xch.bcast(pD, k);
+        }
       };
-      double fx0, fx1;
-      f(x0, x1, fx0, fx1);
+      average();
+      double fx0 = rho0 - R, fx1 = Eint0 - E;
       double dx0 = 2.0 * atol[0] + 1.0, dx1 = 2.0 * atol[1] + 1.0;
       double h00 = 0, h01 = 0, h10 = 0, h11 = 0;  // previous two steps
       bool ok = true;
       int iter = 0;
       while (!(fabs(dx0) <= atol[0] && fabs(dx1) <= atol[1]) && iter < 20) {
-        double J00, J01, J10, J11;
-        {
-          double e = 1e-6 * fabs(x0);
-          double fp0, fp1, fm0, fm1;
-          f(x0 + 0.5 * e, x1, fp0, fp1);
-          f(x0 - 0.5 * e, x1, fm0, fm1);
-          J00 = (fp0 - fm0) / e;
-          J01 = (fp1 - fm1) / e;
-        }
-        {
-          double e = 1e-6 * fabs(x1);
-          double fp0, fp1, fm0, fm1;
-          f(x0, x1 + 0.5 * e, fp0, fp1);
-          f(x0, x1 - 0.5 * e, fm0, fm1);
-          J10 = (fp0 - fm0) / e;
-          J11 = (fp1 - fm1) / e;
-        }
-        double inv_det = 1.0 / (J00 * J11 - J01 * J10);
+        const double bk = bexp / x1;
+        const double J00 = -bexp * D, J01 = -bexp * R, J10 = bk * R, J11 = bk * E;
+        const double inv_det = 1.0 / (J00 * J11 - J01 * J10);
         dx0 = inv_det * (J11 * fx0 - J10 * fx1);
         dx1 = inv_det * (-J01 * fx0 + J00 * fx1);
         x0 -= dx0;
         x1 -= dx1;
-        f(x0, x1, fx0, fx1);
+        average();
+        fx0 = rho0 - R;
+        fx1 = Eint0 - E;
         if (iter >= 4 && !(dx0 <= atol[0] && dx1 <= atol[1])) {
           double rate0 = log(fabs(dx0) / fabs(h10)) / log(fabs(h10) / fabs(h00));
           double rate1 = log(fabs(dx1) / fabs(h11)) / log(fabs(h11) / fabs(h01));
@@ -1305,6 +1373,8 @@ ZFV_HD void reconstruct_lane(const Img &m, int64_t i, const int g, X &xch, const
         th[0] = x0;
         th[1] = x1;
         eq_found = true;
+        ar1 = R;
+        aE1 = E;
       }
     }
   }
@@ -1329,7 +1399,10 @@ ZFV_HD void reconstruct_lane(const Img &m, int64_t i, const int g, X &xch, const
   // that its evaluations need no branch)
   const bool eq_sub = wb && eq_found;
   EqC thc = eq_consts<PH>(m, th, phi_ref);
-  if (!eq_sub) thc.th0 = thc.th1 = thc.phi_ref = thc.a = thc.b = 0.0;
+  if (!eq_sub) {
+    thc.th0 = thc.th1 = thc.phi_ref = thc.a = 0.0;
+    if (!(PH != PH_LIGHT && m.eq == 1)) thc.b = 0.0;  // (isentropic: the exponent)
+  }
 
   const bool series = SERIES && wb && series_ok(eq_sub ? th[1] : 1.0e300);
   const double aa = thc.a * thc.a;
@@ -1392,7 +1465,10 @@ ZFV_HD void reconstruct_lane(const Img &m, int64_t i, const int g, X &xch, const
       // isothermal: the equilibrium is th0 times the function the solve just
       // averaged over this cell (same points, weights and order), so its own
       // average is th0 ar1 (to rounding), with E = b rho pointwise
-      if (ar1 > 0.0) {
+      if (ar1 > 0.0 && PH != PH_LIGHT && m.eq == 1) {
+        er = ar1;
+        eE = aE1;
+      } else if (ar1 > 0.0) {
         er = th[0] * ar1;
         eE = er * thc.b;
       } else if (series) {
