@@ -1,16 +1,16 @@
 // gfx950 kernels of the rate-of-change hot path and the C-ABI of
 // libzfv_hip.so (declared in include/zfv.h).
 //
-// One SSP3 stage = three launches over arrays in HBM:
+// One SSP3 stage = two launches over arrays in HBM:
 //   k_reconstruct  one group of nvars lanes per cell (lane g: variable g):
 //                  stencil gather, LSQ pseudo-inverse mat-vecs, CWENO/WENO-AO,
 //                  equilibrium solve (well-balanced), point values on the
 //                  cell's faces (face frame), gravity source
-//   k_face_flux    one thread per interior face: HLLC/Rusanov at the face
-//                  points, integrated once per face, in the global frame
-//                  times the face's area
-//   k_update       one thread per cell: atomic-free gather of the cell's face
-//                  fluxes, source, flux BC, Butcher-form stage sum, frozen BC
+//   k_update       one lane per cell face: HLLC/Rusanov at the face points,
+//                  integrated over the face, in the global frame times the
+//                  face's area; then one lane per cell and variable: the sum
+//                  of the cell's fluxes, source, flux BC, Butcher-form stage
+//                  sum, frozen BC
 // FP64 throughout; no MFMA (the per-cell mat-vecs are memory-bound).
 #include <hip/hip_runtime.h>
 
@@ -138,61 +138,126 @@ __global__ __launch_bounds__(256, rec_min_waves(PH)) void k_reconstruct(
   }
 }
 
-template <int DIM, int Q>
-__global__ __launch_bounds__(256) void k_face_flux(Img m, const double *__restrict__ fpv, double *__restrict__ G) {
-  const int64_t e = xcd_block(blockIdx.x, gridDim.x) * blockDim.x + threadIdx.x;
-  if (e >= m.ne) return;
-  face_flux<DIM, Q>(m, e, fpv, G);
-}
-
 struct StageCoeffs {
-  double c[4];  // coefficients of k_0 .. k_stage in the next state's sum
-  int nk;       // number of k's in the sum (stage + 1)
+  double c[2];  // coefficients of the earlier stages' tendencies in the next state's sum
+  double cl;    // and of this stage's own
   int write_rate_only;  // 1: store L in K[stage] and stop (zfv_rate)
 };
 
-// k_update: K[stage] = L(Ustage); Unext = U0 + dt * sum_j c_j K[j]
-// (src/zisa/ode/runge_kutta.cpp:122-143), then FrozenBC for ghost cells.
-// Ustage, U0 and Unext may name the same buffer (stages 1 and 2 read and
-// write the stage state X; a thread reads only its own cell's entries before
-// it writes them), so none of them is declared __restrict__.
-template <int DIM>
-__global__ __launch_bounds__(256) void k_update(Img m, StageCoeffs sc, int stage, double dt, const double *dtp,
-                                                const double *Ustage, const double *__restrict__ G,
-                                                const double *__restrict__ src, const double *U0,
-                                                double *__restrict__ K, double *Unext) {
+// What a stage's update reads and writes: K[stage] = L(Ustage); Unext = U0 +
+// dt * sum_j c_j K[j] (src/zisa/ode/runge_kutta.cpp:122-143), then FrozenBC for
+// ghost cells.  Ustage, U0 and Unext may name the same buffer (stages 1 and 2
+// read and write the stage state X; a wavefront reads only its own cells'
+// entries, before it writes them), so none of them is declared __restrict__.
+struct UpdateArgs {
+  StageCoeffs sc;
+  int stage;
+  double dt;
+  const double *Ustage, *fpv, *src, *U0;
+  double *K, *Unext;
+};
+
+// Cells of an update wavefront: as many as have about 64 faces between them
+// along the cells' Hilbert order (32 triangles 58 on average and 66 at most on
+// the jittered lattices, 20 tetrahedra 62 and 68 in the ball), and of a block
+constexpr int update_cells_of_wave(int dim) { return dim == 2 ? 32 : 20; }
+constexpr int update_cells_of_block(int dim) { return 4 * update_cells_of_wave(dim); }
+
+// The update of a wavefront's tile of cells.  First each lane forms the flux
+// through one of the tile's faces (build_update_tiles; a face between two tiles
+// is evaluated by both, with the same operands in the same order: conservation
+// holds bit for bit), then one lane per cell and variable sums its cell's
+// fluxes, which it reads from LDS (lds: NF CW NV doubles).  Bound by latency:
+// a wavefront is one chain of entry, point values, flux, sum, so everything
+// the sum needs is loaded first.  Against a kernel over faces and one over
+// cells it does without a flux array in memory and takes one launch less:
+// 263,520 triangles (3 points a face) 44 -> 34 us, 201,196 tetrahedra 42 -> 38,
+// 1,152 triangles 9.4 -> 4.8.  (One lane per cell face, every face evaluated
+// twice: 48, 50 and 5.0 us; four wavefronts per SIMD spill in 3D: 54 us.)
+template <int DIM, int Q>
+__device__ __forceinline__ void update_cells(const Img &m, const UpdateArgs &a, double dt, int64_t tile, int lane, double *lds) {
   constexpr int NV = DIM + 2;
-  if (dtp) dt = *dtp;  // the step's dt chosen on the device (zfv_advance)
-  const int64_t i = xcd_block(blockIdx.x, gridDim.x) * blockDim.x + threadIdx.x;
+  constexpr int NF = DIM + 1;
+  constexpr int CW = update_cells_of_wave(DIM);
+  constexpr int NP = (CW * NV + 63) / 64;  // passes over the tile's cells and variables
   const int64_t n = m.n;
-  if (i >= n) return;
-  if (!sc.write_rate_only && m.steady != nullptr && (m.meta[i] & META_FAR_GHOST) == META_FAR_GHOST) {
-    // frozen far ghost: its tendency is never used
-    for (int v = 0; v < NV; ++v) {
-      K[(int64_t(stage) * n + i) * NV + v] = 0.0;
-      Unext[i * NV + v] = m.steady[i * NV + v];
-    }
-    return;
-  }
-  double L[NV];
-  cell_rate<DIM, true>(m, i, Ustage, G, src, L);
-  // the last stage's tendency enters only its own sum (no later stage reads it)
-  if (sc.write_rate_only || stage + 1 < 3)
-    for (int v = 0; v < NV; ++v) K[(int64_t(stage) * n + i) * NV + v] = L[v];
-  if (sc.write_rate_only) return;
-  const bool ghost = (m.meta[i] & 16) != 0 && m.steady != nullptr;
-  for (int v = 0; v < NV; ++v) {
-    double dudt = 0.0;
-    for (int j = 0; j < sc.nk; ++j) {
-      if (sc.c[j] != 0.0) {
-        const double kj = (j == stage) ? L[v] : K[(int64_t(j) * n + i) * NV + v];
-        dudt += sc.c[j] * kj;
+  const int64_t i0 = tile * CW;
+  const UpdateFace mine = reinterpret_cast<const UpdateFace *>(m.uent)[tile * 64 + lane];
+  const int more0 = m.uoff[tile], more1 = m.uoff[tile + 1];
+  // What the second part needs besides the fluxes is loaded first, to be in
+  // flight with the faces' entries and point values
+  double part[NP], base[NP], src[NP], vol[NP];
+  uint32_t word[NP];
+  bool store[NP];
+#pragma unroll
+  for (int p = 0; p < NP; ++p) {
+    const int e = p * 64 + lane, c = e / NV;
+    int64_t i = i0 + c;
+    store[p] = e < CW * NV && i < n;
+    i = store[p] ? i : i0;
+    const int64_t at = i * NV + (e - c * NV);
+    const int32_t meta = m.meta[i];
+    word[p] = m.ucell[i];
+    vol[p] = m.vol[i];
+    src[p] = m.gravity != 0 && a.src != nullptr ? a.src[at] : 0.0;
+    part[p] = base[p] = 0.0;
+    if (!a.sc.write_rate_only) {
+      base[p] = a.U0[at];
+#pragma unroll
+      for (int j = 0; j < 2; ++j)
+        if (j < a.stage && a.sc.c[j] != 0.0) part[p] += a.sc.c[j] * a.K[int64_t(j) * NV * n + at];
+      // frozen ghost cells keep the steady state whatever their fluxes
+      if ((meta & 16) != 0 && m.steady != nullptr) {
+        a.Unext[at] = m.steady[at];
+        store[p] = false;
       }
     }
-    double un = U0[i * NV + v] + dt * dudt;
-    if (ghost) un = m.steady[i * NV + v];
-    Unext[i * NV + v] = un;
   }
+  UpdateFace face = mine;
+  for (int k = lane; face.l >= 0;) {
+    double g[NV];
+    update_face_flux<DIM, Q>(m, face, a.Ustage, a.fpv, g);
+#pragma unroll
+    for (int v = 0; v < NV; ++v) lds[k * NV + v] = g[v];
+    k += 64;  // (tiles of more than 64 faces)
+    if (k >= 64 + more1 - more0) break;
+    face = reinterpret_cast<const UpdateFace *>(m.umore)[more0 + k - 64];
+  }
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+#pragma unroll
+  for (int p = 0; p < NP; ++p) {
+    if (!store[p]) continue;
+    const int e = p * 64 + lane, v = e % NV;
+    const int64_t at = i0 * NV + e;
+    double L = 0.0;
+#pragma unroll
+    for (int f = 0; f < NF; ++f) {
+      const uint32_t k = (word[p] >> (8 * f)) & 127u;
+      const bool right = (word[p] >> (8 * f)) & 128u;
+      if (k != UPDATE_NO_FACE) {
+        const double g = lds[k * NV + v];
+        L += right ? g : -g;
+      }
+    }
+    L = L / vol[p];
+    if (m.gravity != 0 && a.src != nullptr) L += src[p];
+    // the last stage's tendency enters only its own sum (no later stage reads it)
+    if (a.sc.write_rate_only || a.stage < 2) a.K[int64_t(a.stage) * NV * n + at] = L;
+    if (a.sc.write_rate_only) continue;
+    a.Unext[at] = base[p] + dt * (part[p] + a.sc.cl * L);
+  }
+}
+
+template <int DIM, int Q>
+__global__ __launch_bounds__(256, 3) void k_update(Img m, UpdateArgs a, const double *dtp) {
+  __shared__ double flux[4][update_cells_of_wave(DIM) * (DIM + 1) * (DIM + 2)];
+  const double dt = dtp ? *dtp : a.dt;  // zfv_advance: the step's dt, chosen on the device
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int64_t tile = xcd_block(blockIdx.x, gridDim.x) * 4 + wave;
+  if (tile * update_cells_of_wave(DIM) >= m.n) return;
+  update_cells<DIM, Q>(m, a, dt, tile, threadIdx.x & 63, flux[wave]);
 }
 
 // LocalCFL: min_i inradius_i / (|v_i| + a_i); positive doubles order like
@@ -343,14 +408,41 @@ __global__ __launch_bounds__(256, rec_min_waves(PH)) void kb_reconstruct(const D
                                                       x);
 }
 
+// one block updates update_cells_of_block cells of a member
 template <int DIM, int Q>
-__global__ __launch_bounds__(256) void kb_face_flux(const DevInst *insts, const BlockRef *blk) {
-  kb_face_flux_thread<DIM, Q>(insts, blk[blockIdx.x], threadIdx.x);
-}
-
-template <int DIM>
-__global__ __launch_bounds__(256) void kb_update(DevInst *insts, const BlockRef *blk, int stage) {
-  kb_update_thread<DIM, true>(insts, blk[blockIdx.x], threadIdx.x, stage);
+__global__ __launch_bounds__(256, 3) void kb_update(DevInst *insts, const BlockRef *blk, int stage, StageCoeffs sc) {
+  __shared__ double flux[4][update_cells_of_wave(DIM) * (DIM + 1) * (DIM + 2)];
+  const BlockRef b = blk[blockIdx.x];
+  if (b.inst < 0) return;
+  DevInst &d = insts[b.inst];
+  if (!d.active) return;
+  UpdateArgs a;
+  a.sc = sc;
+  a.stage = stage;
+  a.dt = 0.0;
+  double dt = d.dt;
+  if (stage == 0) {
+    // the step's dt, from the CFL minimum of this step: every thread of the
+    // member forms the same value; the member's first thread records it for
+    // the later stages and the step's end (and stops a member that cannot
+    // advance, whose threads all leave here)
+    dt = kb_step_dt(d);
+    if (b.local == 0 && threadIdx.x == 0) {
+      d.dt = dt;
+      if (!(dt > 0.0)) d.active = 0;
+    }
+    if (!(dt > 0.0)) return;
+  }
+  a.Ustage = stage == 0 ? d.U : d.X;
+  a.fpv = d.fpv;
+  a.src = d.src;
+  a.U0 = d.U;
+  a.K = d.K;
+  a.Unext = stage == 2 ? d.U : d.X;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int64_t tile = int64_t(b.local) * 4 + wave;
+  if (tile * update_cells_of_wave(DIM) >= d.m.n) return;
+  update_cells<DIM, Q>(d.m, a, dt, tile, threadIdx.x & 63, flux[wave]);
 }
 
 template <int DIM>
@@ -484,18 +576,23 @@ __global__ __launch_bounds__(256) void k_copy_probe(const double2 *__restrict__ 
 // ---------------------------------------------------------------------------
 // launch plan for one shape
 
+static StageCoeffs ssp3_coeffs(int stage) {
+  // next-state coefficients after stage s: a[s+1][:] and b for the last stage
+  // (src/zisa/ode/runge_kutta.cpp:154-165)
+  if (stage == 0) return StageCoeffs{{0.0, 0.0}, 1.0, 0};
+  if (stage == 1) return StageCoeffs{{0.25, 0.0}, 0.25, 0};
+  return StageCoeffs{{1.0 / 6, 1.0 / 6}, 2.0 / 3, 0};
+}
+
 struct Launcher {
   // rec[ph]: physics set ph (PH_LIGHT / PH_FULL / PH_LIN); cfg: reconstruction
   // launch configuration (rec_cfg_waves)
   void (*rec[3])(const Img &, const double *, double *, double *, int cfg, int skip_far_ghosts, hipStream_t);
-  void (*face)(const Img &, const double *, double *, hipStream_t);
-  void (*update)(const Img &, StageCoeffs, int, double, const double *, const double *, const double *,
-                 const double *, const double *, double *, double *, hipStream_t);
+  void (*update)(const Img &, const UpdateArgs &, const double *dtp, hipStream_t);
   void (*cfl)(const Img &, const double *, unsigned long long *, hipStream_t);
   void (*source_moments)(const Img &, double *, hipStream_t);  // setup: Img::smom
   // batched variants: grid = number of block-table entries
   void (*brec[3])(DevInst *, const BlockRef *, unsigned, int, int cfg, hipStream_t);
-  void (*bface)(DevInst *, const BlockRef *, unsigned, hipStream_t);
   void (*bupdate)(DevInst *, const BlockRef *, unsigned, int, hipStream_t);
   void (*bcfl)(DevInst *, const BlockRef *, unsigned, hipStream_t);
   int dim = 2;
@@ -545,14 +642,8 @@ Launcher make_launcher() {
   l.rec[PH_LIN] = [](const Img &m, const double *U, double *fpv, double *src, int cfg, int skip, hipStream_t s) {
     launch_rec<DIM, DOFC, RC, NB, RB, Q, PH_LIN>(m, U, fpv, src, cfg, skip, s);
   };
-  l.face = [](const Img &m, const double *fpv, double *G, hipStream_t s) {
-    if (m.ne > 0)
-      hipLaunchKernelGGL((k_face_flux<DIM, Q>), dim3(xcd_grid(m.ne, 256)), dim3(256), 0, s, m, fpv, G);
-  };
-  l.update = [](const Img &m, StageCoeffs sc, int stage, double dt, const double *dtp, const double *Us,
-                const double *G, const double *src, const double *U0, double *K, double *Un, hipStream_t s) {
-    hipLaunchKernelGGL((k_update<DIM>), dim3(xcd_grid(m.n, 256)), dim3(256), 0, s, m, sc, stage, dt, dtp, Us, G,
-                       src, U0, K, Un);
+  l.update = [](const Img &m, const UpdateArgs &a, const double *dtp, hipStream_t s) {
+    hipLaunchKernelGGL((k_update<DIM, Q>), dim3(xcd_grid(m.n, update_cells_of_block(DIM))), dim3(256), 0, s, m, a, dtp);
   };
   l.cfl = [](const Img &m, const double *U, unsigned long long *out, hipStream_t s) {
     hipLaunchKernelGGL((k_cfl<DIM>), dim3(std::min(blocks_for(m.n, 256), 512u)), dim3(256), 0, s, m, U, out);
@@ -566,11 +657,8 @@ Launcher make_launcher() {
   l.brec[PH_LIN] = [](DevInst *d, const BlockRef *b, unsigned nb, int stage, int cfg, hipStream_t s) {
     launch_brec<DIM, DOFC, RC, NB, RB, Q, PH_LIN>(d, b, nb, stage, cfg, s);
   };
-  l.bface = [](DevInst *d, const BlockRef *b, unsigned nb, hipStream_t s) {
-    hipLaunchKernelGGL((kb_face_flux<DIM, Q>), dim3(nb), dim3(256), 0, s, d, b);
-  };
   l.bupdate = [](DevInst *d, const BlockRef *b, unsigned nb, int stage, hipStream_t s) {
-    hipLaunchKernelGGL((kb_update<DIM>), dim3(nb), dim3(256), 0, s, d, b, stage);
+    hipLaunchKernelGGL((kb_update<DIM, Q>), dim3(nb), dim3(256), 0, s, d, b, stage, ssp3_coeffs(stage));
   };
   l.bcfl = [](DevInst *d, const BlockRef *b, unsigned nb, hipStream_t s) {
     hipLaunchKernelGGL((kb_cfl<DIM>), dim3(nb), dim3(256), 0, s, d, b);
@@ -616,7 +704,7 @@ struct zfv_handle {
   std::vector<void *> allocations;
   int64_t device_bytes = 0;
   // state buffers (device)
-  double *U = nullptr, *X = nullptr, *K = nullptr, *fpv = nullptr, *G = nullptr, *src = nullptr;
+  double *U = nullptr, *X = nullptr, *K = nullptr, *fpv = nullptr, *src = nullptr;
   double *steady = nullptr;
   unsigned long long *dt_bits = nullptr;
   double *host_stage = nullptr;  // pinned staging n * nvars
@@ -703,27 +791,6 @@ static void check_device() {
     throw ZfvError(ZFV_ERR_NO_DEVICE, std::string("libzfv_hip is built for gfx950; device is ") + prop.gcnArchName);
 }
 
-static StageCoeffs ssp3_coeffs(int stage) {
-  // next-state coefficients after stage s: a[s+1][:] and b for the last stage
-  // (src/zisa/ode/runge_kutta.cpp:154-165)
-  StageCoeffs c{};
-  if (stage == 0) {
-    c.c[0] = 1.0;
-    c.nk = 1;
-  } else if (stage == 1) {
-    c.c[0] = 0.25;
-    c.c[1] = 0.25;
-    c.nk = 2;
-  } else {
-    c.c[0] = 1.0 / 6;
-    c.c[1] = 1.0 / 6;
-    c.c[2] = 2.0 / 3;
-    c.nk = 3;
-  }
-  c.write_rate_only = 0;
-  return c;
-}
-
 // the image with stateful equilibria switched off: its launches recompute
 // every cell's equilibrium and leave the kept ones and their counters alone
 static Img stateless(const Img &m) {
@@ -760,8 +827,8 @@ static void tune_rec(zfv_handle *h, const double *Ustate) {
         if (k >= 0) HIP_CHECK(hipEventRecord(ev[2 * k], h->stream));
         h->L.rec[h->ph](m, Ustate, h->fpv, h->src, c, frozen(h), h->stream);
         if (k >= 0) HIP_CHECK(hipEventRecord(ev[2 * k + 1], h->stream));
-        h->L.face(m, h->fpv, h->G, h->stream);
-        h->L.update(m, rate_only, 0, 0.0, nullptr, Ustate, h->G, h->src, Ustate, h->K, nullptr, h->stream);
+        h->L.update(m, UpdateArgs{rate_only, 0, 0.0, Ustate, h->fpv, h->src, Ustate, h->K, nullptr}, nullptr,
+                    h->stream);
       }
       HIP_CHECK(hipEventSynchronize(ev[2 * kTimed - 1]));
       HIP_CHECK(hipGetLastError());
@@ -793,9 +860,8 @@ static void enqueue_step(zfv_handle *h, double dt) {
   const double *Us = h->U;
   for (int s = 0; s < 3; ++s) {
     h->L.rec[h->ph](m, Us, h->fpv, h->src, h->rec_cfg, frozen(h), h->stream);
-    h->L.face(m, h->fpv, h->G, h->stream);
     double *Un = (s == 2) ? h->U : h->X;
-    h->L.update(m, ssp3_coeffs(s), s, dt, nullptr, Us, h->G, h->src, h->U, h->K, Un, h->stream);
+    h->L.update(m, UpdateArgs{ssp3_coeffs(s), s, dt, Us, h->fpv, h->src, h->U, h->K, Un}, nullptr, h->stream);
     Us = h->X;
   }
 }
@@ -823,9 +889,8 @@ static void enqueue_adaptive_step(zfv_handle *h, bool reject, int cfg, AdvState 
   const double *Us = h->U;
   for (int s = 0; s < 3; ++s) {
     h->L.rec[h->ph](m, Us, h->fpv, h->src, cfg, frozen(h), h->stream);
-    h->L.face(m, h->fpv, h->G, h->stream);
     double *Un = (s == 2) ? h->U : h->X;
-    h->L.update(m, ssp3_coeffs(s), s, 0.0, &adv->dt, Us, h->G, h->src, h->U, h->K, Un, h->stream);
+    h->L.update(m, UpdateArgs{ssp3_coeffs(s), s, 0.0, Us, h->fpv, h->src, h->U, h->K, Un}, &adv->dt, h->stream);
     Us = h->X;
   }
   if (reject) {
@@ -1015,9 +1080,8 @@ int create_device(zfv_handle *h) {
   const int nv = s.nvars;
   h->U = h->alloc<double>(size_t(nv) * n);
   h->X = h->alloc<double>(size_t(nv) * n);
-  h->K = h->alloc<double>(size_t(3) * nv * n);
+  h->K = h->alloc<double>(size_t(2) * nv * n);  // the last stage's tendency is not stored
   h->fpv = h->alloc<double>(size_t(s.nfaces) * ((s.q * nv + 1) & ~1) * n);  // Q x NV per cell-face slot, even
-  h->G = h->alloc<double>(size_t(nv) * std::max<int64_t>(im.ne, 1));
   if (params->gravity != ZFV_GRAVITY_NONE) h->src = h->alloc<double>(size_t(nv) * n);
   h->dt_bits = h->alloc<unsigned long long>(1);
   if (params->equilibrium == ZFV_EQ_ISENTROPIC && params->gravity != ZFV_GRAVITY_NONE && params->gamma == 2.0) {
@@ -1031,7 +1095,7 @@ int create_device(zfv_handle *h) {
     m.phim = pm;
   }
   {
-    // face frames of every cell's local faces
+    // normals and areas of every cell's local faces
     double *tab = h->alloc<double>(size_t(s.dim == 2 ? 3 * frame_words<2>() : 4 * frame_words<3>()) * n);
     if (s.dim == 2)
       hipLaunchKernelGGL(k_face_frames<2>, dim3(blocks_for(n, 256)), dim3(256), 0, h->stream, m, tab);
@@ -1042,7 +1106,7 @@ int create_device(zfv_handle *h) {
     m.frm = tab;
   }
   {
-    // the interior faces' frames in face order, for the face kernel
+    // the interior faces' normals and areas in face order, for the fluxes
     double *tab = h->alloc<double>(size_t(s.dim == 2 ? frame_words<2>() : frame_words<3>()) * std::max<int64_t>(im.ne, 1));
     if (im.ne > 0) {
       if (s.dim == 2)
@@ -1061,6 +1125,15 @@ int create_device(zfv_handle *h) {
     HIP_CHECK(hipGetLastError());
     HIP_CHECK(hipStreamSynchronize(h->stream));
     m.fan = tab;
+  }
+  {
+    std::vector<int32_t> off, entries, more;
+    std::vector<uint32_t> words;
+    build_update_tiles(im, update_cells_of_wave(s.dim), params->flux_bc == ZFV_FLUX_BC_CONSTANT, entries, off, more, words);
+    m.uoff = h->upload(off);
+    m.uent = h->upload(entries);
+    m.umore = h->upload(more);
+    m.ucell = h->upload(words);
   }
   m.es_dist = m.es_p2 = 0.0;
   h->ph = physics_set(m);
@@ -1221,10 +1294,9 @@ int zfv_rate(zfv_handle *h, const double *u, double *dudt, double t) {
   HIP_CHECK(hipMemcpyAsync(h->X, h->host_stage, sizeof(double) * nv * n, hipMemcpyHostToDevice, h->stream));
   const Img &m = h->dimg;
   h->L.rec[h->ph](m, h->X, h->fpv, h->src, rec_config(h, h->X), 0, h->stream);
-  h->L.face(m, h->fpv, h->G, h->stream);
   StageCoeffs sc{};
   sc.write_rate_only = 1;
-  h->L.update(m, sc, 0, 0.0, nullptr, h->X, h->G, h->src, h->X, h->K, h->X, h->stream);
+  h->L.update(m, UpdateArgs{sc, 0, 0.0, h->X, h->fpv, h->src, h->X, h->K, h->X}, nullptr, h->stream);
   HIP_CHECK(hipGetLastError());
   HIP_CHECK(hipMemcpyAsync(h->host_stage, h->K, sizeof(double) * nv * n, hipMemcpyDeviceToHost, h->stream));
   HIP_CHECK(hipStreamSynchronize(h->stream));
@@ -1393,10 +1465,11 @@ int zfv_get_info(zfv_handle *h, zfv_info *info) {
   const double rec = 8.0 * s.m + 4.0 * s.nrows + 8.0 * nv + 8.0 * (s.nfaces * s.dim + s.dim + 2 + s.nmom) +
                      4.0 * (1 + s.nfaces + 1) + tables +
                      8.0 * (2.0 * ne / n) * s.q * nv + (h->src ? 8.0 * nv : 0.0);
-  const double face = (ne / n) * (8.0 * 2 * s.q * nv + 8.0 * nv + 4.0 * 2 + 8.0 * frame);
-  const double upd = 4.0 * s.nfaces + 8.0 * s.nfaces * nv + 8.0 + 4.0 + 8.0 * nv * 5;
+  // the update: each face's point values on both sides and its frame once, per
+  // cell its face word, volume, meta, source and stage arrays
+  const double upd = (ne / n) * (8.0 * 2 * s.q * nv + 8.0 * frame + 16.0) + 4.0 + 8.0 + 4.0 + 8.0 * nv * 5;
   info->recon_bytes_per_cell = rec;
-  info->bytes_per_cell_stage = rec + face + upd;
+  info->bytes_per_cell_stage = rec + upd;
   int maxs = 0;
   for (size_t i = 0; i + 1 < h->img.l2g_off.size(); ++i)
     maxs = std::max(maxs, h->img.l2g_off[i + 1] - h->img.l2g_off[i]);
@@ -1441,7 +1514,7 @@ int zfv_time_kernels(zfv_handle *h, int32_t n_steps, double dt, zfv_kernel_times
   ZFV_API_BEGIN
   const Img m = stateless(h->dimg);
   const int cfg = rec_config(h, h->U);
-  std::vector<hipEvent_t> ev(2 * 9 * std::max(n_steps, 1));
+  std::vector<hipEvent_t> ev(2 * 6 * std::max(n_steps, 1));
   for (auto &e : ev) HIP_CHECK(hipEventCreate(&e));
   int k = 0;
   for (int st = 0; st < n_steps; ++st) {
@@ -1450,12 +1523,9 @@ int zfv_time_kernels(zfv_handle *h, int32_t n_steps, double dt, zfv_kernel_times
       HIP_CHECK(hipEventRecord(ev[k++], h->stream));
       h->L.rec[h->ph](m, Us, h->fpv, h->src, cfg, frozen(h), h->stream);
       HIP_CHECK(hipEventRecord(ev[k++], h->stream));
-      HIP_CHECK(hipEventRecord(ev[k++], h->stream));
-      h->L.face(m, h->fpv, h->G, h->stream);
-      HIP_CHECK(hipEventRecord(ev[k++], h->stream));
       double *Un = (s == 2) ? h->U : h->X;
       HIP_CHECK(hipEventRecord(ev[k++], h->stream));
-      h->L.update(m, ssp3_coeffs(s), s, dt, nullptr, Us, h->G, h->src, h->U, h->K, Un, h->stream);
+      h->L.update(m, UpdateArgs{ssp3_coeffs(s), s, dt, Us, h->fpv, h->src, h->U, h->K, Un}, nullptr, h->stream);
       HIP_CHECK(hipEventRecord(ev[k++], h->stream));
       Us = h->X;
     }
@@ -1463,14 +1533,12 @@ int zfv_time_kernels(zfv_handle *h, int32_t n_steps, double dt, zfv_kernel_times
   HIP_CHECK(hipGetLastError());
   HIP_CHECK(hipStreamSynchronize(h->stream));
   zfv_kernel_times t{};
-  for (int q = 0; q < k; q += 6) {
-    float a = 0, b = 0, c = 0;
+  for (int q = 0; q < k; q += 4) {
+    float a = 0, b = 0;
     HIP_CHECK(hipEventElapsedTime(&a, ev[q], ev[q + 1]));
     HIP_CHECK(hipEventElapsedTime(&b, ev[q + 2], ev[q + 3]));
-    HIP_CHECK(hipEventElapsedTime(&c, ev[q + 4], ev[q + 5]));
     t.reconstruct_ms += a;
-    t.face_flux_ms += b;
-    t.update_ms += c;
+    t.update_ms += b;
     t.n_launches += 1;
   }
   for (auto &e : ev) (void)hipEventDestroy(e);
@@ -1489,7 +1557,7 @@ int zfv_estimate_device_bytes(const zfv_mesh *mesh, const zfv_params *params, in
   double per_cell = 8.0 * s.m + 4.0 * s.nrows + 1.0 * (s.nrows - s.rc) +
                     8.0 * ((s.dim == 2 ? 6 : 16) + s.dim + 3 + s.nmom) + 4.0 * (2 + 4) +
                     8.0 * s.nfaces * frame +    // face frames
-                    8.0 * nv * (1 + 1 + 3);     // U, X, K[3]
+                    8.0 * nv * (1 + 1 + 2);     // U, X, K[2]
   if (params->gravity != ZFV_GRAVITY_NONE) {
     per_cell += 8.0 * nv;                       // source
     per_cell += 8.0 * 2;                        // potential moments
@@ -1501,7 +1569,8 @@ int zfv_estimate_device_bytes(const zfv_mesh *mesh, const zfv_params *params, in
   if (params->equilibrium != ZFV_EQ_NONE) per_cell += 8.0 * s.nfaces;  // corner potentials (light set)
   if (params->equilibrium != ZFV_EQ_NONE && s.dim == 3) per_cell += 8.0 * 12;  // outward area normals
   if (params->gravity != ZFV_GRAVITY_NONE) per_cell += 8.0 * s.dofc * s.dim;  // source moments
-  double per_face = 8.0 * nv + 4.0 * 2 + 8.0 * frame;  // fluxes, the two slots, the frame and area
+  per_cell += 4.0 + 16.0 * 64 / update_cells_of_wave(s.dim) + 1.0;  // the update's face words, entries and offsets
+  double per_face = 4.0 * 2 + 8.0 * frame;      // the two slots, the frame and area
   *bytes = int64_t(n * per_cell + ne * per_face) + (1 << 20);
   return ZFV_OK;
   ZFV_API_END
@@ -1580,14 +1649,14 @@ struct zfv_batch {
   zfv::Shape shape{};
   hipStream_t stream = nullptr;
   int max_inst = 0;
-  int64_t cap_cell_blocks = 0, cap_face_blocks = 0, cap_rec_blocks = 0;
-  int64_t n_cell_blocks = 0, n_face_blocks = 0, n_rec_blocks = 0;  // current launch sizes
+  int64_t cap_cell_blocks = 0, cap_face_blocks = 0, cap_upd_blocks = 0, cap_rec_blocks = 0;
+  int64_t n_cell_blocks = 0, n_upd_blocks = 0, n_rec_blocks = 0;  // current launch sizes
   bool xcd_chunks = true;
   int rec_cfg = -1;   // reconstruction launch configuration; -1 = not tuned yet
   double rec_ms[zfv::kRecConfigs] = {0, 0, 0};
   int ph = 0;         // physics set: the widest any member needs
   zfv::DevInst *d_inst = nullptr;
-  zfv::BlockRef *d_bcell = nullptr, *d_bface = nullptr, *d_brec = nullptr;
+  zfv::BlockRef *d_bcell = nullptr, *d_bupd = nullptr, *d_brec = nullptr;
   std::vector<zfv::DevInst> h_inst;
   std::vector<zfv_handle *> members;
   hipGraphExec_t graph = nullptr;
@@ -1600,7 +1669,7 @@ struct zfv_batch {
     if (graph) (void)hipGraphExecDestroy(graph);
     if (d_inst) (void)hipFree(d_inst);
     if (d_bcell) (void)hipFree(d_bcell);
-    if (d_bface) (void)hipFree(d_bface);
+    if (d_bupd) (void)hipFree(d_bupd);
     if (d_brec) (void)hipFree(d_brec);
     if (stream) (void)hipStreamDestroy(stream);
   }
@@ -1641,12 +1710,14 @@ static void member_settle(zfv_handle *h) {
 }
 
 static void batch_upload(zfv_batch *b) {
-  std::vector<int64_t> cells(b->max_inst, 0), faces(b->max_inst, 0);
+  std::vector<int64_t> cells(b->max_inst, 0);
+  int64_t face_blocks = 0;
   for (int s = 0; s < b->max_inst; ++s)
     if (b->members[s] && b->h_inst[s].active) {
       cells[s] = b->h_inst[s].m.n;
-      faces[s] = b->h_inst[s].m.ne;
+      face_blocks += (b->h_inst[s].m.ne + 255) / 256;
     }
+  if (face_blocks > b->cap_face_blocks) throw ZfvError(ZFV_ERR_MEMORY, "batch capacity exceeded");
   int ph = -1;
   for (int s = 0; s < b->max_inst; ++s)
     if (b->members[s] && b->h_inst[s].active) {
@@ -1660,14 +1731,14 @@ static void batch_upload(zfv_batch *b) {
   }
   b->ph = ph;
   auto tc = checked_table(cells, 256, b->cap_cell_blocks, b->xcd_chunks);
-  auto tf = checked_table(faces, 256, b->cap_face_blocks, b->xcd_chunks);
+  auto tu = checked_table(cells, update_cells_of_block(b->shape.dim), b->cap_upd_blocks, b->xcd_chunks);
   const int waves = rec_cfg_waves(b->rec_cfg >= 0 ? b->rec_cfg : kRecConfigs - 1);
   auto tr = checked_table(cells, int64_t(waves) * b->L.groups_per_wave, b->cap_rec_blocks, b->xcd_chunks);
-  if (int64_t(tc.size()) != b->n_cell_blocks || int64_t(tf.size()) != b->n_face_blocks ||
+  if (int64_t(tc.size()) != b->n_cell_blocks || int64_t(tu.size()) != b->n_upd_blocks ||
       int64_t(tr.size()) != b->n_rec_blocks) {
     // launch sizes change: the step graph is captured again on the next run
     b->n_cell_blocks = int64_t(tc.size());
-    b->n_face_blocks = int64_t(tf.size());
+    b->n_upd_blocks = int64_t(tu.size());
     b->n_rec_blocks = int64_t(tr.size());
     if (b->graph) {
       HIP_CHECK(hipGraphExecDestroy(b->graph));
@@ -1677,7 +1748,7 @@ static void batch_upload(zfv_batch *b) {
   HIP_CHECK(hipMemcpyAsync(b->d_inst, b->h_inst.data(), sizeof(DevInst) * b->max_inst, hipMemcpyHostToDevice,
                            b->stream));
   HIP_CHECK(hipMemcpyAsync(b->d_bcell, tc.data(), sizeof(BlockRef) * tc.size(), hipMemcpyHostToDevice, b->stream));
-  HIP_CHECK(hipMemcpyAsync(b->d_bface, tf.data(), sizeof(BlockRef) * tf.size(), hipMemcpyHostToDevice, b->stream));
+  HIP_CHECK(hipMemcpyAsync(b->d_bupd, tu.data(), sizeof(BlockRef) * tu.size(), hipMemcpyHostToDevice, b->stream));
   HIP_CHECK(hipMemcpyAsync(b->d_brec, tr.data(), sizeof(BlockRef) * tr.size(), hipMemcpyHostToDevice, b->stream));
   HIP_CHECK(hipStreamSynchronize(b->stream));
   b->dirty = false;
@@ -1740,15 +1811,14 @@ static bool batch_has_active(const zfv_batch *b) {
 }
 
 static void batch_enqueue_step(zfv_batch *b) {
-  const unsigned nc = unsigned(b->n_cell_blocks), nf = unsigned(b->n_face_blocks), nr = unsigned(b->n_rec_blocks);
+  const unsigned nc = unsigned(b->n_cell_blocks), nu = unsigned(b->n_upd_blocks), nr = unsigned(b->n_rec_blocks);
   const unsigned ib = unsigned((b->max_inst + 63) / 64);
   // the step's CFL minimum (reset at the end of the previous step or when
   // the member joined); stage 0's update turns it into the step's dt
   b->L.bcfl(b->d_inst, b->d_bcell, nc, b->stream);
   for (int s = 0; s < 3; ++s) {
     b->L.brec[b->ph](b->d_inst, b->d_brec, nr, s, b->rec_cfg, b->stream);
-    b->L.bface(b->d_inst, b->d_bface, nf, b->stream);
-    b->L.bupdate(b->d_inst, b->d_bcell, nc, s, b->stream);
+    b->L.bupdate(b->d_inst, b->d_bupd, nu, s, b->stream);
   }
   hipLaunchKernelGGL(kb_end_step, dim3(ib), dim3(64), 0, b->stream, b->d_inst, b->max_inst);
 }
@@ -1795,11 +1865,13 @@ int zfv_batch_create(const zfv_params *params, int64_t cell_capacity, int64_t fa
   auto round8 = [](int64_t x) { return ((x + 7) / 8) * 8; };
   b->cap_cell_blocks = round8((cell_capacity + 255) / 256 + max_instances);
   b->cap_face_blocks = round8((std::max<int64_t>(face_capacity, 1) + 255) / 256 + max_instances);
+  const int ub = update_cells_of_block(b->shape.dim);
+  b->cap_upd_blocks = round8((cell_capacity + ub - 1) / ub + max_instances);
   b->cap_rec_blocks = round8((cell_capacity + b->L.groups_per_wave - 1) / b->L.groups_per_wave + max_instances);
   HIP_CHECK(hipStreamCreateWithFlags(&b->stream, hipStreamNonBlocking));
   HIP_CHECK(hipMalloc(&b->d_inst, sizeof(DevInst) * max_instances));
   HIP_CHECK(hipMalloc(&b->d_bcell, sizeof(BlockRef) * b->cap_cell_blocks));
-  HIP_CHECK(hipMalloc(&b->d_bface, sizeof(BlockRef) * b->cap_face_blocks));
+  HIP_CHECK(hipMalloc(&b->d_bupd, sizeof(BlockRef) * b->cap_upd_blocks));
   HIP_CHECK(hipMalloc(&b->d_brec, sizeof(BlockRef) * b->cap_rec_blocks));
   b->h_inst.assign(max_instances, DevInst{});
   b->members.assign(max_instances, nullptr);
@@ -1842,7 +1914,6 @@ int zfv_batch_add(zfv_batch *b, zfv_handle *h, double cfl, double t0, double t_e
   d.X = h->X;
   d.K = h->K;
   d.fpv = h->fpv;
-  d.G = h->G;
   d.src = h->src;
   d.cfl = cfl;
   d.t = t0;

@@ -1157,6 +1157,58 @@ void build_image(const zfv_mesh &mesh, const zfv_params &p, HostImage &img) {
   for (int k = 0; k < p.n_stencils; ++k) img.linear_weights[k] = p.linear_weights[k] / tot;
 }
 
+void build_update_tiles(const HostImage &img, int cells, bool flux_bc, std::vector<int32_t> &entries,
+                        std::vector<int32_t> &off, std::vector<int32_t> &more, std::vector<uint32_t> &cell_words) {
+  const int64_t n = img.n, tiles = (n + cells - 1) / cells;
+  const int nf = img.s.nfaces;
+  if (cells * nf > int(UPDATE_NO_FACE)) throw ZfvError(ZFV_ERR_INVALID, "update tile too large");
+  entries.resize(size_t(4) * 64 * tiles);
+  off.assign(tiles + 1, 0);
+  cell_words.assign(n, 0);
+  auto *first = reinterpret_cast<UpdateFace *>(entries.data());
+  // two passes over every tile: the first 64 entries and the count, then the rest
+  for (int pass = 0; pass < 2; ++pass) {
+    auto *rest = reinterpret_cast<UpdateFace *>(more.data());
+#pragma omp parallel for schedule(static)
+    for (int64_t t = 0; t < tiles; ++t) {
+      if (pass && off[t] == off[t + 1]) continue;
+      const int64_t i0 = t * cells, i1 = std::min(n, i0 + cells);
+      int32_t face[UPDATE_NO_FACE];
+      int count = 0;
+      auto put = [&](int32_t id, const UpdateFace &u) {
+        if (count >= 64 && pass) rest[off[t] + count - 64] = u;
+        if (count < 64 && !pass) first[64 * t + count] = u;
+        face[count++] = id;
+      };
+      for (int64_t i = i0; i < i1; ++i) {
+        uint32_t word = 0xFFFFFFFFu;
+        for (int f = 0; f < nf; ++f) {
+          const int32_t cf = img.cface[size_t(i) * 4 + f];
+          uint32_t at = UPDATE_NO_FACE;
+          if (!(cf & CFACE_EXTERIOR)) {
+            const int32_t e = cf >> 2;
+            int k = 0;
+            while (k < count && face[k] != e) ++k;
+            if (k == count) put(e, UpdateFace{img.fslot[size_t(e) * 2], img.fslot[size_t(e) * 2 + 1], e, 0});
+            at = uint32_t(k) | ((cf & CFACE_SIDE_R) ? 128u : 0u);
+          } else if (flux_bc && !(cf & CFACE_SIDE_R)) {
+            at = uint32_t(count);
+            put(-1, UpdateFace{0, -1, int32_t(i), f});
+          }
+          word = (word & ~(0xFFu << (8 * f))) | (at << (8 * f));
+        }
+        cell_words[i] = word;
+      }
+      if (pass) continue;
+      for (int k = count; k < 64; ++k) first[64 * t + k] = UpdateFace{-1, -1, 0, 0};
+      off[t + 1] = std::max(0, count - 64);
+    }
+    if (pass) break;
+    for (int64_t t = 0; t < tiles; ++t) off[t + 1] += off[t];
+    more.assign(size_t(4) * std::max(off[tiles], 1), 0);
+  }
+}
+
 void to_soa(const HostImage &img, const double *aos, double *soa) {
   const int64_t n = img.n;
   const int nv = img.s.nvars, dim = img.s.dim;

@@ -96,6 +96,14 @@ Shape shape_for(const zfv_params &p);
 // mean zero), which the light set's gravity volume term uses
 bool volume_mean_is_constant_term(const zfv_params &p, const Shape &s);
 
+// The faces of the update kernel's tiles of `cells` consecutive cells: per tile
+// its interior faces once each (both sides where both cells are in the tile)
+// and, with the constant flux BC, its boundary faces: 64 UpdateFace entries a
+// tile, tile t's further ones in more from off[t]; per cell a word naming its
+// faces' entries.
+void build_update_tiles(const HostImage &img, int cells, bool flux_bc, std::vector<int32_t> &entries,
+                        std::vector<int32_t> &off, std::vector<int32_t> &more, std::vector<uint32_t> &cell_words);
+
 // The caller's n x 5 row-major state (AllVariables::cvars) to and from the
 // product's nvars x n planes in product order (perm: product index -> caller
 // index), on the host's threads.  from_soa adds into aos when accumulate.

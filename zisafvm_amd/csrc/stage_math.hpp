@@ -57,12 +57,20 @@ struct Img {
   const int32_t *meta;
   const int32_t *cface;  // per cell its face words, 4 int32 (one 16-byte load; 2D's fourth unused)
   const int32_t *fslot;  // ne pairs: cell-face slots of each interior face's left and right cell
+  // the faces that an update wavefront evaluates for its tile of cells
+  // (build_update_tiles): tile t's first 64 at uent + 64 t (l < 0: none), any
+  // more in umore from uoff[t] to uoff[t + 1]; and per cell which of its tile's
+  // entries its faces are.  Null in the host emulation.
+  const int32_t *uent;
+  const int32_t *uoff;
+  const int32_t *umore;
+  const uint32_t *ucell;
   const uint32_t *fperm;
   const double *steady;  // as the state (ghost cells only are read)
   const double *phim;    // n pairs: cell mean of phi and of (phi - mean)^2 (one 16-byte load), or null
   const double *pot;     // potential tables of the cell's own points (pot_index), or null
   const double *frm;     // face frames of the cells' local faces (load_face_frame)
-  const double *ffr;     // per interior face its frame and area, t1, area (2D) or n, t1, area (3D), x ne
+  const double *ffr;     // per interior face its normal and area (face_table_frame)
   // 3D with an equilibrium: per cell its faces' outward normals times their
   // areas, n x (face 3 + d) (store_face_normals), or null
   const double *fan;
@@ -191,10 +199,6 @@ struct alignas(16) PPair {
 struct alignas(8) SlotPair {
   int32_t l, r;
 };
-
-// Face fluxes G: 2D per face its 4 values (two 16-byte pieces), 3D one
-// plane of ne values per variable (an odd count would need a pad word per
-// face; measured slower)
 
 // a cell's four face words (face id << 2 | exterior << 1 | side), one load
 struct alignas(16) FaceWords {
@@ -487,20 +491,18 @@ ZFV_HD int face_point_in_left_order(uint32_t fperm, int f, int q) {
   return q - t + pos;
 }
 
-// Face frame (src/zisa/math/face_factory.cpp:11-34): n, t1, t2 and the face
-// measure (edge length / Heron area).
+// Face normal (src/zisa/math/face_factory.cpp:11-34) and measure (edge length /
+// Heron area).  (The fluxes are formed in the global frame and need no
+// tangents.)
 template <int DIM>
-ZFV_HD void face_frame(const double (*w)[3], double *n, double *t1, double *t2, double &area) {
+ZFV_HD void face_frame(const double (*w)[3], double *n, double &area) {
   if (DIM == 2) {
     double dx = w[1][0] - w[0][0], dy = w[1][1] - w[0][1];
     double l = sqrt(dx * dx + dy * dy);
     area = l;
-    t1[0] = dx / l;
-    t1[1] = dy / l;
-    t1[2] = 0.0 / l;
-    n[0] = t1[1];
-    n[1] = -t1[0];
-    n[2] = t1[2];
+    n[0] = dy / l;
+    n[1] = -(dx / l);
+    n[2] = 0.0;
   } else {
     double a[3] = {w[1][0] - w[0][0], w[1][1] - w[0][1], w[1][2] - w[0][2]};
     double b[3] = {w[2][0] - w[0][0], w[2][1] - w[0][1], w[2][2] - w[0][2]};
@@ -509,33 +511,24 @@ ZFV_HD void face_frame(const double (*w)[3], double *n, double *t1, double *t2, 
     n[0] = c[0] / lc;
     n[1] = c[1] / lc;
     n[2] = c[2] / lc;
-    double la = sqrt(a[0] * a[0] + a[1] * a[1] + a[2] * a[2]);
-    t1[0] = a[0] / la;
-    t1[1] = a[1] / la;
-    t1[2] = a[2] / la;
     // Heron on the side lengths (src/zisa/math/triangle.cpp:11-18)
     double e0[3] = {w[1][0] - w[2][0], w[1][1] - w[2][1], w[1][2] - w[2][2]};
     double e1[3] = {w[0][0] - w[2][0], w[0][1] - w[2][1], w[0][2] - w[2][2]};
     double sa = sqrt(e0[0] * e0[0] + e0[1] * e0[1] + e0[2] * e0[2]);
     double sb = sqrt(e1[0] * e1[0] + e1[1] * e1[1] + e1[2] * e1[2]);
-    double sc = la;
+    double sc = sqrt(a[0] * a[0] + a[1] * a[1] + a[2] * a[2]);
     double s = 0.5 * (sa + sb + sc);
     area = sqrt(s * (s - sa) * (s - sb) * (s - sc));
   }
-  t2[0] = n[1] * t1[2] - n[2] * t1[1];
-  t2[1] = n[2] * t1[0] - n[0] * t1[2];
-  t2[2] = n[0] * t1[1] - n[1] * t1[0];
 }
 
-// Face frames are time independent: each cell's local faces keep theirs in a
-// table written once at setup (store_face_frames, with face_frame itself),
-// 3 (2D: t1, area) or 7 (3D: n, t1, area) doubles per face, and the interior
-// faces' frames (the left cell's view) are copied into a table in face order
-// for the face kernel (store_face_table); the flux BC of the cell update
-// reads a cell's own.  n (2D) and t2 follow from the stored values with
-// face_frame's own formulas, so every value equals face_frame's.
+// Face normals are time independent: each cell's local faces keep theirs and
+// the face measures in a table written once at setup (store_face_frames, with
+// face_frame itself), DIM + 1 doubles per face, and the interior faces' (the
+// left cell's view) are copied into a table in face order for the fluxes
+// (store_face_table); the flux BC reads a cell's own.
 template <int DIM>
-constexpr int frame_words() { return DIM == 2 ? 3 : 7; }
+constexpr int frame_words() { return DIM + 1; }
 // doubles of one cell-face slot of face-point values: Q x NV rounded up to
 // even, so that every slot starts on 16 bytes
 template <int DIM, int Q>
@@ -629,7 +622,7 @@ ZFV_HD double exp_near(double z) {
   return fma(r, z, 1.0);
 }
 
-// writes the frames of cell i's local faces (tab has frame_words (d+1) n entries)
+// writes the normals of cell i's local faces (tab has frame_words (d+1) n entries)
 template <int DIM>
 ZFV_HD void store_face_frames(const Img &m, int64_t i, double *tab) {
   constexpr int W = frame_words<DIM>();
@@ -637,50 +630,29 @@ ZFV_HD void store_face_frames(const Img &m, int64_t i, double *tab) {
   load_corners<DIM>(m, i, vtx);
   const uint32_t fperm = m.fperm[i];
   for (int f = 0; f < DIM + 1; ++f) {
-    double w3[3][3], n[3], t1[3], t2[3], area;
+    double w3[3][3], n[3], area;
     face_vertices<DIM>(fperm, f, vtx, w3);
-    face_frame<DIM>(w3, n, t1, t2, area);
+    face_frame<DIM>(w3, n, area);
     double *p = tab + int64_t(f * W) * m.n + i;
-    if (DIM == 2) {
-      p[0] = t1[0];
-      p[m.n] = t1[1];
-      p[2 * m.n] = area;
-    } else {
-      for (int d = 0; d < 3; ++d) p[int64_t(d) * m.n] = n[d];
-      for (int d = 0; d < 3; ++d) p[int64_t(3 + d) * m.n] = t1[d];
-      p[int64_t(6) * m.n] = area;
-    }
+    for (int d = 0; d < DIM; ++d) p[int64_t(d) * m.n] = n[d];
+    p[int64_t(DIM) * m.n] = area;
   }
 }
 
 template <int DIM>
-ZFV_HD void load_face_frame(const Img &m, int64_t i, int f, double *n, double *t1, double *t2, double &area) {
+ZFV_HD void load_face_frame(const Img &m, int64_t i, int f, double *n, double &area) {
   constexpr int W = frame_words<DIM>();
   const double *p = m.frm + int64_t(f * W) * m.n + i;
-  if (DIM == 2) {
-    t1[0] = p[0];
-    t1[1] = p[m.n];
-    t1[2] = 0.0;
-    area = p[2 * m.n];
-    n[0] = t1[1];
-    n[1] = -t1[0];
-    n[2] = t1[2];
-  } else {
-    for (int d = 0; d < 3; ++d) n[d] = p[int64_t(d) * m.n];
-    for (int d = 0; d < 3; ++d) t1[d] = p[int64_t(3 + d) * m.n];
-    area = p[int64_t(6) * m.n];
-  }
-  t2[0] = n[1] * t1[2] - n[2] * t1[1];
-  t2[1] = n[2] * t1[0] - n[0] * t1[2];
-  t2[2] = n[0] * t1[1] - n[1] * t1[0];
+  for (int d = 0; d < DIM; ++d) n[d] = p[int64_t(d) * m.n];
+  area = p[int64_t(DIM) * m.n];
 }
 
 // the outward normal of cell i's face f times its area (3D; the area and the
 // normal of its frame table entry, so that the well-balanced source's face
 // term and the fluxes see the same values)
 ZFV_HD void face_normal_out(const Img &m, int64_t i, int f, double *an) {
-  double n[3], t1[3], t2[3], area, c[4][3], xc[3] = {0.0, 0.0, 0.0};
-  load_face_frame<3>(m, i, f, n, t1, t2, area);
+  double n[3], area, c[4][3], xc[3] = {0.0, 0.0, 0.0};
+  load_face_frame<3>(m, i, f, n, area);
   load_corners<3>(m, i, c);
   // (the sign against the vector from the cell's mean corner to the face's)
   for (int k = 0; k < 4; ++k)
@@ -698,45 +670,23 @@ ZFV_HD void store_face_normals(const Img &m, int64_t i, double *tab) {
   for (int f = 0; f < 4; ++f) face_normal_out(m, i, f, tab + 12 * i + 3 * f);
 }
 
-// Per interior face its frame in face order (the face kernel reads it
-// coalesced): written once at setup from the left cell's frame table entry
+// Per interior face its normal and area in face order, each face's values
+// contiguous: written once at setup from the left cell's table entry
 template <int DIM>
 ZFV_HD void store_face_table(const Img &m, int64_t e, double *tab) {
   constexpr int NF = DIM + 1;
   const int64_t s = m.fslot[2 * e];
-  double n[3], t1[3], t2[3], area;
-  load_face_frame<DIM>(m, s / NF, int(s % NF), n, t1, t2, area);
-  if (DIM == 2) {
-    tab[e] = t1[0];
-    tab[m.ne + e] = t1[1];
-    tab[2 * m.ne + e] = area;
-  } else {
-    for (int d = 0; d < 3; ++d) tab[int64_t(d) * m.ne + e] = n[d];
-    for (int d = 0; d < 3; ++d) tab[int64_t(3 + d) * m.ne + e] = t1[d];
-    tab[int64_t(6) * m.ne + e] = area;
-  }
+  double n[3], area;
+  load_face_frame<DIM>(m, s / NF, int(s % NF), n, area);
+  for (int d = 0; d < DIM; ++d) tab[e * (DIM + 1) + d] = n[d];
+  tab[e * (DIM + 1) + DIM] = area;
 }
 
-// the frame of interior face e from the face table (the same values, and the
-// same derived n (2D) and t2, as load_face_frame)
 template <int DIM>
-ZFV_HD void face_table_frame(const Img &m, int64_t e, double *n, double *t1, double *t2, double &area) {
-  if (DIM == 2) {
-    t1[0] = m.ffr[e];
-    t1[1] = m.ffr[m.ne + e];
-    t1[2] = 0.0;
-    area = m.ffr[2 * m.ne + e];
-    n[0] = t1[1];
-    n[1] = -t1[0];
-    n[2] = t1[2];
-  } else {
-    for (int d = 0; d < 3; ++d) n[d] = m.ffr[int64_t(d) * m.ne + e];
-    for (int d = 0; d < 3; ++d) t1[d] = m.ffr[int64_t(3 + d) * m.ne + e];
-    area = m.ffr[int64_t(6) * m.ne + e];
-  }
-  t2[0] = n[1] * t1[2] - n[2] * t1[1];
-  t2[1] = n[2] * t1[0] - n[0] * t1[2];
-  t2[2] = n[0] * t1[1] - n[1] * t1[0];
+ZFV_HD void face_table_frame(const Img &m, int64_t e, double *n, double &area) {
+  const double *p = m.ffr + e * (DIM + 1);
+  for (int d = 0; d < DIM; ++d) n[d] = p[d];
+  area = p[DIM];
 }
 
 // quadrature point q of a face given its vertices in left-cell order
@@ -972,74 +922,91 @@ ZFV_HD void store_source_moments(const Img &m, int64_t i, double *tab) {
 }
 
 // ---- ideal gas / fluxes -------------------------------------------------------
-// Rotated 2D states carry 4 variables (rho, m_n, m_t, E): the t2 component of
-// a 2D state is identically zero and stays zero through HLLC.
-template <int NV>
-ZFV_HD double pressure_of(const double *u, double gamma) {
+// States (rho, momentum (DIM), E) in the global frame; n: the face's unit
+// normal.  A flux in direction n needs the momentum's normal part and its
+// length only, so no state is turned into a face frame and no flux back.
+
+// What both fluxes need of a state: one division by the density serves the
+// velocity, the pressure and the sound speed.  (The fluxes were bound by
+// arithmetic, and a double precision division is some 14 instructions: 20 a
+// point before, 5 now.)
+template <int DIM>
+struct FaceState {
+  double r, mn, vn, p, a;  // 1/rho, momentum and velocity along n, pressure, sound speed
+};
+template <int DIM>
+ZFV_HD FaceState<DIM> face_state(const double *u, const double *n, double gamma) {
+  FaceState<DIM> s;
+  s.r = 1.0 / u[0];
+  s.mn = u[1] * n[0] + u[2] * n[1];
   double m2 = u[1] * u[1] + u[2] * u[2];
-  if (NV == 5) m2 += u[3] * u[3];
-  double kin = 0.5 * m2 / u[0];
-  return (u[NV - 1] - kin) * (gamma - 1.0);
-}
-
-template <int NV>
-ZFV_HD void euler_flux(const double *u, double p, double *f) {
-  double v = u[1] / u[0];
-  f[0] = u[1];
-  f[1] = v * u[1] + p;
-  f[2] = v * u[2];
-  if (NV == 5) f[3] = v * u[3];
-  f[NV - 1] = v * (u[NV - 1] + p);
-}
-
-template <int NV>
-ZFV_HD void hllc(const double *uL, const double *uR, double gamma, double *nf) {
-  double pL = pressure_of<NV>(uL, gamma), aL = sqrt(gamma * pL / uL[0]);
-  double pR = pressure_of<NV>(uR, gamma), aR = sqrt(gamma * pR / uR[0]);
-  double roe_ratio = sqrt(uR[0] / uL[0]);
-  double inv1 = 1.0 + roe_ratio;
-  double vL = uL[1] / uL[0];
-  double vR = uR[1] / uR[0];
-  double v_tilda = (vL + vR * roe_ratio) / inv1;
-  double HL = (uL[NV - 1] + pL) / uL[0];
-  double HR = (uR[NV - 1] + pR) / uR[0];
-  double H_tilda = (HL + HR * roe_ratio) / inv1;
-  double r1 = (uL[1] / uL[0] + (uR[1] / uR[0]) * roe_ratio) / inv1;
-  double r2 = (uL[2] / uL[0] + (uR[2] / uR[0]) * roe_ratio) / inv1;
-  double vroe = r1 * r1 + r2 * r2;
-  if (NV == 5) {
-    double r3 = (uL[3] / uL[0] + (uR[3] / uR[0]) * roe_ratio) / inv1;
-    vroe += r3 * r3;
+  if (DIM == 3) {
+    s.mn += u[3] * n[2];
+    m2 += u[3] * u[3];
   }
-  double a_tilda = sqrt((gamma - 1.0) * (H_tilda - 0.5 * vroe));
-  double sL = dmin(vL - aL, v_tilda - a_tilda);
-  double sR = dmax(vR + aR, v_tilda + a_tilda);
-  double s_star = (uR[1] * (sR - vR) - uL[1] * (sL - vL) + pL - pR) / (uR[0] * (sR - vR) - uL[0] * (sL - vL));
+  s.vn = s.mn * s.r;
+  s.p = (u[DIM + 1] - 0.5 * (m2 * s.r)) * (gamma - 1.0);
+  s.a = sqrt(gamma * s.p * s.r);
+  return s;
+}
+
+// the physical flux in direction n
+template <int DIM>
+ZFV_HD void euler_flux(const double *u, const FaceState<DIM> &s, const double *n, double *f) {
+  f[0] = s.mn;
+  for (int d = 0; d < DIM; ++d) f[1 + d] = s.vn * u[1 + d] + s.p * n[d];
+  f[DIM + 1] = s.vn * (u[DIM + 1] + s.p);
+}
+
+template <int DIM>
+ZFV_HD void hllc(const double *uL, const double *uR, const double *n, double gamma, double *nf) {
+  constexpr int NV = DIM + 2;
+  const FaceState<DIM> L = face_state<DIM>(uL, n, gamma), R = face_state<DIM>(uR, n, gamma);
+  const double roe_ratio = sqrt(uR[0] * L.r);
+  const double inv1 = 1.0 / (1.0 + roe_ratio);
+  auto mean = [&](double x, double y) { return (x + y * roe_ratio) * inv1; };
+  const double H = mean((uL[NV - 1] + L.p) * L.r, (uR[NV - 1] + R.p) * R.r);
+  const double v = mean(L.vn, R.vn);
+  double vroe = 0.0;
+  for (int d = 0; d < DIM; ++d) {
+    const double w = mean(uL[1 + d] * L.r, uR[1 + d] * R.r);
+    vroe = d == 0 ? w * w : vroe + w * w;
+  }
+  const double a = sqrt((gamma - 1.0) * (H - 0.5 * vroe));
+  const double sL = dmin(L.vn - L.a, v - a);
+  const double sR = dmax(R.vn + R.a, v + a);
+  const double s_star = (R.mn * (sR - R.vn) - L.mn * (sL - L.vn) + L.p - R.p) /
+                        (uR[0] * (sR - R.vn) - uL[0] * (sL - L.vn));
   const bool left = 0.0 <= s_star;
-  const double *uK = left ? uL : uR;
-  double pK = left ? pL : pR;
-  euler_flux<NV>(uK, pK, nf);
+  FaceState<DIM> K;
+  K.mn = left ? L.mn : R.mn;
+  K.vn = left ? L.vn : R.vn;
+  K.p = left ? L.p : R.p;
+  double uK[NV];
+  for (int k = 0; k < NV; ++k) uK[k] = left ? uL[k] : uR[k];
+  euler_flux<DIM>(uK, K, n, nf);
   if (sL < 0.0 && 0.0 <= sR) {
-    double sK = left ? sL : sR;
-    double vK = left ? vL : vR;
-    double cK = (sK - vK) / (sK - s_star);
+    // the star state: cK = (sK - vK) / (sK - s_star) times (rho, m + rho
+    // (s_star - vK) n, E + (s_star - vK) (rho s_star + pK / (sK - vK)))
+    const double sK = left ? sL : sR;
+    const double iK = 1.0 / (sK - s_star);
+    const double cK = (sK - K.vn) * iK, dv = s_star - K.vn;
     nf[0] += sK * (cK * uK[0] - uK[0]);
-    nf[1] += sK * (cK * uK[0] * s_star - uK[1]);
-    nf[2] += sK * (cK * uK[2] - uK[2]);
-    if (NV == 5) nf[3] += sK * (cK * uK[3] - uK[3]);
-    nf[NV - 1] += sK * (cK * (uK[NV - 1] + (s_star - vK) * (uK[0] * s_star + pK / (sK - vK))) - uK[NV - 1]);
+    const double dm = cK * (uK[0] * dv);
+    for (int d = 0; d < DIM; ++d) nf[1 + d] += sK * (cK * uK[1 + d] + dm * n[d] - uK[1 + d]);
+    nf[NV - 1] += sK * (cK * (uK[NV - 1] + dv * (uK[0] * s_star)) + dv * K.p * iK - uK[NV - 1]);
   }
 }
 
-template <int NV>
-ZFV_HD void rusanov(const double *uL, const double *uR, double gamma, double *f) {
-  double pL = pressure_of<NV>(uL, gamma), aL = sqrt(gamma * pL / uL[0]);
-  double pR = pressure_of<NV>(uR, gamma), aR = sqrt(gamma * pR / uR[0]);
+template <int DIM>
+ZFV_HD void rusanov(const double *uL, const double *uR, const double *n, double gamma, double *f) {
+  constexpr int NV = DIM + 2;
+  const FaceState<DIM> L = face_state<DIM>(uL, n, gamma), R = face_state<DIM>(uR, n, gamma);
+  const double s = dmax(fabs(L.vn) + L.a, fabs(R.vn) + R.a);
   double fL[NV], fR[NV];
-  euler_flux<NV>(uL, pL, fL);
-  euler_flux<NV>(uR, pR, fR);
-  double s = dmax(fabs(uL[1] / uL[0]) + aL, fabs(uR[1] / uR[0]) + aR);
-  for (int v = 0; v < NV; ++v) f[v] = 0.5 * (fL[v] + fR[v]) - 0.5 * s * (uR[v] - uL[v]);
+  euler_flux<DIM>(uL, L, n, fL);
+  euler_flux<DIM>(uR, R, n, fR);
+  for (int k = 0; k < NV; ++k) f[k] = 0.5 * (fL[k] + fR[k]) - 0.5 * s * (uR[k] - uL[k]);
 }
 
 // ---- the per-cell reconstruction, one lane per conserved variable --------------
@@ -1816,7 +1783,7 @@ ZFV_HD void reconstruct_lane(const Img &m, int64_t i, const int g, X &xch, const
 
   // The face points along the cell's own vertex order, so that every corner
   // index is known at compile time; a point's values go to the place of the
-  // same point in the left cell's order, which the face kernel reads.
+  // same point in the left cell's order, in which the fluxes read them.
   const FaceWords cfw = load_face_words(m, i);
   double V[DIM + 1][3];
   load_corners<DIM>(m, i, V);
@@ -1920,8 +1887,7 @@ ZFV_HD void reconstruct_lane(const Img &m, int64_t i, const int g, X &xch, const
       }
     }
     computed_here<Q>(u);
-    // in the global frame: the face kernel rotates the momentum into the
-    // face frame, with every component in one thread
+    // in the global frame, as the fluxes take them
     if (!exterior) {
       double *slot = fpv + (int64_t(i) * NF + f) * slot_doubles<DIM, Q>() + g;
 #pragma unroll
@@ -2003,80 +1969,86 @@ ZFV_HD void reconstruct_lane(const Img &m, int64_t i, const int g, X &xch, const
 }
 
 // ---- the per-face flux ----------------------------------------------------------
-// G[v][e] = sum_q w_q F(uL_q, uR_q) in the face frame, w_q the normalized
-// face weights (the face measure is applied by the cell update).
-// a flux g given in the face frame (normal, t1, t2 components of the
-// momentum) in the global frame
-template <int DIM>
-ZFV_HD void world_flux(const double *g, const double *nn, const double *t1, const double *t2, double *wv) {
+// the flux through interior face e from its left to its right cell (global
+// frame, times the face's measure), which the left cell loses and the right
+// cell gains, from the two cells' point values (slot layout)
+template <int DIM, int Q>
+ZFV_HD void flux_between(const Img &m, int64_t e, const double *bL, const double *bR, double *flux) {
   constexpr int NV = DIM + 2;
-  wv[0] = g[0];
-  wv[NV - 1] = g[NV - 1];
-  if (DIM == 2) {
-    wv[1] = g[1] * nn[0] + g[2] * t1[0];
-    wv[2] = g[1] * nn[1] + g[2] * t1[1];
-  } else {
-    wv[1] = g[1] * nn[0] + g[2] * t1[0] + g[3] * t2[0];
-    wv[2] = g[1] * nn[1] + g[2] * t1[1] + g[3] * t2[1];
-    wv[3] = g[1] * nn[2] + g[2] * t1[2] + g[3] * t2[2];
+  double nn[3], area;
+  face_table_frame<DIM>(m, e, nn, area);
+  for (int v = 0; v < NV; ++v) flux[v] = 0.0;
+#pragma unroll
+  for (int q = 0; q < Q; ++q) {
+    double f[NV];
+    if (m.flux == 0) hllc<DIM>(bL + q * NV, bR + q * NV, nn, m.gamma, f);
+    else rusanov<DIM>(bL + q * NV, bR + q * NV, nn, m.gamma, f);
+    for (int v = 0; v < NV; ++v) flux[v] = flux[v] + m.fw[q] * f[v];
+  }
+  for (int v = 0; v < NV; ++v) flux[v] = area * flux[v];
+}
+
+// the point values of one cell-face slot, in 16-byte loads
+template <int DIM, int Q>
+ZFV_HD void load_slot(const double *__restrict__ fpv, int64_t slot, double *b) {
+  constexpr int SQ = slot_doubles<DIM, Q>();
+  const PPair *p = reinterpret_cast<const PPair *>(fpv + slot * SQ);
+#pragma unroll
+  for (int k = 0; k < SQ / 2; ++k) {
+    const PPair v = p[k];
+    b[2 * k] = v.lo;
+    b[2 * k + 1] = v.hi;
   }
 }
 
+// every interior face's flux stored once per face (the host emulation's form;
+// the kernels form a cell's fluxes where the cell is updated)
 template <int DIM, int Q>
 ZFV_HD void face_flux(const Img &m, int64_t e, const double *__restrict__ fpv, double *__restrict__ G) {
   constexpr int NV = DIM + 2;
-  constexpr int NF = DIM + 1;
-  const int64_t ne = m.ne;
-  // the two cells' point values of this face (Q x NV doubles at the start of
-  // each slot, momentum in the global frame), in 16-byte loads
   constexpr int SQ = slot_doubles<DIM, Q>();
-  double bL[SQ], bR[SQ];
+  double bL[SQ], bR[SQ], flux[NV];
   const SlotPair sl = reinterpret_cast<const SlotPair *>(m.fslot)[e];
-  const PPair *pL = reinterpret_cast<const PPair *>(fpv + int64_t(sl.l) * SQ);
-  const PPair *pR = reinterpret_cast<const PPair *>(fpv + int64_t(sl.r) * SQ);
-#pragma unroll
-  for (int k = 0; k < SQ / 2; ++k) {
-    const PPair l = pL[k], r = pR[k];
-    bL[2 * k] = l.lo;
-    bL[2 * k + 1] = l.hi;
-    bR[2 * k] = r.lo;
-    bR[2 * k + 1] = r.hi;
+  load_slot<DIM, Q>(fpv, sl.l, bL);
+  load_slot<DIM, Q>(fpv, sl.r, bR);
+  flux_between<DIM, Q>(m, e, bL, bR, flux);
+  for (int v = 0; v < NV; ++v) G[v * m.ne + e] = flux[v];
+}
+
+// One face of an update tile: an interior face e with the slots of its left and
+// right cell, or (r < 0) the boundary face f of cell e
+struct alignas(16) UpdateFace {
+  int32_t l, r, e, f;
+};
+// a cell's word: 8 bits per face, the entry's place in the tile (7 bits; 127:
+// no contribution) and whether the cell is on the face's right side
+constexpr uint32_t UPDATE_NO_FACE = 127u;
+
+// FluxBC at a boundary face f of cell i: the physical flux of the cell average
+// out of the cell (global frame, times the face measure; the weights sum to one)
+template <int DIM, bool AOS>
+ZFV_HD void boundary_flux(const Img &m, int64_t i, int f, const double *__restrict__ U, double *flux) {
+  constexpr int NV = DIM + 2;
+  double nn[3], area, u[NV];
+  load_face_frame<DIM>(m, i, f, nn, area);
+  for (int v = 0; v < NV; ++v) u[v] = U[state_at<AOS, NV>(m.n, v, i)];
+  euler_flux<DIM>(u, face_state<DIM>(u, nn, m.gamma), nn, flux);
+  for (int v = 0; v < NV; ++v) flux[v] = area * flux[v];
+}
+
+// the flux of one face of an update tile
+template <int DIM, int Q>
+ZFV_HD void update_face_flux(const Img &m, const UpdateFace &u, const double *__restrict__ U,
+                             const double *__restrict__ fpv, double *flux) {
+  constexpr int SQ = slot_doubles<DIM, Q>();
+  if (u.r < 0) {
+    boundary_flux<DIM, true>(m, u.e, u.f, U, flux);
+    return;
   }
-  // the face frame (the left cell's vertex order, as both cells see it)
-  double nn[3], t1[3], t2[3], area;
-  face_table_frame<DIM>(m, e, nn, t1, t2, area);
-  auto rotate = [&](double *u) {
-    const double mc[3] = {u[1], u[2], DIM == 3 ? u[3] : 0.0};
-    u[1] = DIM == 2 ? mc[0] * nn[0] + mc[1] * nn[1] : mc[0] * nn[0] + mc[1] * nn[1] + mc[2] * nn[2];
-    u[2] = DIM == 2 ? mc[0] * t1[0] + mc[1] * t1[1] : mc[0] * t1[0] + mc[1] * t1[1] + mc[2] * t1[2];
-    if (DIM == 3) u[3] = mc[0] * t2[0] + mc[1] * t2[1] + mc[2] * t2[2];
-  };
-  double acc[NV];
-  for (int v = 0; v < NV; ++v) acc[v] = 0.0;
-#pragma unroll
-  for (int q = 0; q < Q; ++q) {
-    double uL[NV], uR[NV], f[NV];
-    for (int v = 0; v < NV; ++v) {
-      uL[v] = bL[q * NV + v];
-      uR[v] = bR[q * NV + v];
-    }
-    rotate(uL);
-    rotate(uR);
-    if (m.flux == 0) hllc<NV>(uL, uR, m.gamma, f);
-    else rusanov<NV>(uL, uR, m.gamma, f);
-    for (int v = 0; v < NV; ++v) acc[v] = acc[v] + m.fw[q] * f[v];
-  }
-  // back to the global frame, times the face's measure: the flux through the
-  // face, which the left cell loses and the right cell gains (cell_rate)
-  double wv[NV];
-  world_flux<DIM>(acc, nn, t1, t2, wv);
-  if (DIM == 2) {
-    PPair *gp = reinterpret_cast<PPair *>(G + e * NV);
-    gp[0] = PPair{area * wv[0], area * wv[1]};
-    gp[1] = PPair{area * wv[2], area * wv[NV - 1]};
-  } else {
-    for (int v = 0; v < NV; ++v) G[v * ne + e] = area * wv[v];
-  }
+  double bL[SQ], bR[SQ];
+  load_slot<DIM, Q>(fpv, u.l, bL);
+  load_slot<DIM, Q>(fpv, u.r, bR);
+  flux_between<DIM, Q>(m, u.e, bL, bR, flux);
 }
 
 // ---- the per-cell rate of change -------------------------------------------------
@@ -2097,44 +2069,16 @@ ZFV_HD void cell_rate(const Img &m, int64_t i, const double *__restrict__ U, con
     // ghost-pair faces (cf == 3) carry neither a flux nor the flux BC; the
     // equilibrium flux BC (flux_bc 2) is part of the source term
     if (exterior && (m.flux_bc != 1 || (cf & 1))) continue;
+    double g[NV];
     if (!exterior) {
-      // the face kernel's flux through the face (global frame, times area)
-      const int64_t e = cf >> 2;
+      // the flux through the face (global frame, times area)
       const double sgn = (cf & 1) ? 1.0 : -1.0;
-      double g[NV];
-      if (DIM == 2) {
-        const PPair *gp = reinterpret_cast<const PPair *>(G + e * NV);
-        const PPair g0 = gp[0], g1 = gp[1];
-        g[0] = g0.lo;
-        g[1] = g0.hi;
-        g[2] = g1.lo;
-        g[NV - 1] = g1.hi;
-      } else {
-        for (int v = 0; v < NV; ++v) g[v] = G[v * m.ne + e];
-      }
-      for (int v = 0; v < NV; ++v) acc[v] += sgn * g[v];
-      continue;
-    }
-    // FluxBC: physical flux of the cell average in the face frame
-    double nn[3], t1[3], t2[3], area;
-    load_face_frame<DIM>(m, i, f, nn, t1, t2, area);
-    double g[NV], u[NV], r[NV];
-    for (int v = 0; v < NV; ++v) u[v] = U[state_at<AOS, NV>(n, v, i)];
-    r[0] = u[0];
-    r[NV - 1] = u[NV - 1];
-    if (DIM == 2) {
-      r[1] = u[1] * nn[0] + u[2] * nn[1];
-      r[2] = u[1] * t1[0] + u[2] * t1[1];
+      for (int v = 0; v < NV; ++v) g[v] = sgn * G[v * m.ne + (cf >> 2)];
     } else {
-      r[1] = u[1] * nn[0] + u[2] * nn[1] + u[3] * nn[2];
-      r[2] = u[1] * t1[0] + u[2] * t1[1] + u[3] * t1[2];
-      r[3] = u[1] * t2[0] + u[2] * t2[1] + u[3] * t2[2];
+      boundary_flux<DIM, AOS>(m, i, f, U, g);
+      for (int v = 0; v < NV; ++v) g[v] = -1.0 * g[v];
     }
-    euler_flux<NV>(r, pressure_of<NV>(r, m.gamma), g);
-    // the flux BC uses the face measure directly (weights sum to one)
-    double wv[NV];
-    world_flux<DIM>(g, nn, t1, t2, wv);
-    for (int v = 0; v < NV; ++v) acc[v] += -1.0 * (area * wv[v]);
+    for (int v = 0; v < NV; ++v) acc[v] += g[v];
   }
   const double vol = m.vol[i];
   for (int v = 0; v < NV; ++v) L[v] = acc[v] / vol;
