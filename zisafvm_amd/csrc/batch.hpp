@@ -25,7 +25,7 @@ struct DevInst {
   int active;
   int steps_done;
   int max_steps;
-  int pad;
+  int running;  // the step under way advances this member (set by its first stage)
 };
 
 struct BlockRef {
@@ -33,9 +33,13 @@ struct BlockRef {
   int local;  // block index inside the instance
 };
 
-// the step's dt of a member: cfl times its CFL minimum (the bits of a
+// a member that has reached its end time or step limit
+ZFV_HD bool kb_finished(const DevInst &d) { return d.t >= d.t_end || d.steps_done >= d.max_steps; }
+
+// the step's dt of a member (0 or less: none): cfl times its CFL minimum (the bits of a
 // positive double in dt_bits), clamped to its end time
 ZFV_HD double kb_step_dt(const DevInst &d) {
+  if (kb_finished(d)) return 0.0;
   double m;
   const unsigned long long bits = d.dt_bits;
   memcpy(&m, &bits, sizeof(m));
@@ -43,6 +47,13 @@ ZFV_HD double kb_step_dt(const DevInst &d) {
   const double rest = d.t_end - d.t;
   if (dt > rest) dt = rest;
   return dt;
+}
+
+// the first stage's record of the step's dt
+ZFV_HD void kb_begin_instance(DevInst &d, double dt) {
+  d.running = dt > 0.0;
+  if (d.running) d.dt = dt;
+  else d.active = 0;
 }
 
 // groups of NV lanes per 64-wide wavefront (2D: 16 cells, 3D: 12 cells)
@@ -88,7 +99,7 @@ ZFV_HD void kb_reconstruct_group(const DevInst *insts, BlockRef b, int waves, in
   if (b.inst < 0) return;
   const DevInst &d = insts[b.inst];
   if (!d.active) return;
-  if (stage == 0 && !(kb_step_dt(d) > 0.0)) return;  // stops this step (kb_update_thread)
+  if (stage == 0 ? !(kb_step_dt(d) > 0.0) : !d.running) return;  // no step (kb_begin_instance)
   const int64_t i = (int64_t(b.local) * waves + wave) * GPW + grp;
   if (grp >= GPW || i >= d.m.n) return;
   if (d.m.steady != nullptr && (d.m.meta[i] & META_FAR_GHOST) == META_FAR_GHOST) return;
@@ -122,11 +133,10 @@ ZFV_HD void kb_update_thread(DevInst *insts, BlockRef b, int t, int stage) {
     // the later stages and the step's end (and stops a member that cannot
     // advance, whose threads all leave here)
     dt = kb_step_dt(d);
-    if (b.local == 0 && t == 0) {
-      d.dt = dt;
-      if (!(dt > 0.0)) d.active = 0;
-    }
+    if (b.local == 0 && t == 0) kb_begin_instance(d, dt);
     if (!(dt > 0.0)) return;
+  } else if (!d.running) {
+    return;
   }
   const int64_t i = int64_t(b.local) * 256 + t;
   const Img &m = d.m;
@@ -183,21 +193,14 @@ ZFV_HD double kb_cfl_thread(const DevInst &d, BlockRef b, int t) {
     const int64_t n = m.n;
     double u[NV];
     for (int v = 0; v < NV; ++v) u[v] = d.U[state_at<AOS, NV>(n, v, i)];
-    double m2 = u[1] * u[1] + u[2] * u[2];
-    if (DIM == 3) m2 += u[3] * u[3];
-    double v2 = m2 / (u[0] * u[0]);
-    double p = (u[NV - 1] - 0.5 * m2 / u[0]) * (m.gamma - 1.0);
-    double a = sqrt(m.gamma * p / u[0]);
-    r = m.inr[i] / (sqrt(v2) + a);
-    if (!(r > 0.0)) r = 0.0;
+    r = cfl_of_cell<DIM>(u, m.inr[i], m.gamma);
   }
   return r;
 }
 
-// per-instance step bookkeeping: the CFL minimum of a step starts at 1e300
-// (set when the member joins and at the end of every step); the step's dt is
-// cfl times the minimum, clamped to t_end (an instance that cannot advance
-// stops: kb_update_thread of stage 0); the end of a step advances the time
+// per-instance step bookkeeping: the CFL minimum of a step starts at 1e300;
+// the step's dt is cfl times the minimum, clamped to t_end (an instance that
+// cannot advance stops: kb_begin_instance); the end of a step advances the time
 ZFV_HD unsigned long long kb_no_bound() {
   const double big = 1.0e300;
   unsigned long long bits;
@@ -206,10 +209,9 @@ ZFV_HD unsigned long long kb_no_bound() {
 }
 
 ZFV_HD void kb_end_instance(DevInst &d) {
-  if (!d.active) return;
+  if (!d.active || !d.running) return;
   d.t += d.dt;
   d.steps_done += 1;
-  if (d.t >= d.t_end || d.steps_done >= d.max_steps) d.active = 0;
   d.dt_bits = kb_no_bound();
 }
 

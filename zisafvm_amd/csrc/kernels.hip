@@ -144,11 +144,88 @@ struct StageCoeffs {
   int write_rate_only;  // 1: store L in K[stage] and stop (zfv_rate)
 };
 
+// A single instance's time loop on the device (zfv_advance): TimeLoop's
+// step with LocalCFL (src/zisa/fvm_loops/time_loop.cpp:36-81,
+// include/zisa/model/local_cfl_condition_impl.hpp:25-40), dt clamped to the
+// end time as the simulation clock does (its library is not vendored in the
+// reference), with no host round trip per step.
+struct AdvState {
+  double t, t_end, cfl, dt;
+  int steps, max_steps, active;
+  unsigned blocks_done;  // of k_adv_commit
+  // RejectLargeDensityChange (src/zisa/ode/step_rejection.cpp:17-57; off
+  // when drho_crit <= 0): factor scales the CFL step, halves on a rejected
+  // step (which is retried with factor * its dt, TimeLoop::reject_step,
+  // src/zisa/fvm_loops/time_loop.cpp:182-196) and doubles after two good
+  // steps in a row, within [min_factor, 1]
+  double drho_crit, factor, min_factor, retry_dt;
+  int bad, prev_good, retry, rejections;
+};
+
+// The step's CFL minimum is reduced into kAdvSlots words of 128 bytes (one word
+// would serialise thousands of atomics): the last stage's update leaves the new
+// state's minimum there, the next step's first update picks dt from it, and the
+// second stage's update sets the words back.
+constexpr int kAdvSlots = 64, kAdvSlotStride = 16;
+constexpr size_t kAdvSlotBytes = size_t(kAdvSlots) * kAdvSlotStride * sizeof(unsigned long long);
+
+// start value of the CFL reduction (bits of 1e300)
+__host__ __device__ inline unsigned long long adv_no_bound() {
+  const double big = 1.0e300;
+  unsigned long long bits;
+  memcpy(&bits, &big, sizeof(bits));
+  return bits;
+}
+
+// StepRejection::pick_time_step: factor * the CFL step, or the retry step;
+// zero when finished, when the CFL gives no positive step (a non-physical
+// state) or when the step no longer advances the time
+__device__ __forceinline__ double adv_pick(const AdvState &a, double cfl_min) {
+  double dt = a.retry ? a.retry_dt : a.factor * (a.cfl * cfl_min);
+  const double rest = a.t_end - a.t;
+  if (dt > rest) dt = rest;
+  if (!a.active || !(dt > 0.0) || a.t + dt == a.t) dt = 0.0;  // the stages leave U as it is (U + 0 * dudt)
+  return dt;
+}
+
+// the end of a step: the time advances, or the step is to be retried
+__device__ __forceinline__ void adv_end(AdvState *a) {
+  if (!a->active) return;
+  const int bad = a->bad;
+  a->bad = 0;
+  a->retry = 0;
+  if (a->drho_crit > 0.0) {
+    const double f = a->factor;
+    if (bad) {
+      a->prev_good = 0;
+      a->factor = fmax(a->min_factor, fmin(f / 2.0, 1.0));
+      a->retry = 1;
+      a->retry_dt = a->factor * a->dt;
+      a->rejections += 1;
+      return;  // the time does not advance; the state was kept
+    }
+    a->factor = fmax(a->min_factor, fmin(a->prev_good ? f * 2.0 : f, 1.0));
+    a->prev_good = 1;
+  }
+  a->t += a->dt;
+  a->steps += 1;
+  if (a->t >= a->t_end || a->steps >= a->max_steps) a->active = 0;
+}
+
 // What a stage's update reads and writes: K[stage] = L(Ustage); Unext = U0 +
 // dt * sum_j c_j K[j] (src/zisa/ode/runge_kutta.cpp:122-143), then FrozenBC for
 // ghost cells.  Ustage, U0 and Unext may name the same buffer (stages 1 and 2
 // read and write the stage state X; a wavefront reads only its own cells'
 // entries, before it writes them), so none of them is declared __restrict__.
+// What the last stage's update also does in a time loop that chooses its steps:
+// the new state's CFL minimum goes to cfl[slot] (null: not wanted), a density
+// change of more than crit times its old value in any cell sets *bad (crit 0:
+// not asked)
+struct UpdateChecks {
+  unsigned long long *cfl;
+  double crit;
+  int *bad;
+};
 struct UpdateArgs {
   StageCoeffs sc;
   int stage;
@@ -175,7 +252,8 @@ constexpr int update_cells_of_block(int dim) { return 4 * update_cells_of_wave(d
 // 1,152 triangles 9.4 -> 4.8.  (One lane per cell face, every face evaluated
 // twice: 48, 50 and 5.0 us; four wavefronts per SIMD spill in 3D: 54 us.)
 template <int DIM, int Q>
-__device__ __forceinline__ void update_cells(const Img &m, const UpdateArgs &a, double dt, int64_t tile, int lane, double *lds) {
+__device__ __forceinline__ void update_cells(const Img &m, const UpdateArgs &a, double dt, const UpdateChecks &chk, int64_t tile,
+                                             int lane, double *lds) {
   constexpr int NV = DIM + 2;
   constexpr int NF = DIM + 1;
   constexpr int CW = update_cells_of_wave(DIM);
@@ -188,13 +266,13 @@ __device__ __forceinline__ void update_cells(const Img &m, const UpdateArgs &a, 
   // flight with the faces' entries and point values
   double part[NP], base[NP], src[NP], vol[NP];
   uint32_t word[NP];
-  bool store[NP];
+  bool inside[NP], frozen_cell[NP];
 #pragma unroll
   for (int p = 0; p < NP; ++p) {
     const int e = p * 64 + lane, c = e / NV;
     int64_t i = i0 + c;
-    store[p] = e < CW * NV && i < n;
-    i = store[p] ? i : i0;
+    inside[p] = e < CW * NV && i < n;
+    i = inside[p] ? i : i0;
     const int64_t at = i * NV + (e - c * NV);
     const int32_t meta = m.meta[i];
     word[p] = m.ucell[i];
@@ -206,12 +284,10 @@ __device__ __forceinline__ void update_cells(const Img &m, const UpdateArgs &a, 
 #pragma unroll
       for (int j = 0; j < 2; ++j)
         if (j < a.stage && a.sc.c[j] != 0.0) part[p] += a.sc.c[j] * a.K[int64_t(j) * NV * n + at];
-      // frozen ghost cells keep the steady state whatever their fluxes
-      if ((meta & 16) != 0 && m.steady != nullptr) {
-        a.Unext[at] = m.steady[at];
-        store[p] = false;
-      }
     }
+    // frozen ghost cells keep the steady state whatever their fluxes
+    frozen_cell[p] = !a.sc.write_rate_only && (meta & 16) != 0 && m.steady != nullptr;
+    if (frozen_cell[p]) base[p] = m.steady[at];
   }
   UpdateFace face = mine;
   for (int k = lane; face.l >= 0;) {
@@ -228,9 +304,18 @@ __device__ __forceinline__ void update_cells(const Img &m, const UpdateArgs &a, 
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 #pragma unroll
   for (int p = 0; p < NP; ++p) {
-    if (!store[p]) continue;
+    if (!inside[p]) continue;
     const int e = p * 64 + lane, v = e % NV;
     const int64_t at = i0 * NV + e;
+    // RejectLargeDensityChange::check: |rho1 - rho0| > crit rho0
+    auto check = [&](double r0, double r1) {
+      if (chk.crit > 0.0 && v == 0 && fabs(r0 - r1) > chk.crit * r0) atomicOr(chk.bad, 1);
+    };
+    if (frozen_cell[p]) {
+      if (chk.crit > 0.0) check(a.U0[at], base[p]);
+      a.Unext[at] = base[p];
+      continue;
+    }
     double L = 0.0;
 #pragma unroll
     for (int f = 0; f < NF; ++f) {
@@ -246,18 +331,67 @@ __device__ __forceinline__ void update_cells(const Img &m, const UpdateArgs &a, 
     // the last stage's tendency enters only its own sum (no later stage reads it)
     if (a.sc.write_rate_only || a.stage < 2) a.K[int64_t(a.stage) * NV * n + at] = L;
     if (a.sc.write_rate_only) continue;
-    a.Unext[at] = base[p] + dt * (part[p] + a.sc.cl * L);
+    const double un = base[p] + dt * (part[p] + a.sc.cl * L);
+    check(base[p], un);
+    base[p] = un;
+    a.Unext[at] = un;
   }
+  if (chk.cfl == nullptr) return;
+  // the CFL minimum of the new state: its values go through LDS to one lane a cell
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+#pragma unroll
+  for (int p = 0; p < NP; ++p)
+    if (p * 64 + lane < CW * NV) lds[p * 64 + lane] = base[p];
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+  double r = 1.0e300;
+  if (lane < CW && i0 + lane < n) r = cfl_of_cell<DIM>(lds + lane * NV, m.inr[i0 + lane], m.gamma);
+  for (int off = 32; off > 0; off >>= 1) r = fmin(r, __shfl_down(r, off, 64));
+  if (lane == 0) atomicMin(chk.cfl, (unsigned long long)__double_as_longlong(r));
 }
 
 template <int DIM, int Q>
-__global__ __launch_bounds__(256, 3) void k_update(Img m, UpdateArgs a, const double *dtp) {
+__global__ __launch_bounds__(256, 3) void k_update(Img m, UpdateArgs a) {
   __shared__ double flux[4][update_cells_of_wave(DIM) * (DIM + 1) * (DIM + 2)];
-  const double dt = dtp ? *dtp : a.dt;  // zfv_advance: the step's dt, chosen on the device
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int64_t tile = xcd_block(blockIdx.x, gridDim.x) * 4 + wave;
   if (tile * update_cells_of_wave(DIM) >= m.n) return;
-  update_cells<DIM, Q>(m, a, dt, tile, threadIdx.x & 63, flux[wave]);
+  update_cells<DIM, Q>(m, a, a.dt, UpdateChecks{nullptr, 0.0, nullptr}, tile, threadIdx.x & 63, flux[wave]);
+}
+
+// the update inside the time loop of zfv_advance, with its bookkeeping: the
+// first stage picks the step's dt (every wavefront for itself, the first one
+// for the record), the second sets the CFL words back and, without step
+// rejection, advances the time, the third reduces the next step's CFL minimum
+template <int DIM, int Q>
+__global__ __launch_bounds__(256, 3) void k_update_adv(Img m, UpdateArgs a, AdvState *adv, unsigned long long *slots) {
+  __shared__ double flux[4][update_cells_of_wave(DIM) * (DIM + 1) * (DIM + 2)];
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int lane = threadIdx.x & 63;
+  const int64_t tile = xcd_block(blockIdx.x, gridDim.x) * 4 + wave;
+  if (tile * update_cells_of_wave(DIM) >= m.n) return;
+  double dt;
+  if (a.stage == 0) {
+    double r = __longlong_as_double((long long)slots[lane * kAdvSlotStride]);
+    for (int off = 32; off > 0; off >>= 1) r = fmin(r, __shfl_xor(r, off, 64));
+    dt = adv_pick(*adv, r);
+    if (tile == 0 && lane == 0) {
+      adv->dt = dt;
+      if (!(dt > 0.0)) adv->active = 0;
+    }
+  } else {
+    dt = adv->dt;
+    if (a.stage == 1 && tile == 0) {
+      slots[lane * kAdvSlotStride] = adv_no_bound();
+      if (lane == 0 && !(adv->drho_crit > 0.0)) adv_end(adv);
+    }
+  }
+  UpdateChecks chk{nullptr, 0.0, nullptr};
+  if (a.stage == 2) chk = UpdateChecks{slots + (tile & (kAdvSlots - 1)) * kAdvSlotStride, adv->drho_crit, &adv->bad};
+  update_cells<DIM, Q>(m, a, dt, chk, tile, lane, flux[wave]);
 }
 
 // LocalCFL: min_i inradius_i / (|v_i| + a_i); positive doubles order like
@@ -271,14 +405,7 @@ __global__ __launch_bounds__(256) void k_cfl(Img m, const double *__restrict__ U
   for (int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x; i < n; i += int64_t(gridDim.x) * blockDim.x) {
     double u[NV];
     for (int v = 0; v < NV; ++v) u[v] = U[i * NV + v];
-    double m2 = u[1] * u[1] + u[2] * u[2];
-    if (DIM == 3) m2 += u[3] * u[3];
-    double v2 = m2 / (u[0] * u[0]);
-    double p = (u[NV - 1] - 0.5 * m2 / u[0]) * (m.gamma - 1.0);
-    double a = sqrt(m.gamma * p / u[0]);
-    double ri = m.inr[i] / (sqrt(v2) + a);
-    if (!(ri > 0.0)) ri = 0.0;  // NaN / non-positive states surface as dt = 0
-    r = fmin(r, ri);
+    r = fmin(r, cfl_of_cell<DIM>(u, m.inr[i], m.gamma));
   }
   // wavefront reduction
   for (int off = 32; off > 0; off >>= 1) r = fmin(r, __shfl_down(r, off, 64));
@@ -421,17 +548,20 @@ __global__ __launch_bounds__(256, 3) void kb_update(DevInst *insts, const BlockR
   a.stage = stage;
   a.dt = 0.0;
   double dt = d.dt;
+  const bool first = b.local == 0 && threadIdx.x == 0;
   if (stage == 0) {
-    // the step's dt, from the CFL minimum of this step: every thread of the
-    // member forms the same value; the member's first thread records it for
-    // the later stages and the step's end (and stops a member that cannot
-    // advance, whose threads all leave here)
+    // the step's dt, from the CFL minimum of the member's state: every thread
+    // of the member forms the same value; the member's first thread records
+    // it for the later stages (and stops a member that cannot advance or has
+    // finished, whose threads all leave here)
     dt = kb_step_dt(d);
-    if (b.local == 0 && threadIdx.x == 0) {
-      d.dt = dt;
-      if (!(dt > 0.0)) d.active = 0;
-    }
+    if (first) kb_begin_instance(d, dt);
     if (!(dt > 0.0)) return;
+  } else {
+    if (!d.running) return;
+    // the time and the CFL minimum are not read before the next step's first
+    // stage but by the last stage's reduction
+    if (stage == 1 && first) kb_end_instance(d);
   }
   a.Ustage = stage == 0 ? d.U : d.X;
   a.fpv = d.fpv;
@@ -442,7 +572,8 @@ __global__ __launch_bounds__(256, 3) void kb_update(DevInst *insts, const BlockR
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int64_t tile = int64_t(b.local) * 4 + wave;
   if (tile * update_cells_of_wave(DIM) >= d.m.n) return;
-  update_cells<DIM, Q>(d.m, a, dt, tile, threadIdx.x & 63, flux[wave]);
+  update_cells<DIM, Q>(d.m, a, dt, UpdateChecks{stage == 2 ? &d.dt_bits : nullptr, 0.0, nullptr}, tile,
+                       threadIdx.x & 63, flux[wave]);
 }
 
 template <int DIM>
@@ -466,104 +597,27 @@ __global__ __launch_bounds__(256) void kb_cfl(DevInst *insts, const BlockRef *bl
 }
 
 
-// A single instance's time loop on the device (zfv_advance): TimeLoop's
-// step with LocalCFL (src/zisa/fvm_loops/time_loop.cpp:36-81,
-// include/zisa/model/local_cfl_condition_impl.hpp:25-40), dt clamped to the
-// end time as the simulation clock does (its library is not vendored in the
-// reference), with no host round trip per step.
-struct AdvState {
-  double t, t_end, cfl, dt;
-  unsigned long long dt_bits;
-  int steps, max_steps, active, pad;
-  // RejectLargeDensityChange (src/zisa/ode/step_rejection.cpp:17-57; off
-  // when drho_crit <= 0): factor scales the CFL step, halves on a rejected
-  // step (which is retried with factor * its dt, TimeLoop::reject_step,
-  // src/zisa/fvm_loops/time_loop.cpp:182-196) and doubles after two good
-  // steps in a row, within [min_factor, 1]
-  double drho_crit, factor, min_factor, retry_dt;
-  int bad, prev_good, retry, rejections;
-};
-
-// start value of the CFL reduction (bits of 1e300)
-__host__ __device__ inline unsigned long long adv_no_bound() {
-  const double big = 1.0e300;
-  unsigned long long bits;
-  memcpy(&bits, &big, sizeof(bits));
-  return bits;
-}
-
-// keeps u0 for a step that may be rejected (only with step rejection on)
-__global__ __launch_bounds__(256) void k_adv_backup(const AdvState *a, int64_t count, const double *U,
-                                                    double *Ubk) {
-  if (!(a->drho_crit > 0.0) || !a->active) return;
-  const int64_t k = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (k < count) Ubk[k] = U[k];
-}
-
-// RejectLargeDensityChange::check: |rho1 - rho0| > drho_crit rho0 in any cell
-// (the density is the first of a cell's nv values)
-__global__ __launch_bounds__(256) void k_adv_check(AdvState *a, int64_t n, int nv, const double *U,
-                                                   const double *Ubk) {
-  if (!(a->drho_crit > 0.0) || !a->active) return;
-  const int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  const double r0 = Ubk[i * nv], r1 = U[i * nv];
-  if (fabs(r0 - r1) > a->drho_crit * r0) atomicOr(&a->bad, 1);
-}
-
-// a rejected step leaves the state as it was
-__global__ __launch_bounds__(256) void k_adv_restore(const AdvState *a, int64_t count, double *U,
-                                                     const double *Ubk) {
-  if (!a->bad || !a->active) return;
-  const int64_t k = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (k < count) U[k] = Ubk[k];
-}
-
-__global__ void k_adv_choose(AdvState *a) {
-  double m;
-  unsigned long long bits = a->dt_bits;
-  memcpy(&m, &bits, sizeof(m));
-  // StepRejection::pick_time_step: factor * the CFL step, or the retry step
-  double dt = a->retry ? a->retry_dt : a->factor * (a->cfl * m);
-  const double rest = a->t_end - a->t;
-  if (dt > rest) dt = rest;
-  // stop when finished, when the CFL gives no positive step (a non-physical
-  // state) or when the step no longer advances the time
-  if (!a->active || !(dt > 0.0) || a->t + dt == a->t) {
-    dt = 0.0;  // a finished run's stages leave U as it is (U + 0 * dudt)
-    a->active = 0;
+// The end of a step that may be rejected: the new state (in X) becomes the
+// state unless it is bad; the last block to finish closes the step.  (The step
+// leaves the old state alone until here, so nothing is backed up or restored.)
+__global__ __launch_bounds__(256) void k_adv_commit(AdvState *a, int64_t count, double *U, const double *X) {
+  if (!a->bad && a->active)
+    for (int64_t k = int64_t(blockIdx.x) * blockDim.x + threadIdx.x; k < count; k += int64_t(gridDim.x) * blockDim.x)
+      U[k] = X[k];
+  __syncthreads();  // every thread has read bad and active
+  if (threadIdx.x == 0 && atomicAdd(&a->blocks_done, 1u) + 1 == gridDim.x) {
+    a->blocks_done = 0;
+    adv_end(a);
   }
-  a->dt = dt;
 }
 
-__global__ void k_adv_end(AdvState *a) {
-  if (!a->active) return;
-  const int bad = a->bad;
-  // the next step's CFL reduction and density check start here
-  a->dt_bits = adv_no_bound();
-  a->bad = 0;
-  a->retry = 0;
-  if (a->drho_crit > 0.0) {
-    const double f = a->factor;
-    if (bad) {
-      a->prev_good = 0;
-      a->factor = fmax(a->min_factor, fmin(f / 2.0, 1.0));
-      a->retry = 1;
-      a->retry_dt = a->factor * a->dt;
-      a->rejections += 1;
-      return;  // the time does not advance; the state was restored
-    }
-    a->factor = fmax(a->min_factor, fmin(a->prev_good ? f * 2.0 : f, 1.0));
-    a->prev_good = 1;
-  }
-  a->t += a->dt;
-  a->steps += 1;
-  if (a->t >= a->t_end || a->steps >= a->max_steps) a->active = 0;
-}
+// the CFL words of a time loop before its first reduction
+__global__ void k_adv_slots(unsigned long long *slots) { slots[threadIdx.x * kAdvSlotStride] = adv_no_bound(); }
 
-__global__ void kb_end_step(DevInst *insts, int n_inst) {
+// the members' CFL minima before the first step of a launch
+__global__ void kb_begin_launch(DevInst *insts, int n_inst) {
   const int k = blockIdx.x * blockDim.x + threadIdx.x;
-  if (k < n_inst) kb_end_instance(insts[k]);
+  if (k < n_inst) insts[k].dt_bits = kb_no_bound();
 }
 
 // plain streaming copy (16-byte vectors, grid-stride) for bandwidth calibration
@@ -588,7 +642,8 @@ struct Launcher {
   // rec[ph]: physics set ph (PH_LIGHT / PH_FULL / PH_LIN); cfg: reconstruction
   // launch configuration (rec_cfg_waves)
   void (*rec[3])(const Img &, const double *, double *, double *, int cfg, int skip_far_ghosts, hipStream_t);
-  void (*update)(const Img &, const UpdateArgs &, const double *dtp, hipStream_t);
+  void (*update)(const Img &, const UpdateArgs &, hipStream_t);
+  void (*update_adv)(const Img &, const UpdateArgs &, AdvState *, unsigned long long *slots, hipStream_t);
   void (*cfl)(const Img &, const double *, unsigned long long *, hipStream_t);
   void (*source_moments)(const Img &, double *, hipStream_t);  // setup: Img::smom
   // batched variants: grid = number of block-table entries
@@ -642,8 +697,12 @@ Launcher make_launcher() {
   l.rec[PH_LIN] = [](const Img &m, const double *U, double *fpv, double *src, int cfg, int skip, hipStream_t s) {
     launch_rec<DIM, DOFC, RC, NB, RB, Q, PH_LIN>(m, U, fpv, src, cfg, skip, s);
   };
-  l.update = [](const Img &m, const UpdateArgs &a, const double *dtp, hipStream_t s) {
-    hipLaunchKernelGGL((k_update<DIM, Q>), dim3(xcd_grid(m.n, update_cells_of_block(DIM))), dim3(256), 0, s, m, a, dtp);
+  l.update = [](const Img &m, const UpdateArgs &a, hipStream_t s) {
+    hipLaunchKernelGGL((k_update<DIM, Q>), dim3(xcd_grid(m.n, update_cells_of_block(DIM))), dim3(256), 0, s, m, a);
+  };
+  l.update_adv = [](const Img &m, const UpdateArgs &a, AdvState *adv, unsigned long long *slots, hipStream_t s) {
+    hipLaunchKernelGGL((k_update_adv<DIM, Q>), dim3(xcd_grid(m.n, update_cells_of_block(DIM))), dim3(256), 0, s, m, a,
+                       adv, slots);
   };
   l.cfl = [](const Img &m, const double *U, unsigned long long *out, hipStream_t s) {
     hipLaunchKernelGGL((k_cfl<DIM>), dim3(std::min(blocks_for(m.n, 256), 512u)), dim3(256), 0, s, m, U, out);
@@ -713,7 +772,7 @@ struct zfv_handle {
   double graph_dt = -1.0;
   int graph_steps = 0;
   zfv::AdvState *adv = nullptr;           // device time-loop state (zfv_advance)
-  double *Ubk = nullptr;                  // u0 of a step that may be rejected
+  unsigned long long *adv_slots = nullptr;  // its CFL words
   hipGraphExec_t adv_graph[2] = {nullptr, nullptr};  // one adaptive step, without / with step rejection
   int rec_cfg = -1;   // reconstruction launch configuration; -1 = not tuned yet
   double rec_ms[zfv::kRecConfigs] = {0, 0, 0};
@@ -827,8 +886,7 @@ static void tune_rec(zfv_handle *h, const double *Ustate) {
         if (k >= 0) HIP_CHECK(hipEventRecord(ev[2 * k], h->stream));
         h->L.rec[h->ph](m, Ustate, h->fpv, h->src, c, frozen(h), h->stream);
         if (k >= 0) HIP_CHECK(hipEventRecord(ev[2 * k + 1], h->stream));
-        h->L.update(m, UpdateArgs{rate_only, 0, 0.0, Ustate, h->fpv, h->src, Ustate, h->K, nullptr}, nullptr,
-                    h->stream);
+        h->L.update(m, UpdateArgs{rate_only, 0, 0.0, Ustate, h->fpv, h->src, Ustate, h->K, nullptr}, h->stream);
       }
       HIP_CHECK(hipEventSynchronize(ev[2 * kTimed - 1]));
       HIP_CHECK(hipGetLastError());
@@ -861,7 +919,7 @@ static void enqueue_step(zfv_handle *h, double dt) {
   for (int s = 0; s < 3; ++s) {
     h->L.rec[h->ph](m, Us, h->fpv, h->src, h->rec_cfg, frozen(h), h->stream);
     double *Un = (s == 2) ? h->U : h->X;
-    h->L.update(m, UpdateArgs{ssp3_coeffs(s), s, dt, Us, h->fpv, h->src, h->U, h->K, Un}, nullptr, h->stream);
+    h->L.update(m, UpdateArgs{ssp3_coeffs(s), s, dt, Us, h->fpv, h->src, h->U, h->K, Un}, h->stream);
     Us = h->X;
   }
 }
@@ -876,29 +934,32 @@ static void drop_graphs(zfv_handle *h) {
   h->graph_exec = nullptr;
 }
 
-// one step with the dt the device chooses (LocalCFL, clamped to t_end);
-// with reject, the step is undone when the density changes too much.  adv is
-// the loop state and Ubk the backup of u0 (used only with reject).
-static void enqueue_adaptive_step(zfv_handle *h, bool reject, int cfg, AdvState *adv, double *Ubk) {
+// one step with the dt the device chooses (LocalCFL, clamped to t_end); with
+// reject, the last stage leaves the new state in X and the step ends by taking
+// it over or not
+static void enqueue_adaptive_step(zfv_handle *h, bool reject, int cfg, AdvState *adv, unsigned long long *slots) {
   const Img &m = h->dimg;
-  const int64_t count = int64_t(h->img.s.nvars) * m.n;
-  if (reject)
-    hipLaunchKernelGGL(k_adv_backup, dim3(blocks_for(count, 256)), dim3(256), 0, h->stream, adv, count, h->U, Ubk);
-  h->L.cfl(m, h->U, &adv->dt_bits, h->stream);
-  hipLaunchKernelGGL(k_adv_choose, dim3(1), dim3(1), 0, h->stream, adv);
   const double *Us = h->U;
   for (int s = 0; s < 3; ++s) {
     h->L.rec[h->ph](m, Us, h->fpv, h->src, cfg, frozen(h), h->stream);
-    double *Un = (s == 2) ? h->U : h->X;
-    h->L.update(m, UpdateArgs{ssp3_coeffs(s), s, 0.0, Us, h->fpv, h->src, h->U, h->K, Un}, &adv->dt, h->stream);
+    double *Un = (s == 2 && !reject) ? h->U : h->X;
+    h->L.update_adv(m, UpdateArgs{ssp3_coeffs(s), s, 0.0, Us, h->fpv, h->src, h->U, h->K, Un}, adv, slots, h->stream);
     Us = h->X;
   }
   if (reject) {
-    hipLaunchKernelGGL(k_adv_check, dim3(blocks_for(m.n, 256)), dim3(256), 0, h->stream, adv, m.n, h->img.s.nvars,
-                       h->U, Ubk);
-    hipLaunchKernelGGL(k_adv_restore, dim3(blocks_for(count, 256)), dim3(256), 0, h->stream, adv, count, h->U, Ubk);
+    const int64_t count = int64_t(h->img.s.nvars) * m.n;
+    hipLaunchKernelGGL(k_adv_commit, dim3(std::min(blocks_for(count, 256), 512u)), dim3(256), 0, h->stream, adv, count,
+                       h->U, h->X);
   }
-  hipLaunchKernelGGL(k_adv_end, dim3(1), dim3(1), 0, h->stream, adv);
+}
+
+// the loop state and the CFL words before the first step
+static void enqueue_adaptive_start(zfv_handle *h, const AdvState &a, AdvState *adv, unsigned long long *slots) {
+  HIP_CHECK(hipMemcpyAsync(adv, &a, sizeof(a), hipMemcpyHostToDevice, h->stream));
+  hipLaunchKernelGGL(k_adv_slots, dim3(1), dim3(kAdvSlots), 0, h->stream, slots);
+  h->L.cfl(h->dimg, h->U, slots, h->stream);
+  HIP_CHECK(hipGetLastError());
+  HIP_CHECK(hipStreamSynchronize(h->stream));
 }
 
 // The loop state of a device time loop starting at t0 (zfv_advance and its
@@ -916,7 +977,7 @@ static AdvState adv_start(double cfl_number, double t0, double t_end, int32_t ma
   a.factor = 1.0;
   a.min_factor = drho_crit_rel > 0.0 ? std::pow(2.0, -double(max_exponent)) : 1.0;
   a.prev_good = 1;
-  a.dt_bits = adv_no_bound();
+  a.blocks_done = 0;
   a.bad = 0;
   return a;
 }
@@ -935,6 +996,7 @@ static void check_advance_args(double cfl_number, double drho_crit_rel, int32_t 
 constexpr size_t kNoAllocScratchBytes = size_t(16) << 20;
 constexpr size_t kNoAllocStateBytes = 256;
 static_assert(sizeof(AdvState) <= kNoAllocStateBytes, "loop state larger than its scratch slot");
+static_assert(kNoAllocStateBytes + kAdvSlotBytes <= kNoAllocScratchBytes, "CFL words outside the scratch");
 static __device__ __align__(256) unsigned char scratch[kNoAllocScratchBytes];
 
 constexpr int kMaxDevices = 64;
@@ -1296,7 +1358,7 @@ int zfv_rate(zfv_handle *h, const double *u, double *dudt, double t) {
   h->L.rec[h->ph](m, h->X, h->fpv, h->src, rec_config(h, h->X), 0, h->stream);
   StageCoeffs sc{};
   sc.write_rate_only = 1;
-  h->L.update(m, UpdateArgs{sc, 0, 0.0, h->X, h->fpv, h->src, h->X, h->K, h->X}, nullptr, h->stream);
+  h->L.update(m, UpdateArgs{sc, 0, 0.0, h->X, h->fpv, h->src, h->X, h->K, h->X}, h->stream);
   HIP_CHECK(hipGetLastError());
   HIP_CHECK(hipMemcpyAsync(h->host_stage, h->K, sizeof(double) * nv * n, hipMemcpyDeviceToHost, h->stream));
   HIP_CHECK(hipStreamSynchronize(h->stream));
@@ -1352,19 +1414,18 @@ int zfv_advance(zfv_handle *h, double cfl_number, double t0, double t_end, int32
   rec_config(h, h->U);
   if (!h->adv) h->adv = h->alloc<AdvState>(1);
   const bool reject = drho_crit_rel > 0.0;
-  if (reject && !h->Ubk) h->Ubk = h->alloc<double>(size_t(h->img.s.nvars) * h->img.n);
+  if (!h->adv_slots) h->adv_slots = h->alloc<unsigned long long>(kAdvSlots * kAdvSlotStride);
   hipGraphExec_t &step = h->adv_graph[reject ? 1 : 0];
   if (!step) {
     hipGraph_t graph;
     HIP_CHECK(hipStreamBeginCapture(h->stream, hipStreamCaptureModeThreadLocal));
-    enqueue_adaptive_step(h, reject, h->rec_cfg, h->adv, h->Ubk);
+    enqueue_adaptive_step(h, reject, h->rec_cfg, h->adv, h->adv_slots);
     HIP_CHECK(hipStreamEndCapture(h->stream, &graph));
     HIP_CHECK(hipGraphInstantiate(&step, graph, nullptr, nullptr, 0));
     HIP_CHECK(hipGraphDestroy(graph));
   }
   AdvState a = adv_start(cfl_number, t0, t_end, max_steps, drho_crit_rel, max_exponent);
-  HIP_CHECK(hipMemcpyAsync(h->adv, &a, sizeof(a), hipMemcpyHostToDevice, h->stream));
-  HIP_CHECK(hipStreamSynchronize(h->stream));
+  enqueue_adaptive_start(h, a, h->adv, h->adv_slots);
   while (a.active) {
     for (int k = 0; k < check_every; ++k) HIP_CHECK(hipGraphLaunch(step, h->stream));
     HIP_CHECK(hipMemcpyAsync(&a, h->adv, sizeof(a), hipMemcpyDeviceToHost, h->stream));
@@ -1396,16 +1457,15 @@ int zfv_advance_noalloc(zfv_handle *h, double cfl_number, double t0, double t_en
                                        " bytes (use zfv_advance)");
   unsigned char *sp = scratch_on(dev);
   AdvState *adv = reinterpret_cast<AdvState *>(sp);
-  double *Ubk = reinterpret_cast<double *>(sp + kNoAllocStateBytes);
+  auto *slots = reinterpret_cast<unsigned long long *>(sp + kNoAllocStateBytes);
   // no tuning here (it creates events): the tuned launch configuration when
   // there is one, else one wavefront per block; results do not depend on it
   const int cfg = h->rec_cfg >= 0 ? h->rec_cfg : 0;
   // the whole loop state is written before the first step reads any of it
   AdvState a = adv_start(cfl_number, t0, t_end, max_steps, drho_crit_rel, max_exponent);
-  HIP_CHECK(hipMemcpyAsync(adv, &a, sizeof(a), hipMemcpyHostToDevice, h->stream));
-  HIP_CHECK(hipStreamSynchronize(h->stream));
+  enqueue_adaptive_start(h, a, adv, slots);
   while (a.active) {
-    for (int k = 0; k < check_every; ++k) enqueue_adaptive_step(h, reject, cfg, adv, Ubk);
+    for (int k = 0; k < check_every; ++k) enqueue_adaptive_step(h, reject, cfg, adv, slots);
     HIP_CHECK(hipGetLastError());
     HIP_CHECK(hipMemcpyAsync(&a, adv, sizeof(a), hipMemcpyDeviceToHost, h->stream));
     HIP_CHECK(hipStreamSynchronize(h->stream));
@@ -1525,7 +1585,7 @@ int zfv_time_kernels(zfv_handle *h, int32_t n_steps, double dt, zfv_kernel_times
       HIP_CHECK(hipEventRecord(ev[k++], h->stream));
       double *Un = (s == 2) ? h->U : h->X;
       HIP_CHECK(hipEventRecord(ev[k++], h->stream));
-      h->L.update(m, UpdateArgs{ssp3_coeffs(s), s, dt, Us, h->fpv, h->src, h->U, h->K, Un}, nullptr, h->stream);
+      h->L.update(m, UpdateArgs{ssp3_coeffs(s), s, dt, Us, h->fpv, h->src, h->U, h->K, Un}, h->stream);
       HIP_CHECK(hipEventRecord(ev[k++], h->stream));
       Us = h->X;
     }
@@ -1662,6 +1722,7 @@ struct zfv_batch {
   hipGraphExec_t graph = nullptr;
   bool dirty = true;
   bool in_flight = false;  // steps launched (zfv_batch_launch) and not yet waited for
+  bool cfl_ready = false;  // the members' CFL minima belong to their present states
   ~zfv_batch() {
     if (stream) (void)hipStreamSynchronize(stream);
     for (zfv_handle *h : members)
@@ -1702,11 +1763,17 @@ static void batch_sync_down(zfv_batch *b) {
                            b->stream));
   HIP_CHECK(hipStreamSynchronize(b->stream));
   b->in_flight = false;
+  // a member that has reached its end is stopped by the next step's first stage
+  for (DevInst &d : b->h_inst)
+    if (kb_finished(d)) d.active = 0;
 }
 
 // a member's own calls wait for its batch's steps in flight
+// (and may change its state)
 static void member_settle(zfv_handle *h) {
-  if (h->batch && h->batch->in_flight) batch_sync_down(h->batch);
+  if (!h->batch) return;
+  if (h->batch->in_flight) batch_sync_down(h->batch);
+  h->batch->cfl_ready = false;
 }
 
 static void batch_upload(zfv_batch *b) {
@@ -1752,6 +1819,7 @@ static void batch_upload(zfv_batch *b) {
   HIP_CHECK(hipMemcpyAsync(b->d_brec, tr.data(), sizeof(BlockRef) * tr.size(), hipMemcpyHostToDevice, b->stream));
   HIP_CHECK(hipStreamSynchronize(b->stream));
   b->dirty = false;
+  b->cfl_ready = false;
 }
 
 // The batch's reconstruction geometry, tuned like a single instance's: each
@@ -1811,16 +1879,19 @@ static bool batch_has_active(const zfv_batch *b) {
 }
 
 static void batch_enqueue_step(zfv_batch *b) {
-  const unsigned nc = unsigned(b->n_cell_blocks), nu = unsigned(b->n_upd_blocks), nr = unsigned(b->n_rec_blocks);
-  const unsigned ib = unsigned((b->max_inst + 63) / 64);
-  // the step's CFL minimum (reset at the end of the previous step or when
-  // the member joined); stage 0's update turns it into the step's dt
-  b->L.bcfl(b->d_inst, b->d_bcell, nc, b->stream);
+  const unsigned nu = unsigned(b->n_upd_blocks), nr = unsigned(b->n_rec_blocks);
   for (int s = 0; s < 3; ++s) {
     b->L.brec[b->ph](b->d_inst, b->d_brec, nr, s, b->rec_cfg, b->stream);
     b->L.bupdate(b->d_inst, b->d_bupd, nu, s, b->stream);
   }
-  hipLaunchKernelGGL(kb_end_step, dim3(ib), dim3(64), 0, b->stream, b->d_inst, b->max_inst);
+}
+
+// the members' CFL minima of the states they have now (a step leaves the next
+// one's, but members join and their states are set between launches)
+static void batch_enqueue_cfl(zfv_batch *b) {
+  hipLaunchKernelGGL(kb_begin_launch, dim3(unsigned((b->max_inst + 63) / 64)), dim3(64), 0, b->stream, b->d_inst,
+                     b->max_inst);
+  b->L.bcfl(b->d_inst, b->d_bcell, unsigned(b->n_cell_blocks), b->stream);
 }
 
 static void batch_forget(zfv_batch *b, int slot) {
@@ -1964,6 +2035,11 @@ int zfv_batch_launch(zfv_batch *b, int32_t n_steps) {
     HIP_CHECK(hipStreamEndCapture(b->stream, &g));
     HIP_CHECK(hipGraphInstantiate(&b->graph, g, nullptr, nullptr, 0));
     HIP_CHECK(hipGraphDestroy(g));
+  }
+  if (n_steps > 0 && !b->cfl_ready) {
+    batch_enqueue_cfl(b);
+    HIP_CHECK(hipGetLastError());
+    b->cfl_ready = true;  // every step leaves the next one's
   }
   for (int k = 0; k < n_steps; ++k) HIP_CHECK(hipGraphLaunch(b->graph, b->stream));
   b->in_flight = true;

@@ -1968,6 +1968,20 @@ ZFV_HD void reconstruct_lane(const Img &m, int64_t i, const int g, X &xch, const
   }
 }
 
+// LocalCFL's candidate of a cell of inradius inr: inradius / (|v| + a); 0 for a
+// NaN or non-physical state, which surfaces as dt = 0
+// (include/zisa/model/local_cfl_condition_impl.hpp:25-40)
+template <int DIM>
+ZFV_HD double cfl_of_cell(const double *u, double inr, double gamma) {
+  double m2 = u[1] * u[1] + u[2] * u[2];
+  if (DIM == 3) m2 += u[3] * u[3];
+  const double v2 = m2 / (u[0] * u[0]);
+  const double p = (u[DIM + 1] - 0.5 * m2 / u[0]) * (gamma - 1.0);
+  const double a = sqrt(gamma * p / u[0]);
+  const double r = inr / (sqrt(v2) + a);
+  return r > 0.0 ? r : 0.0;
+}
+
 // ---- the per-face flux ----------------------------------------------------------
 // the flux through interior face e from its left to its right cell (global
 // frame, times the face's measure), which the left cell loses and the right
