@@ -111,7 +111,7 @@ constexpr int rec_min_waves(int ph) { return ph == PH_FULL ? 1 : 3; }
 // k_reconstruct: blocks of `blockDim.x / 64` waves, 64 / NV cells per wave
 template <int DIM, int DOFC, int RC, int NB, int RB, int Q, int PH>
 __global__ __launch_bounds__(256, rec_min_waves(PH)) void k_reconstruct(
-    Img m, const double *__restrict__ U, double *__restrict__ fpv, double *__restrict__ src, int skip_far_ghosts) {
+    Img m, int64_t n, const double *__restrict__ U, double *__restrict__ fpv, double *__restrict__ src) {
   constexpr int NV = DIM + 2;
   constexpr int GPW = groups_per_wave<NV>();
   // one slice of slice_doubles doubles per cell group, sized at launch
@@ -123,10 +123,7 @@ __global__ __launch_bounds__(256, rec_min_waves(PH)) void k_reconstruct(
   const int g = lane - grp * NV;
   const int64_t blk = xcd_block(blockIdx.x, gridDim.x);
   const int64_t i = (blk * (blockDim.x >> 6) + wave) * GPW + grp;
-  if (grp >= GPW || i >= m.n) return;  // whole groups leave together
-  // under the frozen BC a ghost cell away from the interior feeds no flux and
-  // its own tendency is overwritten: nothing to reconstruct
-  if (skip_far_ghosts && (m.meta[i] & META_FAR_GHOST) == META_FAR_GHOST) return;
+  if (grp >= GPW || i >= n) return;  // whole groups leave together
   double *wv = &slices[wave * wave_block_doubles<DIM, DOFC, RC>()];
   double *sl = wv + wave_lds_doubles<DIM, DOFC>() + grp * group_lds_doubles<RC>();
   if constexpr (NV == 4) {
@@ -229,7 +226,7 @@ struct UpdateChecks {
 struct UpdateArgs {
   StageCoeffs sc;
   int stage;
-  double dt;
+  double dt;  // (zfv_advance: chosen on the device)
   const double *Ustage, *fpv, *src, *U0;
   double *K, *Unext;
 };
@@ -353,12 +350,19 @@ __device__ __forceinline__ void update_cells(const Img &m, const UpdateArgs &a, 
   if (lane == 0) atomicMin(chk.cfl, (unsigned long long)__double_as_longlong(r));
 }
 
+// The cells that a stage's update covers: under the frozen BC the second leaves
+// out the ghosts away from the interior, whose X the first has set (the third
+// sets U)
+__host__ __device__ inline int64_t update_cells_of_stage(const Img &m, const UpdateArgs &a) {
+  return !a.sc.write_rate_only && m.steady != nullptr && a.stage == 1 && m.n_near > 0 ? m.n_near : m.n;
+}
+
 template <int DIM, int Q>
 __global__ __launch_bounds__(256, 3) void k_update(Img m, UpdateArgs a) {
   __shared__ double flux[4][update_cells_of_wave(DIM) * (DIM + 1) * (DIM + 2)];
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int64_t tile = xcd_block(blockIdx.x, gridDim.x) * 4 + wave;
-  if (tile * update_cells_of_wave(DIM) >= m.n) return;
+  if (tile * update_cells_of_wave(DIM) >= update_cells_of_stage(m, a)) return;
   update_cells<DIM, Q>(m, a, a.dt, UpdateChecks{nullptr, 0.0, nullptr}, tile, threadIdx.x & 63, flux[wave]);
 }
 
@@ -372,7 +376,7 @@ __global__ __launch_bounds__(256, 3) void k_update_adv(Img m, UpdateArgs a, AdvS
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int lane = threadIdx.x & 63;
   const int64_t tile = xcd_block(blockIdx.x, gridDim.x) * 4 + wave;
-  if (tile * update_cells_of_wave(DIM) >= m.n) return;
+  if (tile * update_cells_of_wave(DIM) >= update_cells_of_stage(m, a)) return;
   double dt;
   if (a.stage == 0) {
     double r = __longlong_as_double((long long)slots[lane * kAdvSlotStride]);
@@ -674,8 +678,12 @@ void launch_rec(const Img &m, const double *U, double *fpv, double *src, int cfg
   const int waves = rec_cfg_waves(cfg);
   const int cpb = waves * groups_per_wave<DIM + 2>();
   const unsigned lds = rec_lds_bytes<DIM, DOFC, RC>(waves);
-  hipLaunchKernelGGL((k_reconstruct<DIM, DOFC, RC, NB, RB, Q, PH>), dim3(xcd_grid(m.n, cpb)), dim3(64 * waves), lds, s,
-                     m, U, fpv, src, skip);
+  // under the frozen BC a ghost cell away from the interior feeds no flux and
+  // its own tendency is overwritten: nothing to reconstruct (the last cells)
+  const int64_t n = skip ? m.n_near : m.n;
+  if (n == 0) return;
+  hipLaunchKernelGGL((k_reconstruct<DIM, DOFC, RC, NB, RB, Q, PH>), dim3(xcd_grid(n, cpb)), dim3(64 * waves), lds, s, m,
+                     n, U, fpv, src);
 }
 
 template <int DIM, int DOFC, int RC, int NB, int RB, int Q, int PH>
@@ -698,11 +706,12 @@ Launcher make_launcher() {
     launch_rec<DIM, DOFC, RC, NB, RB, Q, PH_LIN>(m, U, fpv, src, cfg, skip, s);
   };
   l.update = [](const Img &m, const UpdateArgs &a, hipStream_t s) {
-    hipLaunchKernelGGL((k_update<DIM, Q>), dim3(xcd_grid(m.n, update_cells_of_block(DIM))), dim3(256), 0, s, m, a);
+    hipLaunchKernelGGL((k_update<DIM, Q>), dim3(xcd_grid(update_cells_of_stage(m, a), update_cells_of_block(DIM))),
+                       dim3(256), 0, s, m, a);
   };
   l.update_adv = [](const Img &m, const UpdateArgs &a, AdvState *adv, unsigned long long *slots, hipStream_t s) {
-    hipLaunchKernelGGL((k_update_adv<DIM, Q>), dim3(xcd_grid(m.n, update_cells_of_block(DIM))), dim3(256), 0, s, m, a,
-                       adv, slots);
+    hipLaunchKernelGGL((k_update_adv<DIM, Q>), dim3(xcd_grid(update_cells_of_stage(m, a), update_cells_of_block(DIM))),
+                       dim3(256), 0, s, m, a, adv, slots);
   };
   l.cfl = [](const Img &m, const double *U, unsigned long long *out, hipStream_t s) {
     hipLaunchKernelGGL((k_cfl<DIM>), dim3(std::min(blocks_for(m.n, 256), 512u)), dim3(256), 0, s, m, U, out);
@@ -1088,6 +1097,7 @@ int create_device(zfv_handle *h) {
   Img &m = h->dimg;
   m.n = im.n;
   m.ne = im.ne;
+  m.n_near = im.n_near;
   m.P = h->upload(im.P);
   m.rows = h->upload(im.rows);
   m.twin = h->upload(im.twin);

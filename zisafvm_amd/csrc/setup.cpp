@@ -1016,7 +1016,12 @@ void build_image(const zfv_mesh &mesh, const zfv_params &p, HostImage &img) {
   }
   img.perm.resize(n);
   std::iota(img.perm.begin(), img.perm.end(), 0);
-  std::stable_sort(img.perm.begin(), img.perm.end(), [&](int a, int b) { return key[a] < key[b]; });
+  // (ghost cells away from the interior last: steps under the frozen BC leave
+  // them out by their place)
+  std::stable_sort(img.perm.begin(), img.perm.end(), [&](int a, int b) {
+    return cs[a].first_order != cs[b].first_order ? cs[b].first_order : key[a] < key[b];
+  });
+  img.n_near = std::count_if(cs.begin(), cs.end(), [](const CellStencils &c) { return !c.first_order; });
   img.iperm.resize(n);
   for (int i = 0; i < n; ++i) img.iperm[img.perm[i]] = i;
 

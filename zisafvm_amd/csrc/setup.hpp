@@ -44,6 +44,7 @@ constexpr int CFACE_GHOST_PAIR = CFACE_EXTERIOR | CFACE_SIDE_R;
 struct HostImage {
   Shape s;
   int64_t n = 0;   // cells
+  int64_t n_near = 0;  // cells that are not ghosts away from the interior: the first ones
   int64_t ne = 0;  // interior faces
   std::vector<double> P;         // m * n in tiles of one wavefront's cells (p_central)
   std::vector<int32_t> rows;     // nrows * n   (product numbering)

@@ -45,6 +45,7 @@ constexpr int32_t ROW_CELL_MASK = (1 << ROW_CELL_BITS) - 1;
 struct Img {
   int64_t n;   // cells
   int64_t ne;  // interior faces
+  int64_t n_near;  // the first cells, those that are not ghosts away from the interior (META_FAR_GHOST)
   const double *P;
   const int32_t *rows;  // cell | shift_code << 27
   const int8_t *twin;   // (nrows - rc) * n: central row with the same member, or -1
