@@ -524,6 +524,18 @@ constexpr int32_t kBatchMaxMembers = 8;
 // tables between replays.  Block tables already place neighbouring blocks on
 // one XCD, so the kernels index them by blockIdx directly.
 
+// A table that no thread writes while the kernel runs, seen as constant
+// memory: its uniform loads are scalar, may move past the kernel's stores, and
+// pointers found in it are known to be global.
+template <class T>
+__device__ const T *unchanging(const T *p) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  return (const T *)(const __attribute__((address_space(4))) T *)reinterpret_cast<uintptr_t>(p);
+#else
+  return p;
+#endif
+}
+
 template <int DIM, int DOFC, int RC, int NB, int RB, int Q, int PH>
 __global__ __launch_bounds__(256, rec_min_waves(PH)) void kb_reconstruct(const DevInst *insts, const BlockRef *blk, int stage) {
   constexpr int NV = DIM + 2;
@@ -535,17 +547,18 @@ __global__ __launch_bounds__(256, rec_min_waves(PH)) void kb_reconstruct(const D
   const int wave = threadIdx.x >> 6;
   double *wv = &slices[wave * wave_block_doubles<DIM, DOFC, RC>()];
   WaveGroup x{lane - g, wv + wave_lds_doubles<DIM, DOFC>() + grp * group_lds_doubles<RC>(), wv};
-  kb_reconstruct_group<DIM, DOFC, RC, NB, RB, Q, PH>(insts, blk[blockIdx.x], blockDim.x >> 6, wave, grp, g, stage,
-                                                      x);
+  kb_reconstruct_group<DIM, DOFC, RC, NB, RB, Q, PH>(unchanging(insts), unchanging(blk)[blockIdx.x], blockDim.x >> 6,
+                                                      wave, grp, g, stage, x);
 }
 
 // one block updates update_cells_of_block cells of a member
 template <int DIM, int Q>
 __global__ __launch_bounds__(256, 3) void kb_update(DevInst *insts, const BlockRef *blk, int stage, StageCoeffs sc) {
   __shared__ double flux[4][update_cells_of_wave(DIM) * (DIM + 1) * (DIM + 2)];
-  const BlockRef b = blk[blockIdx.x];
+  const BlockRef b = unchanging(blk)[blockIdx.x];
   if (b.inst < 0) return;
-  DevInst &d = insts[b.inst];
+  DevInst &d = insts[b.inst];                   // the loop state
+  const DevInst &c = unchanging(insts)[b.inst];  // the rest: mesh, arrays
   if (!d.active) return;
   UpdateArgs a;
   a.sc = sc;
@@ -567,16 +580,16 @@ __global__ __launch_bounds__(256, 3) void kb_update(DevInst *insts, const BlockR
     // stage but by the last stage's reduction
     if (stage == 1 && first) kb_end_instance(d);
   }
-  a.Ustage = stage == 0 ? d.U : d.X;
-  a.fpv = d.fpv;
-  a.src = d.src;
-  a.U0 = d.U;
-  a.K = d.K;
-  a.Unext = stage == 2 ? d.U : d.X;
+  a.Ustage = stage == 0 ? c.U : c.X;
+  a.fpv = c.fpv;
+  a.src = c.src;
+  a.U0 = c.U;
+  a.K = c.K;
+  a.Unext = stage == 2 ? c.U : c.X;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int64_t tile = int64_t(b.local) * 4 + wave;
-  if (tile * update_cells_of_wave(DIM) >= d.m.n) return;
-  update_cells<DIM, Q>(d.m, a, dt, UpdateChecks{stage == 2 ? &d.dt_bits : nullptr, 0.0, nullptr}, tile,
+  if (tile * update_cells_of_wave(DIM) >= c.m.n) return;
+  update_cells<DIM, Q>(c.m, a, dt, UpdateChecks{stage == 2 ? &d.dt_bits : nullptr, 0.0, nullptr}, tile,
                        threadIdx.x & 63, flux[wave]);
 }
 
