@@ -1041,14 +1041,15 @@ ZFV_HD void rusanov(const double *uL, const double *uR, const double *n, double 
 // the member's equilibrium averages; group c at c NV row_doubles, an even
 // stride that puts the groups' 16-byte reads on different banks; at least 6,
 // which holds the exchange of the nonlinear weights), then per
-// cell group its central rows' member equilibrium averages (er, eE per row,
-// for the one-sided rows that share their member; group_lds_doubles).
+// cell group the members' equilibrium averages: er and eE of each central row,
+// for the one-sided rows that share their member, or in the light set er of
+// every row (group_lds_doubles; at least the 4 + 3 x 3 rows of 2D second order).
 template <int DOFC>
 constexpr int row_doubles() { return ((DOFC + 1 + 1) & ~1) > 6 ? ((DOFC + 1 + 1) & ~1) : 6; }
 template <int DIM, int DOFC>
 constexpr int wave_lds_doubles() { return (64 / (DIM + 2)) * (DIM + 2) * row_doubles<DOFC>(); }
 template <int RC>
-constexpr int group_lds_doubles() { return 2 * RC; }
+constexpr int group_lds_doubles() { return 2 * RC > 14 ? 2 * RC : 14; }
 template <int DIM, int DOFC, int RC>
 constexpr int wave_block_doubles() { return wave_lds_doubles<DIM, DOFC>() + (64 / (DIM + 2)) * group_lds_doubles<RC>(); }
 
@@ -1499,7 +1500,10 @@ ZFV_HD void reconstruct_lane(const Img &m, int64_t i, const int g, X &xch, const
     // registers, so that they are in flight during its arithmetic.
     constexpr int ROWW = row_doubles<DOFC>();
     double *pl = xch.wave_lds() + xch.lane0() * ROWW;  // this group's NV rows
-    double *ceq = xch.lds();                           // central rows' member averages (er, eE)
+    // the members' averages: (er, eE) of every central row; in the light set
+    // er of every row (eE is er times the cell constant b)
+    double *ceq = xch.lds();
+    static_assert(RC + NB * RB <= group_lds_doubles<RC>(), "every row's average fits the group's scratch");
     constexpr int NCP = NC / 2;                        // coefficient pairs of a central row
     constexpr int GPW = 64 / NV;
     // the tile of pseudo-inverses of this wavefront's cells
@@ -1560,13 +1564,14 @@ ZFV_HD void reconstruct_lane(const Img &m, int64_t i, const int g, X &xch, const
       const int64_t j = entry & ROW_CELL_MASK;
       const int code = entry >> ROW_CELL_BITS;
       if (PH == PH_LIGHT) {
+        mb.sphi = m.phi_unshifted ? 0.0 : m.shift_phi[code];
+        mb.cell = int32_t(j);
+        if (SERIES) return;  // (averages out of the series' range)
         // the member's potential values (cphi) in w3[k][0] and its
         // translation's potential, added where they are used (so that the
         // loads stay in flight until then)
         const double *cp = m.cphi + uint32_t(j) * uint32_t(DIM + 1);
         for (int k = 0; k < DIM + 1; ++k) mb.w3[k][0] = cp[k];
-        mb.sphi = m.phi_unshifted ? 0.0 : m.shift_phi[code];
-        mb.cell = int32_t(j);
         return;
       }
       mb.lin = PH == PH_LIN || (PH == PH_FULL && linear_isentropic(m) && code == 0) ? 1 : 0;
@@ -1587,13 +1592,6 @@ ZFV_HD void reconstruct_lane(const Img &m, int64_t i, const int g, X &xch, const
       } else if (PH == PH_LIGHT) {
         double w3[DIM + 1][3];
         if (SERIES) {
-          if (series) {
-            // th0 exp(a (mean - phi_ref)) times the average about the mean
-            const double z = (mb.w3[0][0] + (mb.sphi - thc.phi_ref)) * thc.a;
-            er = thc.th0 * (exp_near(z) * exp_average(m, aa * mb.w3[1][0], aa * thc.a * mb.w3[2][0]));
-            eE = er * thc.b;
-            return;
-          }
           // out of the series' range: the rule's points one by one
           load_corners<DIM>(m, mb.cell, w3);
           for (int k = 0; k < DIM + 1; ++k) w3[k][0] = axial_phi<DIM>(m, w3[k]) + (mb.sphi - thc.phi_ref);
@@ -1629,7 +1627,30 @@ ZFV_HD void reconstruct_lane(const Img &m, int64_t i, const int g, X &xch, const
     Member mb{};
     int tw = -1;
     load_P(0, pr);
-    if (wb) load_member(rw[0], mb);
+    if (series) {
+      // In series form all rows' averages come first: the chains of the
+      // chunks are independent, so one lane's chunks overlap, and the members'
+      // data are loaded together.
+      double z[NCH], p2[NCH], p3[NCH];
+#pragma unroll
+      for (int ch = 0; ch < NCH; ++ch) {
+        const int32_t j = rw[ch] & ROW_CELL_MASK;
+        const double *cp = m.cphi + uint32_t(j) * 3u;
+        z[ch] = cp[0];
+        p2[ch] = cp[1];
+        p3[ch] = cp[2];
+        if (!m.phi_unshifted) z[ch] += m.shift_phi[rw[ch] >> ROW_CELL_BITS];
+      }
+#pragma unroll
+      for (int ch = 0; ch < NCH; ++ch) {
+        // th0 exp(a (mean - phi_ref)) times the average about the mean
+        const double er = thc.th0 * (exp_near((z[ch] - thc.phi_ref) * thc.a) *
+                                     exp_average(m, aa * p2[ch], aa * thc.a * p3[ch]));
+        if (g < chunk_rows(ch)) ceq[chunk_row0(ch) + g] = er;
+      }
+    } else if (wb) {
+      load_member(rw[0], mb);
+    }
 #pragma unroll
     for (int ch = 0; ch < NCH; ++ch) {
       const int cnt = chunk_rows(ch);
@@ -1645,22 +1666,28 @@ ZFV_HD void reconstruct_lane(const Img &m, int64_t i, const int g, X &xch, const
         load_P(ch + 1, pr);
         gather(ch + 1, uk);
         tw = twin_of(ch + 1);
-        if (wb && tw < 0) load_member(rw[ch + 1], mb);
+        if (wb && !series && tw < 0) load_member(rw[ch + 1], mb);
       }
-      if (wb) {
+      if (wb && !series) {
         double er = 0.0, eE = 0.0;
-        if (tc >= 0) {
-          er = ceq[2 * tc];
-          eE = ceq[2 * tc + 1];
+        if (PH == PH_LIGHT) {
+          if (tc >= 0) er = ceq[tc];
+          else member_avg_of(mc, er, eE);
+          if (g < cnt) ceq[chunk_row0(ch) + g] = er;
         } else {
-          member_avg_of(mc, er, eE);
+          if (tc >= 0) {
+            er = ceq[2 * tc];
+            eE = ceq[2 * tc + 1];
+          } else {
+            member_avg_of(mc, er, eE);
+          }
+          if (PH != PH_LIN && ch < CCH && g < cnt) {
+            ceq[2 * (ch * NV + g)] = er;
+            ceq[2 * (ch * NV + g) + 1] = eE;
+          }
+          pl[g * ROWW + NC] = er;
+          pl[g * ROWW + NC + 1] = eE;
         }
-        if (PH != PH_LIN && !series && ch < CCH && g < cnt) {
-          ceq[2 * (ch * NV + g)] = er;
-          ceq[2 * (ch * NV + g) + 1] = eE;
-        }
-        pl[g * ROWW + NC] = er;
-        if (PH != PH_LIGHT) pl[g * ROWW + NC + 1] = eE;
       }
       xch.sync();
 #pragma unroll
@@ -1669,7 +1696,7 @@ ZFV_HD void reconstruct_lane(const Img &m, int64_t i, const int g, X &xch, const
         const double *row = pl + k * ROWW;
         double er = 0.0, eE = 0.0;
         if (wb) {
-          er = row[NC];
+          er = PH == PH_LIGHT ? ceq[chunk_row0(ch) + k] : row[NC];
           if (PH != PH_LIGHT) eE = row[NC + 1];
         }
         const double d = deviation(uc[k], er, eE);
