@@ -141,6 +141,8 @@ int zfv_set_steady_state(zfv_handle *h, const double *cvars);
  * FluxLoop + GravitySourceLoop + FluxBC, in that order
  * (src/zisa/ode/rate_of_change.cpp:21-27). */
 int zfv_rate(zfv_handle *h, const double *u, double *dudt, double t);
+/* The same from dudt = 0, whatever dudt holds. */
+int zfv_rate_set(zfv_handle *h, const double *u, double *dudt, double t);
 
 /* TimeIntegration::compute_step for SSP3 on the device-resident state, with the
  * frozen BC after every stage sum (src/zisa/ode/runge_kutta.cpp:87-112). */

@@ -201,6 +201,7 @@ def load_library(path: str = LIB_PATH):
         "zfv_get_state": (c_int, [vp, dp]),
         "zfv_set_steady_state": (c_int, [vp, dp]),
         "zfv_rate": (c_int, [vp, dp, dp, c_double]),
+        "zfv_rate_set": (c_int, [vp, dp, dp, c_double]),
         "zfv_step": (c_int, [vp, c_double, c_double]),
         "zfv_steps": (c_int, [vp, ctypes.c_int32, c_double, c_double]),
         "zfv_cfl_dt": (c_int, [vp, c_double, dp]),
@@ -363,7 +364,7 @@ class Solver:
         _check(self.lib.zfv_set_state(self.h, _dp(u)))
 
     def get_state(self) -> np.ndarray:
-        u = np.zeros((self.n_cells, 5))
+        u = np.empty((self.n_cells, 5))
         _check(self.lib.zfv_get_state(self.h, _dp(u)))
         return u
 
@@ -374,7 +375,7 @@ class Solver:
 
     def snapshot_end(self) -> np.ndarray:
         """The state at the last snapshot_begin (zfv_snapshot_end)."""
-        u = np.zeros((self.n_cells, 5))
+        u = np.empty((self.n_cells, 5))
         _check(self.lib.zfv_snapshot_end(self.h, _dp(u)))
         return u
 
@@ -385,7 +386,11 @@ class Solver:
     def rate(self, u: np.ndarray, t: float = 0.0, dudt: Optional[np.ndarray] = None) -> np.ndarray:
         """RateOfChange::compute: returns dudt + L(u) (dudt defaults to zeros)."""
         u = np.ascontiguousarray(u, dtype=np.float64)
-        out = np.zeros_like(u) if dudt is None else np.ascontiguousarray(dudt, dtype=np.float64)
+        if dudt is None and u.size == 5 * self.n_cells:
+            out = np.empty(u.shape)  # (every entry is set)
+            _check(self.lib.zfv_rate_set(self.h, _dp(u), _dp(out), t))
+            return out
+        out = np.zeros(u.shape) if dudt is None else np.ascontiguousarray(dudt, dtype=np.float64)
         _check(self.lib.zfv_rate(self.h, _dp(u), _dp(out), t))
         return out
 

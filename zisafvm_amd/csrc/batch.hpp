@@ -70,13 +70,18 @@ constexpr int groups_per_wave() {
 // (a multiple of 8, at least 8) as the instances need; the kernels are
 // launched with exactly that many blocks.  Returns an empty table when it
 // would exceed cap entries.
+inline int64_t block_table_size(const std::vector<int64_t> &counts, int64_t per_block) {
+  int64_t blocks = 0;
+  for (int64_t c : counts) blocks += (c + per_block - 1) / per_block;
+  return std::max<int64_t>(8, ((blocks + 7) / 8) * 8);
+}
 inline std::vector<BlockRef> block_table(const std::vector<int64_t> &counts, int64_t per_block, int64_t cap,
                                          bool xcd_chunks) {
+  const int64_t size = block_table_size(counts, per_block);
+  if (size > cap) return {};
   std::vector<BlockRef> logical;
   for (size_t s = 0; s < counts.size(); ++s)
     for (int64_t k = 0; k < (counts[s] + per_block - 1) / per_block; ++k) logical.push_back({int(s), int(k)});
-  const int64_t size = std::max<int64_t>(8, ((int64_t(logical.size()) + 7) / 8) * 8);
-  if (size > cap) return {};
   std::vector<BlockRef> t(size, BlockRef{-1, 0});
   if (!xcd_chunks) {
     std::copy(logical.begin(), logical.end(), t.begin());

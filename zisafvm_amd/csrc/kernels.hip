@@ -1277,6 +1277,25 @@ int create_device(zfv_handle *h) {
   ZFV_API_END
 }
 
+// L(u) of host buffers, into dudt
+static void rate_of_change(zfv_handle *h, const double *u, double *dudt, Into into) {
+  member_settle(h);
+  const int64_t n = h->img.n;
+  const int nv = h->img.s.nvars;
+  to_cells(h->img, u, h->host_stage);
+  HIP_CHECK(hipMemcpyAsync(h->X, h->host_stage, sizeof(double) * nv * n, hipMemcpyHostToDevice, h->stream));
+  const Img &m = h->dimg;
+  h->L.rec[h->ph](m, h->X, h->fpv, h->src, rec_config(h, h->X), 0, h->stream);
+  StageCoeffs sc{};
+  sc.write_rate_only = 1;
+  h->L.update(m, UpdateArgs{sc, 0, 0.0, h->X, h->fpv, h->src, h->X, h->K, h->X}, h->stream);
+  HIP_CHECK(hipGetLastError());
+  HIP_CHECK(hipMemcpyAsync(h->host_stage, h->K, sizeof(double) * nv * n, hipMemcpyDeviceToHost, h->stream));
+  map_pages(dudt, 5 * size_t(n));
+  HIP_CHECK(hipStreamSynchronize(h->stream));
+  from_cells(h->img, h->host_stage, dudt, into);
+}
+
 }  // namespace zfv
 
 extern "C" {
@@ -1312,8 +1331,9 @@ int zfv_get_state(zfv_handle *h, double *cvars) {
   member_settle(h);
   const size_t bytes = sizeof(double) * h->img.s.nvars * h->img.n;
   HIP_CHECK(hipMemcpyAsync(h->host_stage, h->U, bytes, hipMemcpyDeviceToHost, h->stream));
+  map_pages(cvars, 5 * size_t(h->img.n));
   HIP_CHECK(hipStreamSynchronize(h->stream));
-  from_cells(h->img, h->host_stage, cvars, false);
+  from_cells(h->img, h->host_stage, cvars, Into::Set);
   return ZFV_OK;
   ZFV_API_END
 }
@@ -1347,8 +1367,9 @@ int zfv_snapshot_end(zfv_handle *h, double *cvars) {
   ZFV_API_BEGIN
   if (!h->snap_pending) throw ZfvError(ZFV_ERR_INVALID, "no snapshot pending");
   h->snap_pending = false;
+  map_pages(cvars, 5 * size_t(h->img.n));
   HIP_CHECK(hipStreamSynchronize(h->copy_stream));
-  from_cells(h->img, h->snap_host, cvars, false);
+  from_cells(h->img, h->snap_host, cvars, Into::Set);
   return ZFV_OK;
   ZFV_API_END
 }
@@ -1372,20 +1393,15 @@ int zfv_set_steady_state(zfv_handle *h, const double *cvars) {
 int zfv_rate(zfv_handle *h, const double *u, double *dudt, double t) {
   (void)t;
   ZFV_API_BEGIN
-  member_settle(h);
-  const int64_t n = h->img.n;
-  const int nv = h->img.s.nvars;
-  to_cells(h->img, u, h->host_stage);
-  HIP_CHECK(hipMemcpyAsync(h->X, h->host_stage, sizeof(double) * nv * n, hipMemcpyHostToDevice, h->stream));
-  const Img &m = h->dimg;
-  h->L.rec[h->ph](m, h->X, h->fpv, h->src, rec_config(h, h->X), 0, h->stream);
-  StageCoeffs sc{};
-  sc.write_rate_only = 1;
-  h->L.update(m, UpdateArgs{sc, 0, 0.0, h->X, h->fpv, h->src, h->X, h->K, h->X}, h->stream);
-  HIP_CHECK(hipGetLastError());
-  HIP_CHECK(hipMemcpyAsync(h->host_stage, h->K, sizeof(double) * nv * n, hipMemcpyDeviceToHost, h->stream));
-  HIP_CHECK(hipStreamSynchronize(h->stream));
-  from_cells(h->img, h->host_stage, dudt, true);
+  zfv::rate_of_change(h, u, dudt, Into::Add);
+  return ZFV_OK;
+  ZFV_API_END
+}
+
+int zfv_rate_set(zfv_handle *h, const double *u, double *dudt, double t) {
+  (void)t;
+  ZFV_API_BEGIN
+  zfv::rate_of_change(h, u, dudt, Into::FromZero);
   return ZFV_OK;
   ZFV_API_END
 }
@@ -1779,6 +1795,10 @@ static std::vector<BlockRef> checked_table(const std::vector<int64_t> &counts, i
   return t;
 }
 
+static int batch_rec_waves(const zfv_batch *b) {
+  return rec_cfg_waves(b->rec_cfg >= 0 ? b->rec_cfg : kRecConfigs - 1);
+}
+
 // waits for the batch's stream (and so for steps in flight) and refreshes
 // the host copy of the members' loop state
 static void batch_sync_down(zfv_batch *b) {
@@ -1799,7 +1819,8 @@ static void member_settle(zfv_handle *h) {
   h->batch->cfl_ready = false;
 }
 
-static void batch_upload(zfv_batch *b) {
+// the members' cells, by slot; ZFV_ERR_MEMORY if their blocks exceed the capacity
+static std::vector<int64_t> batch_cells(const zfv_batch *b) {
   std::vector<int64_t> cells(b->max_inst, 0);
   int64_t face_blocks = 0;
   for (int s = 0; s < b->max_inst; ++s)
@@ -1807,7 +1828,27 @@ static void batch_upload(zfv_batch *b) {
       cells[s] = b->h_inst[s].m.n;
       face_blocks += (b->h_inst[s].m.ne + 255) / 256;
     }
-  if (face_blocks > b->cap_face_blocks) throw ZfvError(ZFV_ERR_MEMORY, "batch capacity exceeded");
+  auto fits = [&](int64_t per_block, int64_t cap) { return block_table_size(cells, per_block) <= cap; };
+  if (face_blocks > b->cap_face_blocks || !fits(256, b->cap_cell_blocks) ||
+      !fits(update_cells_of_block(b->shape.dim), b->cap_upd_blocks) ||
+      !fits(int64_t(batch_rec_waves(b)) * b->L.groups_per_wave, b->cap_rec_blocks))
+    throw ZfvError(ZFV_ERR_MEMORY, "batch capacity exceeded");
+  return cells;
+}
+
+// Members have changed: the device's tables are stale until the next launch,
+// which uploads them once for all the changes since the last (a round of eight
+// requests that join, run and leave: 16 uploads of 50 us become one, and the
+// step graph is captured again only if a launch's sizes differ from the last
+// launch's).  What does not fit is refused here.
+static void batch_changed(zfv_batch *b) {
+  b->dirty = true;
+  b->cfl_ready = false;
+  (void)batch_cells(b);
+}
+
+static void batch_upload(zfv_batch *b) {
+  const std::vector<int64_t> cells = batch_cells(b);
   int ph = -1;
   for (int s = 0; s < b->max_inst; ++s)
     if (b->members[s] && b->h_inst[s].active) {
@@ -1822,8 +1863,7 @@ static void batch_upload(zfv_batch *b) {
   b->ph = ph;
   auto tc = checked_table(cells, 256, b->cap_cell_blocks, b->xcd_chunks);
   auto tu = checked_table(cells, update_cells_of_block(b->shape.dim), b->cap_upd_blocks, b->xcd_chunks);
-  const int waves = rec_cfg_waves(b->rec_cfg >= 0 ? b->rec_cfg : kRecConfigs - 1);
-  auto tr = checked_table(cells, int64_t(waves) * b->L.groups_per_wave, b->cap_rec_blocks, b->xcd_chunks);
+  auto tr = checked_table(cells, int64_t(batch_rec_waves(b)) * b->L.groups_per_wave, b->cap_rec_blocks, b->xcd_chunks);
   if (int64_t(tc.size()) != b->n_cell_blocks || int64_t(tu.size()) != b->n_upd_blocks ||
       int64_t(tr.size()) != b->n_rec_blocks) {
     // launch sizes change: the step graph is captured again on the next run
@@ -1918,20 +1958,20 @@ static void batch_enqueue_cfl(zfv_batch *b) {
 }
 
 static void batch_forget(zfv_batch *b, int slot) {
-  batch_sync_down(b);
+  if (b->in_flight) batch_sync_down(b);
   if (b->members[slot]) {
     b->members[slot]->batch = nullptr;
     b->members[slot]->batch_slot = -1;
   }
   b->members[slot] = nullptr;
   b->h_inst[slot].active = 0;
-  batch_upload(b);
+  batch_changed(b);
 }
 
 static void batch_member_steady(zfv_batch *b, int slot, const double *steady) {
-  batch_sync_down(b);
+  if (b->in_flight) batch_sync_down(b);
   b->h_inst[slot].m.steady = steady;
-  batch_upload(b);
+  batch_changed(b);
 }
 
 static void batch_after_snapshot(zfv_batch *b, hipEvent_t copied) {
@@ -1982,9 +2022,9 @@ int zfv_batch_destroy(zfv_batch *b) {
 
 int zfv_batch_set_xcd_chunks(zfv_batch *b, int32_t on) {
   ZFV_API_BEGIN
-  batch_sync_down(b);
+  if (b->in_flight) batch_sync_down(b);
   b->xcd_chunks = on != 0;
-  batch_upload(b);
+  batch_changed(b);
   return ZFV_OK;
   ZFV_API_END
 }
@@ -1994,7 +2034,7 @@ int zfv_batch_add(zfv_batch *b, zfv_handle *h, double cfl, double t0, double t_e
   ZFV_API_BEGIN
   if (!same_shape(b->shape, h->img.s)) throw ZfvError(ZFV_ERR_INVALID, "instance shape differs from the batch's");
   if (h->batch) throw ZfvError(ZFV_ERR_INVALID, "the instance is already a member of a batch");
-  batch_sync_down(b);
+  if (b->in_flight) batch_sync_down(b);
   int s = -1;
   for (int k = 0; k < b->max_inst; ++k)
     if (!b->members[k]) {
@@ -2020,11 +2060,11 @@ int zfv_batch_add(zfv_batch *b, zfv_handle *h, double cfl, double t0, double t_e
   b->h_inst[s] = d;
   b->members[s] = h;
   try {
-    batch_upload(b);
+    batch_changed(b);
   } catch (...) {
     b->members[s] = nullptr;
     b->h_inst[s].active = 0;
-    batch_upload(b);
+    batch_changed(b);
     throw;
   }
   h->batch = b;

@@ -16,6 +16,8 @@
 #include "setup.hpp"
 #include "stage_math.hpp"
 
+#include <sys/mman.h>
+
 #include <algorithm>
 #include <array>
 #include <cmath>
@@ -1254,7 +1256,7 @@ void to_cells_dim(const HostImage &img, const double *aos, double *cells) {
   }
 }
 
-template <int DIM, bool ACCUMULATE>
+template <int DIM, Into INTO>
 void from_cells_dim(const HostImage &img, const double *cells, double *aos) {
   constexpr int NV = DIM + 2;
   const int64_t n = img.n;
@@ -1266,21 +1268,37 @@ void from_cells_dim(const HostImage &img, const double *cells, double *aos) {
     const double *c = cells + NV * ip;
     double w[5] = {c[0], 0.0, 0.0, 0.0, c[NV - 1]};
     for (int d = 0; d < DIM; ++d) w[1 + d] = c[1 + d];
-    for (int v = 0; v < 5; ++v) u[v] = ACCUMULATE ? u[v] + w[v] : w[v];
+    for (int v = 0; v < 5; ++v) u[v] = INTO == Into::Set ? w[v] : (INTO == Into::Add ? u[v] : 0.0) + w[v];
   }
 }
+
+template <int DIM>
+void from_cells_into(const HostImage &img, const double *cells, double *aos, Into into) {
+  if (into == Into::Set) from_cells_dim<DIM, Into::Set>(img, cells, aos);
+  else if (into == Into::Add) from_cells_dim<DIM, Into::Add>(img, cells, aos);
+  else from_cells_dim<DIM, Into::FromZero>(img, cells, aos);
+}
 }  // namespace
+
+void map_pages(double *out, size_t n) {
+  constexpr uintptr_t kPage = 4096;
+  const uintptr_t a = reinterpret_cast<uintptr_t>(out) & ~(kPage - 1);
+  const uintptr_t e = (reinterpret_cast<uintptr_t>(out + n) + kPage - 1) & ~(kPage - 1);
+  if (e - a < 32 * kPage) return;
+#if defined(MADV_POPULATE_WRITE)
+  // (an older system refuses it: the pages are then mapped as they are written)
+  (void)madvise(reinterpret_cast<void *>(a), e - a, MADV_POPULATE_WRITE);
+#endif
+}
 
 void to_cells(const HostImage &img, const double *aos, double *cells) {
   if (img.s.dim == 2) to_cells_dim<2>(img, aos, cells);
   else to_cells_dim<3>(img, aos, cells);
 }
 
-void from_cells(const HostImage &img, const double *cells, double *aos, bool accumulate) {
-  if (img.s.dim == 2 && accumulate) from_cells_dim<2, true>(img, cells, aos);
-  else if (img.s.dim == 2) from_cells_dim<2, false>(img, cells, aos);
-  else if (accumulate) from_cells_dim<3, true>(img, cells, aos);
-  else from_cells_dim<3, false>(img, cells, aos);
+void from_cells(const HostImage &img, const double *cells, double *aos, Into into) {
+  if (img.s.dim == 2) from_cells_into<2>(img, cells, aos, into);
+  else from_cells_into<3>(img, cells, aos, into);
 }
 
 }  // namespace zfv
