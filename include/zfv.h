@@ -175,14 +175,15 @@ int zfv_advance(zfv_handle *h, double cfl_number, double t0, double t_end, int32
  * results) for callers that cannot allocate: code that must not call
  * hipMalloc or instantiate graphs (inside a capture, tight serving loops,
  * harnesses that forbid allocation).  No counterpart in the reference.  It
- * allocates nothing: the loop state and, with step rejection, the backup of
- * the state live in a file-scope device array of 16 MiB that each GPU the
- * library runs on holds from module load until the process ends; steps are
- * launched one by one (no graph) with the handle's tuned launch configuration
+ * allocates nothing: the loop state lives in a file-scope device array of 16
+ * MiB that each GPU the library runs on holds from module load until the
+ * process ends; steps are launched one by one (no graph) with the handle's
+ * tuned launch configuration
  * (one wavefront per block if it was never tuned).  Limit: with step
  * rejection (drho_crit_rel > 0) the state must fit 16 MiB - 256 B
  * (nvars * n_cells * 8 bytes: 524,280 triangles or 419,424 tetrahedra),
- * else ZFV_ERR_MEMORY.  The handle's device must be current.  Calls on one
+ * else ZFV_ERR_MEMORY (callers rely on the limit; the steps themselves keep no
+ * copy of the state).  The handle's device must be current.  Calls on one
  * GPU share the array: calls that overlap on one GPU (from several host
  * threads) race and must not be issued. */
 int zfv_advance_noalloc(zfv_handle *h, double cfl_number, double t0, double t_end, int32_t max_steps,
@@ -197,7 +198,7 @@ int zfv_synchronize(zfv_handle *h);
 
 typedef struct zfv_info {
   int64_t n_cells;
-  int64_t n_faces;            /* interior faces evaluated by the face kernel */
+  int64_t n_faces;            /* interior faces */
   int64_t device_bytes;       /* HBM held by the handle */
   double bytes_per_cell_stage;/* algorithmic bytes, all kernels of one stage */
   double recon_bytes_per_cell;/* algorithmic bytes of the reconstruction kernel */
@@ -219,7 +220,8 @@ int zfv_get_stencils(zfv_handle *h, int32_t i, int32_t *l2g, int32_t cap, int32_
 
 /* Runs n_steps SSP3 steps of fixed dt launch by launch (the state advances)
  * with HIP events on the handle's stream around every kernel; returns the
- * milliseconds summed over the launches of each kernel. */
+ * milliseconds summed over the launches of each kernel.  The face fluxes are
+ * formed by the update (face_flux_ms is 0). */
 typedef struct zfv_kernel_times {
   double reconstruct_ms, face_flux_ms, update_ms;
   int32_t n_launches;

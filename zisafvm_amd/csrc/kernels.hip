@@ -11,7 +11,8 @@
 //                  face's area; then one lane per cell and variable: the sum
 //                  of the cell's fluxes, source, flux BC, Butcher-form stage
 //                  sum, frozen BC
-// FP64 throughout; no MFMA (the per-cell mat-vecs are memory-bound).
+// FP64 throughout; no MFMA (every cell has its own matrices: there is no shared
+// operand for a tile, and the matrices' bytes bound the kernel).
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -104,8 +105,8 @@ struct QuadGroup : WaveGroup {
 };
 
 // Wavefronts per SIMD the reconstruction is compiled for: three leave 168
-// registers, which hold the next chunk's data in flight.  (Four in 2D order 4
-// spill 56 bytes: 20 steps of 263,520 triangles take 13.1 instead of 12.3 ms.)
+// registers, which hold the next chunk's data in flight.  (Four in 2D spill 12
+// bytes at order 4: 20 steps of 263,520 triangles take 11.10 instead of 11.04 ms.)
 constexpr int rec_min_waves(int ph) { return ph == PH_FULL ? 1 : 3; }
 
 // k_reconstruct: blocks of `blockDim.x / 64` waves, 64 / NV cells per wave
@@ -209,11 +210,6 @@ __device__ __forceinline__ void adv_end(AdvState *a) {
   if (a->t >= a->t_end || a->steps >= a->max_steps) a->active = 0;
 }
 
-// What a stage's update reads and writes: K[stage] = L(Ustage); Unext = U0 +
-// dt * sum_j c_j K[j] (src/zisa/ode/runge_kutta.cpp:122-143), then FrozenBC for
-// ghost cells.  Ustage, U0 and Unext may name the same buffer (stages 1 and 2
-// read and write the stage state X; a wavefront reads only its own cells'
-// entries, before it writes them), so none of them is declared __restrict__.
 // What the last stage's update also does in a time loop that chooses its steps:
 // the new state's CFL minimum goes to cfl[slot] (null: not wanted), a density
 // change of more than crit times its old value in any cell sets *bad (crit 0:
@@ -223,6 +219,12 @@ struct UpdateChecks {
   double crit;
   int *bad;
 };
+
+// What a stage's update reads and writes: K[stage] = L(Ustage); Unext = U0 +
+// dt * sum_j c_j K[j] (src/zisa/ode/runge_kutta.cpp:122-143), then FrozenBC for
+// ghost cells.  Ustage, U0 and Unext may name the same buffer (stages 1 and 2
+// read and write the stage state X; a wavefront reads only its own cells'
+// entries, before it writes them), so none of them is declared __restrict__.
 struct UpdateArgs {
   StageCoeffs sc;
   int stage;
@@ -1011,10 +1013,12 @@ static void check_advance_args(double cfl_number, double drho_crit_rel, int32_t 
 
 // ---------------------------------------------------------------------------
 // Scratch of the allocation-free device time loop (zfv_advance_noalloc): the
-// loop state (one AdvState) in the first kNoAllocStateBytes, then the backup
-// of u0 that step rejection restores from.  A file-scope device array: each
-// GPU the library runs on holds its own copy from module load until the
-// process ends, and every call on that GPU shares it.
+// loop state (one AdvState) in the first kNoAllocStateBytes, then the CFL words.
+// (A step that is rejected leaves the state alone, so nothing is backed up; the
+// size, and the limit on states with rejection that follows from it, are the
+// entry point's.)  A file-scope device array: each GPU the library runs on holds
+// its own copy from module load until the process ends, and every call on that
+// GPU shares it.
 constexpr size_t kNoAllocScratchBytes = size_t(16) << 20;
 constexpr size_t kNoAllocStateBytes = 256;
 static_assert(sizeof(AdvState) <= kNoAllocStateBytes, "loop state larger than its scratch slot");
