@@ -1195,12 +1195,17 @@ ZFV_HD void reconstruct_lane(const Img &m, int64_t i, const int g, X &xch, const
   bool eq_found = false;
   double y_p2 = 0.0, y_p3 = 0.0;  // the cell's own power sums (SERIES)
   if (wb) {
-    // the potential the equilibrium is written against: the first volume
-    // point's, in the 2D light set the corners' mean
-    if (SERIES) {
+    // The potential the equilibrium is written against: the corners' mean for
+    // the 2D instances that run in the light set by themselves, else the first
+    // volume point's.  (A property of the instance, not of the set it runs in: a
+    // kept theta is read by another set when a member of another kind joins or
+    // leaves its batch.)
+    if (SERIES || (DIM == 2 && PH == PH_FULL && m.cphi != nullptr)) {
       phi_ref = m.cphi[3 * i];
-      y_p2 = m.cphi[3 * i + 1];
-      y_p3 = m.cphi[3 * i + 2];
+      if (SERIES) {
+        y_p2 = m.cphi[3 * i + 1];
+        y_p3 = m.cphi[3 * i + 2];
+      }
     } else {
       double xref[3], vtx[DIM + 1][3];
       load_corners<DIM>(m, i, vtx);
