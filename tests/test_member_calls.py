@@ -1,0 +1,60 @@
+"""Calls on a member of a batch wait for the batch's steps in flight, and a
+call that changes the member's state makes the next batched step reduce the CFL
+minimum anew (zfv_time_kernels advances the state)."""
+import numpy as np
+import pytest
+
+import zisafvm_amd as z
+from zisafvm_amd import workloads as W
+
+pytestmark = pytest.mark.gpu
+
+
+def _members():
+    wls = [W.vortex_2d(n=13), W.isothermal_2d(n=11, amplitude=1e-3, order=3)]
+    solvers = []
+    for w in wls:
+        s = z.Solver(w.mesh, w.params)
+        s.set_state(w.u0)
+        if w.steady is not None:
+            s.set_steady_state(w.steady)
+        solvers.append(s)
+    b = z.Batch(wls[0].params, sum(w.mesh.n_cells for w in wls), 4000, 2)
+    for w, s in zip(wls, solvers):
+        b.add(s, w.cfl, 0.0, 1.0)
+    return wls, solvers, b
+
+
+def _alone(wl, u, steps):
+    s = z.Solver(wl.mesh, wl.params)
+    s.set_state(u)
+    if wl.steady is not None:
+        s.set_steady_state(wl.steady)
+    for _ in range(steps):
+        s.step(0.0, s.cfl_dt(wl.cfl))
+    return s
+
+
+@pytest.mark.parametrize("launched", [False, True])
+def test_time_kernels_between_launches(gpu, launched):
+    wls, solvers, b = _members()
+    (b.launch if launched else b.run)(2)
+    for w, s in zip(wls, solvers):
+        s.time_kernels(3, 0.3 * _alone(w, w.u0, 0).cfl_dt(w.cfl))  # three steps of its own
+    after = [s.get_state() for s in solvers]
+    b.run(2)
+    for w, s, u in zip(wls, solvers, after):
+        np.testing.assert_array_equal(s.get_state(), _alone(w, u, 2).get_state())
+
+
+def test_cfl_dt_and_tune_wait_for_steps_in_flight(gpu):
+    wls, solvers, b = _members()
+    b.launch(5)
+    for w, s in zip(wls, solvers):
+        assert s.cfl_dt(w.cfl) == _alone(w, w.u0, 5).cfl_dt(w.cfl)
+    b.launch(5)
+    solvers[0].tune(0)
+    b.launch(5)
+    solvers[1].synchronize()
+    for w, s in zip(wls, solvers):
+        np.testing.assert_array_equal(s.get_state(), _alone(w, w.u0, 15).get_state())

@@ -886,6 +886,7 @@ namespace zfv {
 static void batch_forget(zfv_batch *b, int slot);
 static void batch_member_steady(zfv_batch *b, int slot, const double *steady);
 static void batch_after_snapshot(zfv_batch *b, hipEvent_t copied);
+static void member_wait(zfv_handle *h);
 static void member_settle(zfv_handle *h);
 
 static int fail(const std::exception &e) {
@@ -1546,6 +1547,7 @@ int zfv_advance_noalloc(zfv_handle *h, double cfl_number, double t0, double t_en
 
 int zfv_cfl_dt(zfv_handle *h, double cfl_number, double *dt) {
   ZFV_API_BEGIN
+  member_wait(h);
   const double big = 1.0e300;
   unsigned long long bits;
   std::memcpy(&bits, &big, sizeof(bits));
@@ -1564,6 +1566,7 @@ int zfv_cfl_dt(zfv_handle *h, double cfl_number, double *dt) {
 
 int zfv_synchronize(zfv_handle *h) {
   ZFV_API_BEGIN
+  member_wait(h);
   HIP_CHECK(hipStreamSynchronize(h->stream));
   return ZFV_OK;
   ZFV_API_END
@@ -1611,6 +1614,7 @@ int zfv_get_info(zfv_handle *h, zfv_info *info) {
 
 int zfv_tune(zfv_handle *h, int32_t rec_threads, zfv_tuning *out) {
   ZFV_API_BEGIN
+  member_wait(h);
   if (rec_threads == 0) {
     tune_rec(h, h->U);
   } else if (rec_threads > 0) {
@@ -1639,6 +1643,7 @@ int zfv_get_stencils(zfv_handle *h, int32_t i, int32_t *l2g, int32_t cap, int32_
 
 int zfv_time_kernels(zfv_handle *h, int32_t n_steps, double dt, zfv_kernel_times *out) {
   ZFV_API_BEGIN
+  member_settle(h);
   const Img m = stateless(h->dimg);
   const int cfg = rec_config(h, h->U);
   std::vector<hipEvent_t> ev(2 * 6 * std::max(n_steps, 1));
@@ -1840,11 +1845,14 @@ static void batch_sync_down(zfv_batch *b) {
 }
 
 // a member's own calls wait for its batch's steps in flight
-// (and may change its state)
+static void member_wait(zfv_handle *h) {
+  if (h->batch && h->batch->in_flight) batch_sync_down(h->batch);
+}
+
+// ... and where they may change its state, the batch's CFL minima are stale
 static void member_settle(zfv_handle *h) {
-  if (!h->batch) return;
-  if (h->batch->in_flight) batch_sync_down(h->batch);
-  h->batch->cfl_ready = false;
+  member_wait(h);
+  if (h->batch) h->batch->cfl_ready = false;
 }
 
 // the members' cells, by slot; ZFV_ERR_MEMORY if their blocks exceed the capacity
