@@ -39,12 +39,17 @@ def _alone(wl, u, steps):
 def test_time_kernels_between_launches(gpu, launched):
     wls, solvers, b = _members()
     (b.launch if launched else b.run)(2)
-    for w, s in zip(wls, solvers):
-        s.time_kernels(3, 0.3 * _alone(w, w.u0, 0).cfl_dt(w.cfl))  # three steps of its own
-    after = [s.get_state() for s in solvers]
+    refs = [_alone(w, w.u0, 2) for w in wls]
+    for w, s, r in zip(wls, solvers, refs):
+        dt = 0.3 * r.cfl_dt(w.cfl)
+        s.time_kernels(3, dt)  # three steps of its own
+        r.time_kernels(3, dt)
+    # (nothing but the next launch asks for the members' states in between)
     b.run(2)
-    for w, s, u in zip(wls, solvers, after):
-        np.testing.assert_array_equal(s.get_state(), _alone(w, u, 2).get_state())
+    for w, s, r in zip(wls, solvers, refs):
+        for _ in range(2):
+            r.step(0.0, r.cfl_dt(w.cfl))
+        np.testing.assert_array_equal(s.get_state(), r.get_state())
 
 
 def test_cfl_dt_and_tune_wait_for_steps_in_flight(gpu):
