@@ -1,6 +1,7 @@
 """Calls on a member of a batch wait for the batch's steps in flight, and a
 call that changes the member's state makes the next batched step reduce the CFL
-minimum anew (zfv_time_kernels advances the state)."""
+minimum anew (zfv_time_kernels advances the state); what a member that stopped
+reports."""
 import numpy as np
 import pytest
 
@@ -63,3 +64,24 @@ def test_cfl_dt_and_tune_wait_for_steps_in_flight(gpu):
     solvers[1].synchronize()
     for w, s in zip(wls, solvers):
         np.testing.assert_array_equal(s.get_state(), _alone(w, w.u0, 15).get_state())
+
+
+def test_query_tells_a_stopped_member_from_a_finished_one(gpu):
+    wls, solvers, b = _members()
+    b.run(2)
+    before = [b.query(k) for k in (0, 1)]
+    assert all(q["active"] and q["dt"] > 0.0 for q in before)
+    bad = wls[0].u0.copy()
+    bad[5, 4] = -bad[5, 4]  # a negative pressure: no sound speed, no step
+    solvers[0].set_state(bad)
+    b.run(2)
+    q = b.query(0)
+    assert not q["active"] and not q["dt"] > 0.0 and q["steps"] == 2 and q["t"] == before[0]["t"]
+    assert b.query(1)["active"] and b.query(1)["steps"] == 4
+    # a finished member keeps its last step's dt
+    b.remove(0)
+    solvers[0].set_state(wls[0].u0)
+    slot = b.add(solvers[0], wls[0].cfl, 0.0, 1.0, 2)
+    b.run(4)
+    q = b.query(slot)
+    assert not q["active"] and q["steps"] == 2 and q["dt"] == before[0]["dt"]

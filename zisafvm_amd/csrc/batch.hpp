@@ -49,11 +49,13 @@ ZFV_HD double kb_step_dt(const DevInst &d) {
   return dt;
 }
 
-// the first stage's record of the step's dt
+// The first stage's record of the step's dt.  A member that stops because its
+// state gives no positive step is left with that dt, a finished one with its
+// last step's: callers tell the two ends apart by it (zfv_batch_query).
 ZFV_HD void kb_begin_instance(DevInst &d, double dt) {
   d.running = dt > 0.0;
-  if (d.running) d.dt = dt;
-  else d.active = 0;
+  if (!kb_finished(d)) d.dt = dt;
+  if (!d.running) d.active = 0;
 }
 
 // groups of NV lanes per 64-wide wavefront (2D: 16 cells, 3D: 12 cells)
