@@ -1,0 +1,74 @@
+"""Rounding errors of the kernels' math against 80-bit arithmetic: the rate of
+change evaluated in double precision on the library's own tables, and single
+formulas whose faster forms must lose no more than the plain ones."""
+import ctypes
+import os
+import subprocess
+
+import numpy as np
+import pytest
+
+import zisafvm_amd as z
+from zisafvm_amd import workloads as W
+from emu_binding import Emu
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+CSRC = os.path.join(os.path.dirname(HERE), "zisafvm_amd", "csrc")
+BUILD = os.path.join(HERE, "cpp", "build")
+
+
+def _library(name, *more):
+    os.makedirs(BUILD, exist_ok=True)
+    out = os.path.join(BUILD, name + ".so")
+    subprocess.run(["g++", "-O2", "-std=c++17", "-fPIC", "-fopenmp", "-ffp-contract=off", "-w", "-shared", "-o", out,
+                    os.path.join(HERE, "cpp", name + ".cpp")] + [os.path.join(CSRC, m) for m in more], check=True)
+    return ctypes.CDLL(out)
+
+
+@pytest.fixture(scope="module")
+def extended():
+    return _library("extended", "setup.cpp", "mesh.cpp")
+
+
+def _weno_rusanov(w):
+    w.params.reconstruction, w.params.flux = z.ZFV_WENO_AO, z.ZFV_FLUX_RUSANOV
+    return w
+
+
+# the root mean square error over the cells and variables, relative to each
+# variable's largest rate, that the plain formulas reach: a division per
+# quotient, the basis functions one by one
+CASES = {
+    "vortex_o3": (lambda s: W.vortex_2d(n=16, order=3, beta=3.0 + s, seed=s), 2.26e-15),
+    "vortex_o4": (lambda s: W.vortex_2d(n=16, order=4, beta=3.0 + s, seed=s), 2.28e-15),
+    "vortex_o3_weno_rusanov": (lambda s: _weno_rusanov(W.vortex_2d(n=16, order=3, beta=3.0 + s, seed=s)), 2.32e-15),
+}
+
+
+def _check(extended, make, name):
+    case, bound = CASES[name]
+    errs = []
+    for seed in (1, 2, 3, 4):
+        w = case(seed)
+        u = np.ascontiguousarray(w.u0)
+        ref = np.zeros(u.shape, dtype=np.longdouble)
+        mesh = w.mesh.c_struct()
+        assert extended.ext_rate(ctypes.byref(mesh), ctypes.byref(w.params), ctypes.c_void_p(u.ctypes.data),
+                                 ctypes.c_void_p(ref.ctypes.data)) == 0
+        got = make(w.mesh, w.params).rate(u)
+        keep = np.ix_(w.mesh.ghost == 0, [0, 1, 2, 4])
+        errs.append(float((((got - ref)[keep] / np.abs(ref[keep]).max(axis=0)) ** 2).mean()))
+    err = np.sqrt(np.mean(errs))
+    print(name, "rms", err, "bound", bound, flush=True)
+    assert err <= bound
+
+
+@pytest.mark.parametrize("name", sorted(CASES))
+def test_rate_rounds_no_worse_than_the_plain_formulas(extended, name):
+    _check(extended, Emu, name)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("name", sorted(CASES))
+def test_rate_on_the_device_rounds_no_worse_than_the_plain_formulas(gpu, extended, name):
+    _check(extended, z.Solver, name)

@@ -135,6 +135,11 @@ ZFV_HD double sqr(double x) { return x * x; }
 
 ZFV_HD double dmin(double a, double b) { return a < b ? a : b; }
 ZFV_HD double dmax(double a, double b) { return a > b ? a : b; }
+// a / b where r = 1 / b is at hand, to the last place of a division
+ZFV_HD double quotient(double a, double b, double r) {
+  const double q = a * r;
+  return fma(fma(-q, b, a), r, q);
+}
 
 // Where variable v of cell i stands in a state-shaped array (state, stage
 // state, tendencies, source, steady state).  The kernels keep the NV values of
@@ -1798,12 +1803,12 @@ ZFV_HD void reconstruct_lane(const Img &m, int64_t i, const int g, X &xch, const
       al_tot += alpha[k];
     }
     const double inv_tot = 1.0 / al_tot;
-    const double w0 = alpha[0] * inv_tot;
+    const double w0 = quotient(alpha[0], al_tot, inv_tot);
     a[0] = 0.0 + w0 * a0[0];
     for (int al = 1; al < DOFC; ++al) a[al] = 0.0 + w0 * c[al - 1];
 #pragma unroll
     for (int k = 0; k < NB; ++k) {
-      const double w = alpha[k + 1] * inv_tot;
+      const double w = quotient(alpha[k + 1], al_tot, inv_tot);
       a[0] = a[0] + w * a0[k + 1];
       for (int al = 1; al <= NBC; ++al) a[al] = a[al] + w * b[k][al - 1];
     }
@@ -1820,9 +1825,12 @@ ZFV_HD void reconstruct_lane(const Img &m, int64_t i, const int g, X &xch, const
 
   // The deviation of this variable, sum_alpha a_alpha (X^alpha - c_alpha): the
   // variable's scale goes into the coefficients and the moments into the
-  // constant one, so that a point costs one nested evaluation.
+  // constant one, so that a point costs one nested evaluation.  The mean (the
+  // coefficient of the basis function 1) is added last: the rest is a difference
+  // from it, small where the state varies little, and keeps its own last places.
   for (int al = 0; al < DOFC; ++al) a[al] = scale_g * a[al];
-  const double mean = a[0];  // the coefficient of the basis function 1
+  const double mean = a[0];
+  a[0] = 0.0;
   for (int al = 3; al < DOFC; ++al) a[0] = fma(-a[al], cm[al], a[0]);
 
   double s_acc = 0.0;
@@ -1936,7 +1944,7 @@ ZFV_HD void reconstruct_lane(const Img &m, int64_t i, const int g, X &xch, const
     for (int q = 0; q < Q; ++q) {
       double Xs[3];
       face_point<DIM>(m, q, w3, Xs);
-      u[q] = poly_nested<DIM, DEGC>(a, Xs);
+      u[q] = mean + poly_nested<DIM, DEGC>(a, Xs);
       if (wb) {
         u[q] = fma(eq_rho, eqr[q], fma(eq_E, eqE[q], u[q]));
         fs = fma(m.fw[q], eqE[q], fs);
@@ -1983,7 +1991,7 @@ ZFV_HD void reconstruct_lane(const Img &m, int64_t i, const int g, X &xch, const
         double x[3], Xs[3] = {0.0, 0.0, 0.0};
         volume_point<DIM>(m, q, vtx, x);
         for (int d = 0; d < DIM; ++d) Xs[d] = (x[d] - xc[d]) * inv_len;
-        const double dl = poly_nested<DIM, DEGC>(a, Xs);
+        const double dl = mean + poly_nested<DIM, DEGC>(a, Xs);
         double gp[3];
         grad_phi<DIM, PH>(m, x, gp);
         const double w = vol_i * m.vw[q];
@@ -2005,7 +2013,7 @@ ZFV_HD void reconstruct_lane(const Img &m, int64_t i, const int g, X &xch, const
           sm[2 * k + 1] = v.hi;
         }
       }
-      // (a[0] holds the constant of the nested form; the basis's is mean)
+      // (a[0] holds the nested form's moments; the basis function 1 has mean)
 #pragma unroll
       for (int al = 0; al < DOFC; ++al)
 #pragma unroll
