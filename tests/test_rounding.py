@@ -72,3 +72,22 @@ def test_rate_rounds_no_worse_than_the_plain_formulas(extended, name):
 @pytest.mark.parametrize("name", sorted(CASES))
 def test_rate_on_the_device_rounds_no_worse_than_the_plain_formulas(gpu, extended, name):
     _check(extended, z.Solver, name)
+
+
+def _ptr(a):
+    return ctypes.c_void_p(a.ctypes.data)
+
+
+def test_hllc_of_a_state_at_rest_is_its_pressure():
+    # no mass or energy crosses the face, exactly; the pressure to a few places
+    lib = _library("rounding")
+    rng = np.random.default_rng(3)
+    n, gamma = 20000, 1.4
+    p = np.exp(rng.uniform(-3.0, 3.0, n))
+    u = np.stack([np.exp(rng.uniform(-3.0, 3.0, n)), np.zeros(n), np.zeros(n), p / (gamma - 1.0)], axis=1)
+    a = rng.uniform(0.0, 2.0 * np.pi, n)
+    nn = np.stack([np.cos(a), np.sin(a)], axis=1)
+    f = np.empty((n, 4))
+    lib.unit_hllc(ctypes.c_double(gamma), n, _ptr(u), _ptr(u), _ptr(nn), _ptr(f))
+    assert not f[:, 0].any() and not f[:, 3].any()
+    assert (np.abs(f[:, 1:3] - p[:, None] * nn) <= 4 * np.finfo(float).eps * p[:, None]).all()

@@ -995,15 +995,14 @@ ZFV_HD void hllc(const double *uL, const double *uR, const double *n, double gam
   for (int k = 0; k < NV; ++k) uK[k] = left ? uL[k] : uR[k];
   euler_flux<DIM>(uK, K, n, nf);
   if (sL < 0.0 && 0.0 <= sR) {
-    // the star state: cK = (sK - vK) / (sK - s_star) times (rho, m + rho
-    // (s_star - vK) n, E + (s_star - vK) (rho s_star + pK / (sK - vK)))
+    // sK times the star state's difference from the cell's, with w = (s_star -
+    // vK) / (sK - s_star): w (rho, m + rho (sK - vK) n, E + pK + rho (sK - vK)
+    // s_star).  (The star state less the cell's, term by term, cancels.)
     const double sK = left ? sL : sR;
-    const double iK = 1.0 / (sK - s_star);
-    const double cK = (sK - K.vn) * iK, dv = s_star - K.vn;
-    nf[0] += sK * (cK * uK[0] - uK[0]);
-    const double dm = cK * (uK[0] * dv);
-    for (int d = 0; d < DIM; ++d) nf[1 + d] += sK * (cK * uK[1 + d] + dm * n[d] - uK[1 + d]);
-    nf[NV - 1] += sK * (cK * (uK[NV - 1] + dv * (uK[0] * s_star)) + dv * K.p * iK - uK[NV - 1]);
+    const double w = sK * ((s_star - K.vn) / (sK - s_star)), r = uK[0] * (sK - K.vn);
+    nf[0] += w * uK[0];
+    for (int d = 0; d < DIM; ++d) nf[1 + d] += w * (uK[1 + d] + r * n[d]);
+    nf[NV - 1] += w * (uK[NV - 1] + K.p + r * s_star);
   }
 }
 
