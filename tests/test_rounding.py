@@ -91,3 +91,16 @@ def test_hllc_of_a_state_at_rest_is_its_pressure():
     lib.unit_hllc(ctypes.c_double(gamma), n, _ptr(u), _ptr(u), _ptr(nn), _ptr(f))
     assert not f[:, 0].any() and not f[:, 3].any()
     assert (np.abs(f[:, 1:3] - p[:, None] * nn) <= 4 * np.finfo(float).eps * p[:, None]).all()
+
+
+@pytest.mark.parametrize("gamma", [7.0 / 5.0, 5.0 / 3.0, 4.0 / 3.0, 1.5, 2.0, 1.2, 9.0 / 7.0, 11.0 / 9.0, 1.1, 3.0, 1.3])
+def test_equilibrium_power_to_half_a_place(gamma):
+    # as accurate as pow: half a unit in the last place, and 1 % of one beyond
+    # (the powers of 1.4e1 .. 4.5 orders of magnitude, both sides of one)
+    lib = _library("rounding")
+    x = np.exp(np.random.default_rng(5).uniform(-5.0, 5.0, 100000))
+    y = np.empty_like(x)
+    lib.unit_eq_pow(ctypes.c_double(gamma), len(x), _ptr(x), _ptr(y))
+    ref = x.astype(np.longdouble) ** np.longdouble(1.0 / (gamma - 1.0))
+    ulp = np.spacing(ref.astype(float))
+    assert (np.abs(y - ref) <= 0.51 * ulp).all(), float((np.abs(y - ref) / ulp).max())
