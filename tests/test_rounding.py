@@ -37,11 +37,15 @@ def _weno_rusanov(w):
 
 # the root mean square error over the cells and variables, relative to each
 # variable's largest rate, that the plain formulas reach: a division per
-# quotient, the basis functions one by one
+# quotient, the basis functions one by one, the source's face terms in full
+# (weights, point values, HLLC's star state and the face terms have other forms)
 CASES = {
     "vortex_o3": (lambda s: W.vortex_2d(n=16, order=3, beta=3.0 + s, seed=s), 2.26e-15),
     "vortex_o4": (lambda s: W.vortex_2d(n=16, order=4, beta=3.0 + s, seed=s), 2.28e-15),
     "vortex_o3_weno_rusanov": (lambda s: _weno_rusanov(W.vortex_2d(n=16, order=3, beta=3.0 + s, seed=s)), 2.32e-15),
+    "isothermal_o3": (lambda s: W.isothermal_2d(n=14, order=3, amplitude=1e-4, seed=s), 2.47e-11),
+    "isothermal_o4": (lambda s: W.isothermal_2d(n=14, order=4, amplitude=1e-4, seed=s), 4.89e-11),
+    "isentropic_o3": (lambda s: W.isentropic_2d(n=14, order=3, amplitude=1e-4, seed=s), 3.61e-11),
 }
 
 
