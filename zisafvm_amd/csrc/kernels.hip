@@ -1318,6 +1318,13 @@ int create_device(zfv_handle *h) {
   ZFV_API_END
 }
 
+// work is left on the stream (its errors are the synchronisation's to report)
+static bool still_running(hipStream_t s) {
+  if (hipStreamQuery(s) != hipErrorNotReady) return false;
+  (void)hipGetLastError();  // "not ready" is no error of this thread's calls
+  return true;
+}
+
 // L(u) of host buffers, into dudt
 static void rate_of_change(zfv_handle *h, const double *u, double *dudt, Into into) {
   member_settle(h);
@@ -1336,7 +1343,7 @@ static void rate_of_change(zfv_handle *h, const double *u, double *dudt, Into in
   sc.write_rate_only = 1;
   h->L.update(m, UpdateArgs{sc, 0, 0.0, h->X, h->fpv, h->src, h->X, h->host_stage, h->X}, h->stream);
   HIP_CHECK(hipGetLastError());
-  map_pages(dudt, 5 * size_t(n));
+  map_pages(dudt, 5 * size_t(n), into == Into::Add, [&] { return still_running(h->stream); });
   HIP_CHECK(hipStreamSynchronize(h->stream));
   from_cells(h->img, h->host_stage, dudt, into);
 }
@@ -1376,7 +1383,7 @@ int zfv_get_state(zfv_handle *h, double *cvars) {
   member_settle(h);
   const size_t bytes = sizeof(double) * h->img.s.nvars * h->img.n;
   HIP_CHECK(hipMemcpyAsync(h->host_stage, h->U, bytes, hipMemcpyDeviceToHost, h->stream));
-  map_pages(cvars, 5 * size_t(h->img.n));
+  map_pages(cvars, 5 * size_t(h->img.n), false, [&] { return still_running(h->stream); });
   HIP_CHECK(hipStreamSynchronize(h->stream));
   from_cells(h->img, h->host_stage, cvars, Into::Set);
   return ZFV_OK;
@@ -1412,7 +1419,7 @@ int zfv_snapshot_end(zfv_handle *h, double *cvars) {
   ZFV_API_BEGIN
   if (!h->snap_pending) throw ZfvError(ZFV_ERR_INVALID, "no snapshot pending");
   h->snap_pending = false;
-  map_pages(cvars, 5 * size_t(h->img.n));
+  map_pages(cvars, 5 * size_t(h->img.n), false, [&] { return still_running(h->copy_stream); });
   HIP_CHECK(hipStreamSynchronize(h->copy_stream));
   from_cells(h->img, h->snap_host, cvars, Into::Set);
   return ZFV_OK;

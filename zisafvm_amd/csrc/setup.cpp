@@ -1280,14 +1280,26 @@ void from_cells_into(const HostImage &img, const double *cells, double *aos, Int
 }
 }  // namespace
 
-void map_pages(double *out, size_t n) {
-  constexpr uintptr_t kPage = 4096;
-  const uintptr_t a = reinterpret_cast<uintptr_t>(out) & ~(kPage - 1);
-  const uintptr_t e = (reinterpret_cast<uintptr_t>(out + n) + kPage - 1) & ~(kPage - 1);
-  if (e - a < 32 * kPage) return;
+void map_pages(double *out, size_t n, bool all, const std::function<bool()> &busy) {
 #if defined(MADV_POPULATE_WRITE)
-  // (an older system refuses it: the pages are then mapped as they are written)
-  (void)madvise(reinterpret_cast<void *>(a), e - a, MADV_POPULATE_WRITE);
+  constexpr uintptr_t kPage = 4096, kPiece = 64 * kPage;
+  uintptr_t a = reinterpret_cast<uintptr_t>(out) & ~(kPage - 1);
+  const uintptr_t e = (reinterpret_cast<uintptr_t>(out + n) + kPage - 1) & ~(kPage - 1);
+  // (an older system refuses the advice: the pages are then mapped as they are written)
+  auto populate = [](uintptr_t from, uintptr_t to) {
+    (void)madvise(reinterpret_cast<void *>(from), to - from, MADV_POPULATE_WRITE);
+  };
+  if (e - a < 32 * kPage) return;
+  if (e - a <= (all ? 2 : 1) * kMapWhole) return populate(a, e);
+  do {
+    const uintptr_t to = std::min(e, (a / kPiece + 1) * kPiece);
+    populate(a, to);
+    a = to;
+  } while (a < e && busy());
+  if (!all) return;
+  const int64_t pieces = int64_t((e - a + kPiece - 1) / kPiece);
+#pragma omp parallel for schedule(dynamic, 1)
+  for (int64_t k = 0; k < pieces; ++k) populate(a + k * kPiece, std::min(e, a + (k + 1) * kPiece));
 #endif
 }
 

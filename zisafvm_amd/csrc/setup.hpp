@@ -3,6 +3,7 @@
 #pragma once
 
 #include <cstdint>
+#include <functional>
 #include <vector>
 
 #include "common.hpp"
@@ -115,11 +116,21 @@ void from_soa(const HostImage &img, const double *soa, double *aos, bool accumul
 void to_cells(const HostImage &img, const double *aos, double *cells);
 enum class Into { Set, Add, FromZero };  // aos = c, aos += c, aos = 0 + c (which turns -0 into 0)
 void from_cells(const HostImage &img, const double *cells, double *aos, Into into);
-// Has the pages of a caller's output array of n doubles mapped, its contents
-// unchanged, in one call while the device computes or copies.  Left to the
-// threads that write the array, a fresh one's page faults are waited for
-// afterwards and take longer the more threads meet: 661 pages 5 ms from 16
-// threads, 0.6-3.6 ms from one, 0.2 ms here (0.06 ms where they are mapped already).
-void map_pages(double *out, size_t n);
+// Has pages of a caller's output array of n doubles mapped while the device
+// computes or copies (busy), its contents unchanged: a fresh array's page faults
+// are otherwise waited for afterwards.  Up to kMapWhole bytes all at once (one
+// call takes 90 us a MB of small pages, 50 of huge ones; 16 writing threads that
+// meet their faults take longer: a state of 2.0 MB is read into small pages in
+// 0.24 instead of 0.41 ms, 3.1 MB 0.34 / 0.41).  Larger ones piece by piece as
+// long as the device is busy; the rest is left to the threads that write, which
+// map it faster than one call does (read into small pages: 8.2 MB 0.47 instead
+// of 0.86 ms, 16.3 MB 0.89 / 1.72, 32.8 MB 1.68 / 3.5; huge pages 0.35 / 0.53,
+// 0.58 / 0.84, 1.08 / 1.8; at 4.1 MB both take 0.44).  Where the threads read
+// before they write (all), the rest is mapped by all of them first, beyond twice
+// kMapWhole: a first read costs a page a second fault (a rate added into untouched
+// small pages, one call / piece by piece: 4.1 MB 0.51 / 0.67 ms, 8.2 MB 0.97 /
+// 0.86, 16.3 MB 1.90 / 1.62; nothing mapped ahead 7.2, 7.5 and 14 ms).
+constexpr size_t kMapWhole = 3500000;
+void map_pages(double *out, size_t n, bool all, const std::function<bool()> &busy);
 
 }  // namespace zfv
