@@ -2,10 +2,12 @@
 // Each instance keeps its own arrays; a device table of DevInst describes
 // them, and block tables map every launched block to (instance, local block).
 //
-// The per-block work of the batch kernels is written here once, for the
-// gfx950 kernels (kernels.hip) and for the test-only host emulation, which
-// runs these same functions over the same block tables with bounds-checked
-// host arrays.
+// The block tables, the members' bookkeeping and the reconstruction's per-block
+// work are written here once, for the gfx950 kernels (kernels.hip) and for the
+// test-only host emulation, which runs the same functions over the same block
+// tables with bounds-checked host arrays.  The kernels' update is in update.hpp,
+// which the host's checks run as well; kb_face_flux_thread and kb_update_thread
+// are the emulation's own: one face and one cell at a time, over planes.
 #pragma once
 
 #include <algorithm>
@@ -19,7 +21,7 @@ namespace zfv {
 
 struct DevInst {
   Img m;
-  double *U, *X, *K, *fpv, *G, *src;
+  double *U, *X, *K, *fpv, *G, *src;  // (G, the faces' fluxes: the emulation's)
   double cfl, t, t_end, dt;
   unsigned long long dt_bits;
   int active;
@@ -113,7 +115,7 @@ ZFV_HD void kb_reconstruct_group(const DevInst *insts, BlockRef b, int waves, in
   reconstruct_lane<DIM, DOFC, RC, NB, RB, Q, PH>(d.m, i, g, x, stage == 0 ? d.U : d.X, d.fpv, d.src);
 }
 
-// the face flux of thread t of logical block b (256 faces per block)
+// (emulation) the face flux of thread t of logical block b (256 faces per block)
 template <int DIM, int Q>
 ZFV_HD void kb_face_flux_thread(const DevInst *insts, BlockRef b, int t) {
   if (b.inst < 0) return;
@@ -124,10 +126,10 @@ ZFV_HD void kb_face_flux_thread(const DevInst *insts, BlockRef b, int t) {
   face_flux<DIM, Q>(d.m, e, d.fpv, d.G);
 }
 
-// the SSP3 stage update of thread t's cell (256 cells per block):
+// (emulation) the SSP3 stage update of thread t's cell (256 cells per block):
 // K[stage] = L(U_stage), U_next = U0 + dt sum_j c_j K[j]
 // (src/zisa/ode/runge_kutta.cpp:122-165), then the frozen BC
-template <int DIM, bool AOS = false>
+template <int DIM>
 ZFV_HD void kb_update_thread(DevInst *insts, BlockRef b, int t, int stage) {
   constexpr int NV = DIM + 2;
   if (b.inst < 0) return;
@@ -153,14 +155,14 @@ ZFV_HD void kb_update_thread(DevInst *insts, BlockRef b, int t, int stage) {
   double *Un = stage == 2 ? d.U : d.X;
   if (m.steady != nullptr && (m.meta[i] & META_FAR_GHOST) == META_FAR_GHOST) {
     for (int v = 0; v < NV; ++v) {
-      const int64_t at = state_at<AOS, NV>(n, v, i);
+      const int64_t at = state_at<false, NV>(n, v, i);
       d.K[int64_t(stage) * NV * n + at] = 0.0;
       Un[at] = m.steady[at];
     }
     return;
   }
   double L[NV];
-  cell_rate<DIM, AOS>(m, i, Us, d.G, d.src, L);
+  cell_rate<DIM>(m, i, Us, d.G, d.src, L);
   // SSP3 next-state coefficients (src/zisa/ode/runge_kutta.cpp:154-165)
   const double c0 = stage == 0 ? 1.0 : (stage == 1 ? 0.25 : 1.0 / 6);
   const double c1 = stage == 1 ? 0.25 : 1.0 / 6;
@@ -168,7 +170,7 @@ ZFV_HD void kb_update_thread(DevInst *insts, BlockRef b, int t, int stage) {
   const bool ghost = (m.meta[i] & 16) != 0 && m.steady != nullptr;
   const double *K0 = d.K, *K1 = d.K + int64_t(NV) * n;
   for (int v = 0; v < NV; ++v) {
-    const int64_t at = state_at<AOS, NV>(n, v, i);
+    const int64_t at = state_at<false, NV>(n, v, i);
     if (stage < 2) d.K[int64_t(stage) * NV * n + at] = L[v];  // the last stage's is read by no later one
     double dudt = 0.0;
     if (stage == 0) {

@@ -26,7 +26,7 @@
 
 #include "common.hpp"
 #include "setup.hpp"
-#include "batch.hpp"
+#include "update.hpp"
 #include "stage_math.hpp"
 
 namespace zfv {
@@ -136,228 +136,37 @@ __global__ __launch_bounds__(256, rec_min_waves(PH)) void k_reconstruct(
   }
 }
 
-struct StageCoeffs {
-  double c[2];  // coefficients of the earlier stages' tendencies in the next state's sum
-  double cl;    // and of this stage's own
-  int write_rate_only;  // 1: store L in K[stage] (pinned host memory) and stop (zfv_rate)
-};
-
-// A single instance's time loop on the device (zfv_advance): TimeLoop's
-// step with LocalCFL (src/zisa/fvm_loops/time_loop.cpp:36-81,
-// include/zisa/model/local_cfl_condition_impl.hpp:25-40), dt clamped to the
-// end time as the simulation clock does (its library is not vendored in the
-// reference), with no host round trip per step.
-struct AdvState {
-  double t, t_end, cfl, dt;
-  int steps, max_steps, active;
-  unsigned blocks_done;  // of k_adv_commit
-  // RejectLargeDensityChange (src/zisa/ode/step_rejection.cpp:17-57; off
-  // when drho_crit <= 0): factor scales the CFL step, halves on a rejected
-  // step (which is retried with factor * its dt, TimeLoop::reject_step,
-  // src/zisa/fvm_loops/time_loop.cpp:182-196) and doubles after two good
-  // steps in a row, within [min_factor, 1]
-  double drho_crit, factor, min_factor, retry_dt;
-  int bad, prev_good, retry, rejections;
-};
-
-// The step's CFL minimum is reduced into kAdvSlots words of 128 bytes (one word
-// would serialise thousands of atomics): the last stage's update leaves the new
-// state's minimum there, the next step's first update picks dt from it, and the
-// second stage's update sets the words back.
-constexpr int kAdvSlots = 64, kAdvSlotStride = 16;
-constexpr size_t kAdvSlotBytes = size_t(kAdvSlots) * kAdvSlotStride * sizeof(unsigned long long);
-
-// start value of the CFL reduction (bits of 1e300)
-__host__ __device__ inline unsigned long long adv_no_bound() {
-  const double big = 1.0e300;
-  unsigned long long bits;
-  memcpy(&bits, &big, sizeof(bits));
-  return bits;
-}
-
-// StepRejection::pick_time_step: factor * the CFL step, or the retry step;
-// zero when finished, when the CFL gives no positive step (a non-physical
-// state) or when the step no longer advances the time
-__device__ __forceinline__ double adv_pick(const AdvState &a, double cfl_min) {
-  double dt = a.retry ? a.retry_dt : a.factor * (a.cfl * cfl_min);
-  const double rest = a.t_end - a.t;
-  if (dt > rest) dt = rest;
-  if (!a.active || !(dt > 0.0) || a.t + dt == a.t) dt = 0.0;  // the stages leave U as it is (U + 0 * dudt)
-  return dt;
-}
-
-// the end of a step: the time advances, or the step is to be retried
-__device__ __forceinline__ void adv_end(AdvState *a) {
-  if (!a->active) return;
-  const int bad = a->bad;
-  a->bad = 0;
-  a->retry = 0;
-  if (a->drho_crit > 0.0) {
-    const double f = a->factor;
-    if (bad) {
-      a->prev_good = 0;
-      a->factor = fmax(a->min_factor, fmin(f / 2.0, 1.0));
-      a->retry = 1;
-      a->retry_dt = a->factor * a->dt;
-      a->rejections += 1;
-      return;  // the time does not advance; the state was kept
-    }
-    a->factor = fmax(a->min_factor, fmin(a->prev_good ? f * 2.0 : f, 1.0));
-    a->prev_good = 1;
+// An update wavefront of the device (update_cells): its lanes run side by side,
+// each with its registers.
+struct UpdateWave {
+  int lane;
+  template <class R>
+  using Lanes = R;
+  template <class R, class F>
+  __device__ __forceinline__ void each(R &r, F &&f) {
+    f(lane, r);
   }
-  a->t += a->dt;
-  a->steps += 1;
-  if (a->t >= a->t_end || a->steps >= a->max_steps) a->active = 0;
-}
-
-// What the last stage's update also does in a time loop that chooses its steps:
-// the new state's CFL minimum goes to cfl[slot] (null: not wanted), a density
-// change of more than crit times its old value in any cell sets *bad (crit 0:
-// not asked)
-struct UpdateChecks {
-  unsigned long long *cfl;
-  double crit;
-  int *bad;
+  __device__ __forceinline__ void sync() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+  }
+  // the least of the lanes' values, for every lane
+  template <class F>
+  __device__ __forceinline__ double least(F &&f) {
+    double r = f(lane);
+    for (int off = 32; off > 0; off >>= 1) r = fmin(r, __shfl_xor(r, off, 64));
+    return r;
+  }
+  // *word becomes the least of the lanes' values and its own (bits of doubles >= 0)
+  template <class F>
+  __device__ __forceinline__ void lower(unsigned long long *word, F &&f) {
+    double r = f(lane);
+    for (int off = 32; off > 0; off >>= 1) r = fmin(r, __shfl_down(r, off, 64));
+    if (lane == 0) atomicMin(word, (unsigned long long)__double_as_longlong(r));
+  }
+  __device__ __forceinline__ void flag(int *word) { atomicOr(word, 1); }
 };
-
-// What a stage's update reads and writes: K[stage] = L(Ustage); Unext = U0 +
-// dt * sum_j c_j K[j] (src/zisa/ode/runge_kutta.cpp:122-143), then FrozenBC for
-// ghost cells.  Ustage, U0 and Unext may name the same buffer (stages 1 and 2
-// read and write the stage state X; a wavefront reads only its own cells'
-// entries, before it writes them), so none of them is declared __restrict__.
-struct UpdateArgs {
-  StageCoeffs sc;
-  int stage;
-  double dt;  // (zfv_advance: chosen on the device)
-  const double *Ustage, *fpv, *src, *U0;
-  double *K, *Unext;
-};
-
-// Cells of an update wavefront: as many as have about 64 faces between them
-// along the cells' Hilbert order (32 triangles 58 on average and 66 at most on
-// the jittered lattices, 20 tetrahedra 62 and 68 in the ball), and of a block
-constexpr int update_cells_of_wave(int dim) { return dim == 2 ? 32 : 20; }
-constexpr int update_cells_of_block(int dim) { return 4 * update_cells_of_wave(dim); }
-
-// The update of a wavefront's tile of cells.  First each lane forms the flux
-// through one of the tile's faces (build_update_tiles; a face between two tiles
-// is evaluated by both, with the same operands in the same order: conservation
-// holds bit for bit), then one lane per cell and variable sums its cell's
-// fluxes, which it reads from LDS (lds: NF CW NV doubles).  Bound by latency:
-// a wavefront is one chain of entry, point values, flux, sum, so everything
-// the sum needs is loaded first.  Against a kernel over faces and one over
-// cells it does without a flux array in memory and takes one launch less:
-// 263,520 triangles (3 points a face) 44 -> 34 us, 201,196 tetrahedra 42 -> 38,
-// 1,152 triangles 9.4 -> 4.8.  (One lane per cell face, every face evaluated
-// twice: 48, 50 and 5.0 us; four wavefronts per SIMD spill in 3D: 54 us.)
-template <int DIM, int Q>
-__device__ __forceinline__ void update_cells(const Img &m, const UpdateArgs &a, double dt, const UpdateChecks &chk, int64_t tile,
-                                             int lane, double *lds) {
-  constexpr int NV = DIM + 2;
-  constexpr int NF = DIM + 1;
-  constexpr int CW = update_cells_of_wave(DIM);
-  constexpr int NP = (CW * NV + 63) / 64;  // passes over the tile's cells and variables
-  const int64_t n = m.n;
-  const int64_t i0 = tile * CW;
-  const UpdateFace mine = reinterpret_cast<const UpdateFace *>(m.uent)[tile * 64 + lane];
-  const int more0 = m.uoff[tile], more1 = m.uoff[tile + 1];
-  // What the second part needs besides the fluxes is loaded first, to be in
-  // flight with the faces' entries and point values
-  double part[NP], base[NP], src[NP], vol[NP];
-  uint32_t word[NP];
-  bool inside[NP], frozen_cell[NP];
-#pragma unroll
-  for (int p = 0; p < NP; ++p) {
-    const int e = p * 64 + lane, c = e / NV;
-    int64_t i = i0 + c;
-    inside[p] = e < CW * NV && i < n;
-    i = inside[p] ? i : i0;
-    const int64_t at = i * NV + (e - c * NV);
-    const int32_t meta = m.meta[i];
-    word[p] = m.ucell[i];
-    vol[p] = m.vol[i];
-    src[p] = m.gravity != 0 && a.src != nullptr ? a.src[at] : 0.0;
-    part[p] = base[p] = 0.0;
-    if (!a.sc.write_rate_only) {
-      base[p] = a.U0[at];
-#pragma unroll
-      for (int j = 0; j < 2; ++j)
-        if (j < a.stage && a.sc.c[j] != 0.0) part[p] += a.sc.c[j] * a.K[int64_t(j) * NV * n + at];
-    }
-    // frozen ghost cells keep the steady state whatever their fluxes
-    frozen_cell[p] = !a.sc.write_rate_only && (meta & 16) != 0 && m.steady != nullptr;
-    if (frozen_cell[p]) base[p] = m.steady[at];
-  }
-  UpdateFace face = mine;
-  for (int k = lane; face.l >= 0;) {
-    double g[NV];
-    update_face_flux<DIM, Q>(m, face, a.Ustage, a.fpv, g);
-#pragma unroll
-    for (int v = 0; v < NV; ++v) lds[k * NV + v] = g[v];
-    k += 64;  // (tiles of more than 64 faces)
-    if (k >= 64 + more1 - more0) break;
-    face = reinterpret_cast<const UpdateFace *>(m.umore)[more0 + k - 64];
-  }
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-#pragma unroll
-  for (int p = 0; p < NP; ++p) {
-    if (!inside[p]) continue;
-    const int e = p * 64 + lane, v = e % NV;
-    const int64_t at = i0 * NV + e;
-    // RejectLargeDensityChange::check: |rho1 - rho0| > crit rho0
-    auto check = [&](double r0, double r1) {
-      if (chk.crit > 0.0 && v == 0 && fabs(r0 - r1) > chk.crit * r0) atomicOr(chk.bad, 1);
-    };
-    if (frozen_cell[p]) {
-      if (chk.crit > 0.0) check(a.U0[at], base[p]);
-      a.Unext[at] = base[p];
-      continue;
-    }
-    double L = 0.0;
-#pragma unroll
-    for (int f = 0; f < NF; ++f) {
-      const uint32_t k = (word[p] >> (8 * f)) & 127u;
-      const bool right = (word[p] >> (8 * f)) & 128u;
-      if (k != UPDATE_NO_FACE) {
-        const double g = lds[k * NV + v];
-        L += right ? g : -g;
-      }
-    }
-    L = L / vol[p];
-    if (m.gravity != 0 && a.src != nullptr) L += src[p];
-    // the last stage's tendency enters only its own sum (no later stage reads it)
-    if (a.sc.write_rate_only || a.stage < 2) a.K[int64_t(a.stage) * NV * n + at] = L;
-    if (a.sc.write_rate_only) continue;
-    const double un = base[p] + dt * (part[p] + a.sc.cl * L);
-    check(base[p], un);
-    base[p] = un;
-    a.Unext[at] = un;
-  }
-  if (chk.cfl == nullptr) return;
-  // the CFL minimum of the new state: its values go through LDS to one lane a cell
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-#pragma unroll
-  for (int p = 0; p < NP; ++p)
-    if (p * 64 + lane < CW * NV) lds[p * 64 + lane] = base[p];
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-  double r = 1.0e300;
-  if (lane < CW && i0 + lane < n) r = cfl_of_cell<DIM>(lds + lane * NV, m.inr[i0 + lane], m.gamma);
-  for (int off = 32; off > 0; off >>= 1) r = fmin(r, __shfl_down(r, off, 64));
-  if (lane == 0) atomicMin(chk.cfl, (unsigned long long)__double_as_longlong(r));
-}
-
-// The cells that a stage's update covers: under the frozen BC the second leaves
-// out the ghosts away from the interior, whose X the first has set (the third
-// sets U)
-__host__ __device__ inline int64_t update_cells_of_stage(const Img &m, const UpdateArgs &a) {
-  return !a.sc.write_rate_only && m.steady != nullptr && a.stage == 1 && m.n_near > 0 ? m.n_near : m.n;
-}
 
 template <int DIM, int Q>
 __global__ __launch_bounds__(256, 3) void k_update(Img m, UpdateArgs a) {
@@ -365,39 +174,19 @@ __global__ __launch_bounds__(256, 3) void k_update(Img m, UpdateArgs a) {
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int64_t tile = xcd_block(blockIdx.x, gridDim.x) * 4 + wave;
   if (tile * update_cells_of_wave(DIM) >= update_cells_of_stage(m, a)) return;
-  update_cells<DIM, Q>(m, a, a.dt, UpdateChecks{nullptr, 0.0, nullptr}, tile, threadIdx.x & 63, flux[wave]);
+  UpdateWave w{int(threadIdx.x & 63)};
+  update_cells<DIM, Q>(m, a, a.dt, UpdateChecks{nullptr, 0.0, nullptr}, tile, flux[wave], w);
 }
 
-// the update inside the time loop of zfv_advance, with its bookkeeping: the
-// first stage picks the step's dt (every wavefront for itself, the first one
-// for the record), the second sets the CFL words back and, without step
-// rejection, advances the time, the third reduces the next step's CFL minimum
+// the update inside the time loop of zfv_advance, with its bookkeeping
 template <int DIM, int Q>
 __global__ __launch_bounds__(256, 3) void k_update_adv(Img m, UpdateArgs a, AdvState *adv, unsigned long long *slots) {
   __shared__ double flux[4][update_cells_of_wave(DIM) * (DIM + 1) * (DIM + 2)];
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int lane = threadIdx.x & 63;
   const int64_t tile = xcd_block(blockIdx.x, gridDim.x) * 4 + wave;
   if (tile * update_cells_of_wave(DIM) >= update_cells_of_stage(m, a)) return;
-  double dt;
-  if (a.stage == 0) {
-    double r = __longlong_as_double((long long)slots[lane * kAdvSlotStride]);
-    for (int off = 32; off > 0; off >>= 1) r = fmin(r, __shfl_xor(r, off, 64));
-    dt = adv_pick(*adv, r);
-    if (tile == 0 && lane == 0) {
-      adv->dt = dt;
-      if (!(dt > 0.0)) adv->active = 0;
-    }
-  } else {
-    dt = adv->dt;
-    if (a.stage == 1 && tile == 0) {
-      slots[lane * kAdvSlotStride] = adv_no_bound();
-      if (lane == 0 && !(adv->drho_crit > 0.0)) adv_end(adv);
-    }
-  }
-  UpdateChecks chk{nullptr, 0.0, nullptr};
-  if (a.stage == 2) chk = UpdateChecks{slots + (tile & (kAdvSlots - 1)) * kAdvSlotStride, adv->drho_crit, &adv->bad};
-  update_cells<DIM, Q>(m, a, dt, chk, tile, lane, flux[wave]);
+  UpdateWave w{int(threadIdx.x & 63)};
+  update_cells_adv<DIM, Q>(m, a, adv, slots, tile, flux[wave], w);
 }
 
 // LocalCFL: min_i inradius_i / (|v_i| + a_i); positive doubles order like
@@ -520,8 +309,8 @@ constexpr int64_t kBatchMaxCells = 65536;
 constexpr int32_t kBatchMaxMembers = 8;
 
 // ---------------------------------------------------------------------------
-// Batched execution (the per-block work is in batch.hpp, shared with the host
-// emulation of the tests).  The graph of one step is captured once for the
+// Batched execution (the per-block work is in batch.hpp and update.hpp, which
+// host checks run too).  The graph of one step is captured once for the
 // batch's capacity; adding or removing instances only rewrites the device
 // tables between replays.  Block tables already place neighbouring blocks on
 // one XCD, so the kernels index them by blockIdx directly.
@@ -561,38 +350,13 @@ __global__ __launch_bounds__(256, 3) void kb_update(DevInst *insts, const BlockR
   if (b.inst < 0) return;
   DevInst &d = insts[b.inst];                   // the loop state
   const DevInst &c = unchanging(insts)[b.inst];  // the rest: mesh, arrays
-  if (!d.active) return;
-  UpdateArgs a;
-  a.sc = sc;
-  a.stage = stage;
-  a.dt = 0.0;
-  double dt = d.dt;
-  const bool first = b.local == 0 && threadIdx.x == 0;
-  if (stage == 0) {
-    // the step's dt, from the CFL minimum of the member's state: every thread
-    // of the member forms the same value; the member's first thread records
-    // it for the later stages (and stops a member that cannot advance or has
-    // finished, whose threads all leave here)
-    dt = kb_step_dt(d);
-    if (first) kb_begin_instance(d, dt);
-    if (!(dt > 0.0)) return;
-  } else {
-    if (!d.running) return;
-    // the time and the CFL minimum are not read before the next step's first
-    // stage but by the last stage's reduction
-    if (stage == 1 && first) kb_end_instance(d);
-  }
-  a.Ustage = stage == 0 ? c.U : c.X;
-  a.fpv = c.fpv;
-  a.src = c.src;
-  a.U0 = c.U;
-  a.K = c.K;
-  a.Unext = stage == 2 ? c.U : c.X;
+  double dt;
+  if (!kb_update_begin(d, stage, b.local == 0 && threadIdx.x == 0, dt)) return;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int64_t tile = int64_t(b.local) * 4 + wave;
   if (tile * update_cells_of_wave(DIM) >= c.m.n) return;
-  update_cells<DIM, Q>(c.m, a, dt, UpdateChecks{stage == 2 ? &d.dt_bits : nullptr, 0.0, nullptr}, tile,
-                       threadIdx.x & 63, flux[wave]);
+  UpdateWave w{int(threadIdx.x & 63)};
+  update_cells<DIM, Q>(c.m, kb_update_args(c, sc, stage), dt, kb_update_checks(d, stage), tile, flux[wave], w);
 }
 
 template <int DIM>
@@ -648,14 +412,6 @@ __global__ __launch_bounds__(256) void k_copy_probe(const double2 *__restrict__ 
 
 // ---------------------------------------------------------------------------
 // launch plan for one shape
-
-static StageCoeffs ssp3_coeffs(int stage) {
-  // next-state coefficients after stage s: a[s+1][:] and b for the last stage
-  // (src/zisa/ode/runge_kutta.cpp:154-165)
-  if (stage == 0) return StageCoeffs{{0.0, 0.0}, 1.0, 0};
-  if (stage == 1) return StageCoeffs{{0.25, 0.0}, 0.25, 0};
-  return StageCoeffs{{1.0 / 6, 1.0 / 6}, 2.0 / 3, 0};
-}
 
 struct Launcher {
   // rec[ph]: physics set ph (PH_LIGHT / PH_FULL / PH_LIN); cfg: reconstruction

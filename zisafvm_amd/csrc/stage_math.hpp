@@ -589,6 +589,7 @@ ZFV_HD void store_cell_phi(const Img &m, int64_t i, double *tab) {
   }
   for (int k = 0; k < DIM + 1; ++k) tab[i * (DIM + 1) + k] = p[k];
 }
+// (the emulation's name for it)
 template <int DIM>
 ZFV_HD void store_corner_phi(const Img &m, int64_t i, double *tab) { store_cell_phi<DIM>(m, i, tab); }
 
@@ -2163,8 +2164,9 @@ ZFV_HD void update_face_flux(const Img &m, const UpdateFace &u, const double *__
 }
 
 // ---- the per-cell rate of change -------------------------------------------------
-// L = -(1/vol) sum_faces (+-) |face| R^T G  (+ source) (+ flux BC)
-template <int DIM, bool AOS = false>
+// (emulation) L = -(1/vol) sum of the cell's fluxes (+ source) (+ flux BC), over
+// planes and stored fluxes
+template <int DIM>
 ZFV_HD void cell_rate(const Img &m, int64_t i, const double *__restrict__ U, const double *__restrict__ G,
                       const double *__restrict__ src, double *L) {
   constexpr int NV = DIM + 2;
@@ -2186,7 +2188,7 @@ ZFV_HD void cell_rate(const Img &m, int64_t i, const double *__restrict__ U, con
       const double sgn = (cf & 1) ? 1.0 : -1.0;
       for (int v = 0; v < NV; ++v) g[v] = sgn * G[v * m.ne + (cf >> 2)];
     } else {
-      boundary_flux<DIM, AOS>(m, i, f, U, g);
+      boundary_flux<DIM, false>(m, i, f, U, g);
       for (int v = 0; v < NV; ++v) g[v] = -1.0 * g[v];
     }
     for (int v = 0; v < NV; ++v) acc[v] += g[v];
@@ -2194,7 +2196,7 @@ ZFV_HD void cell_rate(const Img &m, int64_t i, const double *__restrict__ U, con
   const double vol = m.vol[i];
   for (int v = 0; v < NV; ++v) L[v] = acc[v] / vol;
   if (m.gravity != 0 && src != nullptr)
-    for (int v = 0; v < NV; ++v) L[v] += src[state_at<AOS, NV>(n, v, i)];
+    for (int v = 0; v < NV; ++v) L[v] += src[state_at<false, NV>(n, v, i)];
 }
 
 }  // namespace zfv
