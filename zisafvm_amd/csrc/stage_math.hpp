@@ -1108,9 +1108,9 @@ ZFV_HD int p_onesided(int gpw, int nc, int rc, int nbc, int nb, int rb, int kb, 
 }
 
 // linear isentropic equilibria: the part 4 v / r^2 up to which the solve starts
-// from the root.  (Up to 0.03 the iteration from the guess was never seen to
-// fail or to end elsewhere, for 2e5 random states with the reference potential
-// up to six standard deviations off its mean; above it sometimes fails.)
+// from the root.  (Up to here the iteration from the guess leads to that root for
+// 6e5 random states, the reference potential up to six standard deviations off
+// its mean; from 0.032 on some do not converge.)
 constexpr double kRootsApart = 0.02;
 
 template <int DIM, int DOFC, int RC, int NB, int RB, int Q, int PH, class X>
@@ -1361,7 +1361,8 @@ ZFV_HD void reconstruct_lane(const Img &m, int64_t i, const int g, X &xch, const
       // apart the iteration from the guess leads there; it starts from the root
       // instead and ends after the step that confirms it, one step for about
       // four (7,000 of the 66,000 cycles a wavefront of the polytrope n = 40
-      // spends; reconstruction 119 -> 113 us a launch).  Near a double root and without one it starts from the guess.
+      // spends; reconstruction 119 -> 113 us a launch).  Near a double root and
+      // without one it starts from the guess.
       if (PH == PH_LIN) {
         const double v = m.phim[2 * i + 1], r = guess[0], disc = r * r - 4.0 * v;
         if (r > 0.0 && 4.0 * v <= kRootsApart * (r * r)) {
