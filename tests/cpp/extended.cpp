@@ -96,8 +96,11 @@ void run(const Img &m, int ph, const real *U, real *fpv, real *src, real *L) {
 
 extern "C" {
 
-// dudt (n x 5, caller order) = L(u); -1: no such kernel shape or parameters
-int ext_rate(const zfv_mesh *mesh, const zfv_params *p, const double *u, long double *dudt) {
+// dudt (n x 5, caller order) = L(u); -1: no such kernel shape or parameters.
+// series: the isothermal averages in series form, as the device has them, where
+// the cell's exponents are in range (else an exponential per point throughout);
+// the least and the largest part of the range that a cell's need go to range.
+int ext_rate(const zfv_mesh *mesh, const zfv_params *p, const double *u, long double *dudt, int series, double *range) {
   HostImage im;
   zfv::build_image(*mesh, *p, im);
   const Shape &s = im.s;
@@ -166,6 +169,27 @@ int ext_rate(const zfv_mesh *mesh, const zfv_params *p, const double *u, long do
     real *cphi = room(size_t(3) * n);
     for (int64_t i = 0; i < n; ++i) store_cell_phi<2>(m, i, cphi);
     m.cphi = cphi;
+    if (series && exp_average_constants(m, m.es)) {
+      m.phi_unshifted = 1;
+      for (real v : m.shift_phi) m.phi_unshifted &= v == 0;
+      for (int64_t i = 0; i < n; ++i) {
+        m.es_p2 = std::max(m.es_p2, m.cphi[3 * i + 1]);
+        for (int r = 0; r < s.nrows; ++r) {
+          const int32_t e = m.rows[r * n + i];
+          m.es_dist = std::max(m.es_dist, std::fabs(m.cphi[3 * int64_t(e & ROW_CELL_MASK)] +
+                                                    m.shift_phi[e >> ROW_CELL_BITS] - m.cphi[3 * i]));
+        }
+      }
+      range[0] = 1e300;
+      range[1] = 0.0;
+      for (int64_t i = 0; i < n; ++i) {
+        const double *a = u + 5 * int64_t(im.perm[i]);
+        const real RT = (p->gamma - 1.0) * (a[4] - 0.5 * (a[1] * a[1] + a[2] * a[2]) / a[0]) / a[0];
+        const double part = double(std::max(m.es_dist / (kSeriesMaxArg * RT), std::sqrt(m.es_p2 / (kSeriesMaxY2 * RT * RT))));
+        range[0] = std::min(range[0], part);
+        range[1] = std::max(range[1], part);
+      }
+    }
   }
   real *src = nullptr;
   if (m.gravity != 0) {

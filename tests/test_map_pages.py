@@ -18,9 +18,8 @@ PAGE, PIECE = 4096, 64 * 4096
 
 
 @pytest.fixture(scope="module")
-def lib():
-    out = os.path.join(HERE, "cpp", "build", "pages.so")
-    os.makedirs(os.path.dirname(out), exist_ok=True)
+def lib(tmp_path_factory):
+    out = str(tmp_path_factory.mktemp("pages") / "pages.so")
     subprocess.run(["g++", "-O2", "-std=c++17", "-fPIC", "-fopenmp", "-w", "-shared", "-o", out,
                     os.path.join(HERE, "cpp", "pages.cpp"), os.path.join(CSRC, "setup.cpp"),
                     os.path.join(CSRC, "mesh.cpp")], check=True)

@@ -11,23 +11,31 @@ import pytest
 import zisafvm_amd as z
 from zisafvm_amd import workloads as W
 from emu_binding import Emu
+from conftest import pressure_scale
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(os.path.dirname(HERE), "zisafvm_amd", "csrc")
-BUILD = os.path.join(HERE, "cpp", "build")
 
 
-def _library(name, *more):
-    os.makedirs(BUILD, exist_ok=True)
-    out = os.path.join(BUILD, name + ".so")
+def _ptr(a):
+    return ctypes.c_void_p(a.ctypes.data)
+
+
+def _library(folder, name, *more):
+    out = str(folder / (name + ".so"))
     subprocess.run(["g++", "-O2", "-std=c++17", "-fPIC", "-fopenmp", "-ffp-contract=off", "-w", "-shared", "-o", out,
                     os.path.join(HERE, "cpp", name + ".cpp")] + [os.path.join(CSRC, m) for m in more], check=True)
     return ctypes.CDLL(out)
 
 
 @pytest.fixture(scope="module")
-def extended():
-    return _library("extended", "setup.cpp", "mesh.cpp")
+def extended(tmp_path_factory):
+    return _library(tmp_path_factory.mktemp("extended"), "extended", "setup.cpp", "mesh.cpp")
+
+
+@pytest.fixture(scope="module")
+def units(tmp_path_factory):
+    return _library(tmp_path_factory.mktemp("rounding"), "rounding")
 
 
 def _weno_rusanov(w):
@@ -57,8 +65,7 @@ def _check(extended, make, name):
         u = np.ascontiguousarray(w.u0)
         ref = np.zeros(u.shape, dtype=np.longdouble)
         mesh = w.mesh.c_struct()
-        assert extended.ext_rate(ctypes.byref(mesh), ctypes.byref(w.params), ctypes.c_void_p(u.ctypes.data),
-                                 ctypes.c_void_p(ref.ctypes.data)) == 0
+        assert extended.ext_rate(ctypes.byref(mesh), ctypes.byref(w.params), _ptr(u), _ptr(ref), 0, None) == 0
         got = make(w.mesh, w.params).rate(u)
         keep = np.ix_(w.mesh.ghost == 0, [0, 1, 2, 4])
         errs.append(float((((got - ref)[keep] / np.abs(ref[keep]).max(axis=0)) ** 2).mean()))
@@ -78,13 +85,35 @@ def test_rate_on_the_device_rounds_no_worse_than_the_plain_formulas(gpu, extende
     _check(extended, z.Solver, name)
 
 
-def _ptr(a):
-    return ctypes.c_void_p(a.ctypes.data)
+@pytest.mark.parametrize("order,RT", [(3, 4.0), (3, 0.74), (3, 0.72), (3, 0.5), (4, 4.0), (4, 0.74)])
+def test_series_averages_leave_out_less_than_rounding(extended, order, RT):
+    # inside the range, at its edge, across it and outside, in 80-bit arithmetic:
+    # the terms left out of the averages (1e-17) and of the exponentials near
+    # them (3e-18) times the largest pressures, against the pressures that cancel
+    mesh = z.lattice_mesh_2d(10, jitter=0.2, seed=4, periodic=(True, False), ghost_layers=3)
+    p = z.make_params(n_dims=2, order=order, equilibrium=z.ZFV_EQ_ISOTHERMAL, gravity=z.ZFV_GRAVITY_AXIAL, gravity_g=1.0)
+    if order == 4:
+        p.edge_deg = 4
+
+    def f(x):
+        rho = np.exp(-x[:, 1] / RT)
+        return W.conserved(rho, 0.1 * rho, 0.0 * rho, 0.0 * rho,
+                           RT * rho * (1.0 + 1e-2 * np.sin(6.28 * x[:, 0])), 1.4)
+
+    u = np.ascontiguousarray(W.cell_average(mesh, f))
+    cm, both, part = mesh.c_struct(), [], np.zeros(2)
+    for series in (0, 1):
+        out = np.zeros(u.shape, dtype=np.longdouble)
+        assert extended.ext_rate(ctypes.byref(cm), ctypes.byref(p), _ptr(u), _ptr(out), series, _ptr(part)) == 0
+        both.append(out)
+    diff = np.abs(both[1] - both[0])[mesh.ghost == 0].max() / pressure_scale(mesh, u, 1.4)
+    print("order", order, "RT", RT, "part of the range", part, "difference", float(diff), flush=True)
+    assert diff <= 1e-16
+    assert (diff > 0.0) == (part[0] <= 1.0)  # the series ran where a cell is in range
 
 
-def test_hllc_of_a_state_at_rest_is_its_pressure():
+def test_hllc_of_a_state_at_rest_is_its_pressure(units):
     # no mass or energy crosses the face, exactly; the pressure to a few places
-    lib = _library("rounding")
     rng = np.random.default_rng(3)
     n, gamma = 20000, 1.4
     p = np.exp(rng.uniform(-3.0, 3.0, n))
@@ -92,19 +121,18 @@ def test_hllc_of_a_state_at_rest_is_its_pressure():
     a = rng.uniform(0.0, 2.0 * np.pi, n)
     nn = np.stack([np.cos(a), np.sin(a)], axis=1)
     f = np.empty((n, 4))
-    lib.unit_hllc(ctypes.c_double(gamma), n, _ptr(u), _ptr(u), _ptr(nn), _ptr(f))
+    units.unit_hllc(ctypes.c_double(gamma), n, _ptr(u), _ptr(u), _ptr(nn), _ptr(f))
     assert not f[:, 0].any() and not f[:, 3].any()
     assert (np.abs(f[:, 1:3] - p[:, None] * nn) <= 4 * np.finfo(float).eps * p[:, None]).all()
 
 
 @pytest.mark.parametrize("gamma", [7.0 / 5.0, 5.0 / 3.0, 4.0 / 3.0, 1.5, 2.0, 1.2, 9.0 / 7.0, 11.0 / 9.0, 1.1, 3.0, 1.3])
-def test_equilibrium_power_to_half_a_place(gamma):
+def test_equilibrium_power_to_half_a_place(units, gamma):
     # as accurate as pow: half a unit in the last place, and 1 % of one beyond
     # (the powers of 1.4e1 .. 4.5 orders of magnitude, both sides of one)
-    lib = _library("rounding")
     x = np.exp(np.random.default_rng(5).uniform(-5.0, 5.0, 100000))
     y = np.empty_like(x)
-    lib.unit_eq_pow(ctypes.c_double(gamma), len(x), _ptr(x), _ptr(y))
+    units.unit_eq_pow(ctypes.c_double(gamma), len(x), _ptr(x), _ptr(y))
     ref = x.astype(np.longdouble) ** np.longdouble(1.0 / (gamma - 1.0))
     ulp = np.spacing(ref.astype(float))
     assert (np.abs(y - ref) <= 0.51 * ulp).all(), float((np.abs(y - ref) / ulp).max())
