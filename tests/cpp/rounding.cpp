@@ -21,4 +21,20 @@ void unit_hllc(double gamma, int n, const double *uL, const double *uR, const do
   for (int k = 0; k < n; ++k) hllc<2>(uL + 4 * k, uR + 4 * k, nn + 2 * k, gamma, f + 4 * k);
 }
 
+// the kernels' evaluation at the scaled point X of the polynomial of coefficients
+// a over the basis X^alpha - c[alpha]: the moments in the nested form's constant
+// coefficient, the mean beside it
+double unit_poly(int dims, int degree, int dof, const double *a, const double *c, const double *X) {
+  double b[16] = {0};
+  for (int k = 1; k < dof; ++k) b[k] = a[k];
+  for (int k = 1; k < dof; ++k) b[0] -= a[k] * c[k];
+  double r = 0.0;
+  if (dims == 2 && degree == 1) r = poly_nested<2, 1>(b, X);
+  else if (dims == 2 && degree == 2) r = poly_nested<2, 2>(b, X);
+  else if (dims == 2 && degree == 3) r = poly_nested<2, 3>(b, X);
+  else if (dims == 3 && degree == 1) r = poly_nested<3, 1>(b, X);
+  else r = poly_nested<3, 2>(b, X);
+  return a[0] + r;
+}
+
 }  // extern "C"

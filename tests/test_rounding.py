@@ -126,6 +126,22 @@ def test_hllc_of_a_state_at_rest_is_its_pressure(units):
     assert (np.abs(f[:, 1:3] - p[:, None] * nn) <= 4 * np.finfo(float).eps * p[:, None]).all()
 
 
+@pytest.mark.parametrize("dims,degree", [(2, 1), (2, 2), (2, 3), (3, 1), (3, 2)])
+def test_nested_polynomial_is_the_sum_over_the_basis(units, dims, degree):
+    from oracle import zfv_ref as R
+
+    units.unit_poly.restype = ctypes.c_double
+    dof = [1, 3, 6, 10][degree] if dims == 2 else [1, 4, 10][degree]
+    rng = np.random.default_rng(11)
+    for _ in range(50):
+        a, c, X = rng.normal(size=dof), rng.normal(size=dof), np.append(rng.uniform(-2.0, 2.0, dims), [0.0] * (3 - dims))
+        c[:dims + 1] = 0.0
+        ref = R.poly_eval(dims, degree, a[:, None], c, X)[0]
+        # each of the terms and sums of both forms rounds once
+        size = np.abs(a) @ (np.maximum(1.0, np.abs(X).max()) ** degree + np.abs(c))
+        assert abs(units.unit_poly(dims, degree, dof, _ptr(a), _ptr(c), _ptr(X)) - ref) <= 4 * dof * 2.3e-16 * size
+
+
 @pytest.mark.parametrize("gamma", [7.0 / 5.0, 5.0 / 3.0, 4.0 / 3.0, 1.5, 2.0, 1.2, 9.0 / 7.0, 11.0 / 9.0, 1.1, 3.0, 1.3])
 def test_equilibrium_power_to_half_a_place(units, gamma):
     # as accurate as pow: half a unit in the last place, and 1 % of one beyond
