@@ -148,15 +148,16 @@ int zfv_rate_set(zfv_handle *h, const double *u, double *dudt, double t);
  * frozen BC after every stage sum (src/zisa/ode/runge_kutta.cpp:87-112). */
 int zfv_step(zfv_handle *h, double t, double dt);
 
-/* n_steps fixed-dt SSP3 steps replayed from one captured HIP graph. */
+/* n_steps fixed-dt SSP3 steps replayed from captured HIP graphs (of one step,
+ * in long runs of eight). */
 int zfv_steps(zfv_handle *h, int32_t n_steps, double t, double dt);
 
 /* TimeLoop's inner loop on the device (src/zisa/fvm_loops/time_loop.cpp:36-81):
  * from t0, SSP3 steps with dt = cfl_number * LocalCFL (computed on the device,
  * include/zisa/model/local_cfl_condition_impl.hpp:25-40) clamped to t_end,
  * until t_end or max_steps (<= 0: no limit), or until a step would not advance
- * the time (dt not positive or below the resolution of t).  One captured graph per step;
- * the host reads the loop state back every check_every steps (< 1: 16), so a
+ * the time (dt not positive or below the resolution of t).  Steps are replayed
+ * from captured graphs; the host reads the loop state back every check_every steps (< 1: 16), so a
  * finished run may replay up to check_every - 1 steps of dt 0 (no change).
  * drho_crit_rel > 0 turns on RejectLargeDensityChange
  * (src/zisa/ode/step_rejection.cpp:17-57): a step that changes the density of
@@ -249,7 +250,7 @@ int zfv_tune(zfv_handle *h, int32_t rec_threads, zfv_tuning *out);
  * process); each member behaves exactly like its own TimeLoop
  * (src/zisa/fvm_loops/time_loop.cpp:36-75): per step, dt = cfl * LocalCFL
  * clamped to t_end, one SSP3 step with the frozen BC.  All members of a batch
- * advance in one captured HIP graph per step (block tables map launched
+ * advance in the same captured HIP graphs (block tables map launched
  * blocks to members; no per-member launches).  An instance is a member of
  * at most one batch; zfv_destroy of a member removes it from its batch first,
  * zfv_set_steady_state on a member reaches the batch, and a snapshot
@@ -270,7 +271,7 @@ int zfv_batch_destroy(zfv_batch *b);
 int zfv_batch_add(zfv_batch *b, zfv_handle *h, double cfl, double t0, double t_end, int32_t max_steps,
                   int32_t *slot);
 int zfv_batch_remove(zfv_batch *b, int32_t slot);
-/* n_steps graph replays; members that reach t_end / max_steps stop. */
+/* n_steps steps; members that reach t_end / max_steps stop. */
 int zfv_batch_run(zfv_batch *b, int32_t n_steps);
 /* zfv_batch_run in two halves, for callers that keep several batches in
  * flight at once (each batch has its own stream, so batches of different

@@ -5,12 +5,12 @@
 //   k_reconstruct  one group of nvars lanes per cell (lane g: variable g):
 //                  stencil gather, LSQ pseudo-inverse mat-vecs, CWENO/WENO-AO,
 //                  equilibrium solve (well-balanced), point values on the
-//                  cell's faces (face frame), gravity source
-//   k_update       one lane per cell face: HLLC/Rusanov at the face points,
-//                  integrated over the face, in the global frame times the
-//                  face's area; then one lane per cell and variable: the sum
-//                  of the cell's fluxes, source, flux BC, Butcher-form stage
-//                  sum, frozen BC
+//                  cell's faces (global frame), gravity source
+//   k_update       (update.hpp) one lane per distinct face of a tile of cells:
+//                  HLLC/Rusanov at the face points, integrated over the face,
+//                  in the global frame times the face's area; then one lane
+//                  per cell and variable: the sum of the cell's fluxes,
+//                  source, flux BC, Butcher-form stage sum, frozen BC
 // FP64 throughout; no MFMA (every cell has its own matrices: there is no shared
 // operand for a tile, and the matrices' bytes bound the kernel).
 #include <hip/hip_runtime.h>
@@ -535,7 +535,8 @@ namespace zfv {
 // Captured steps: a graph of one step and one of kGraphSteps, which saves 4-5 us
 // a step between graphs (1,152 triangles: 38.0 -> 33.6 us a step) but takes 510
 // instead of 105 us to capture: captured once the steps asked for are as many as
-// pay for it, in one run or in several.
+// pay for it, in one run or in several.  (96 steps of a dt not used before: 3.5 ms
+// with it, 4.1 without; 64 steps 2.8 without.)
 constexpr int kGraphSteps = 8, kLongRun = 96;
 struct StepGraphs {
   hipGraphExec_t one = nullptr, many = nullptr;
@@ -685,13 +686,13 @@ static int frozen(const zfv_handle *h) { return h->dimg.steady != nullptr ? 1 : 
 
 // Autotuner of the reconstruction launch configuration: every candidate (1,
 // 2, 4 waves per block) runs the instance's own state through stages as the
-// steps do (reconstruction, face fluxes, a rate-only update into K[0]), one
+// steps do (reconstruction, a rate-only update into K[0]), one
 // warm-up and four timed stages, the reconstruction alone between HIP events
 // on the handle's stream; the fastest average wins.  (Launched back to back
 // the reconstruction finds the caches as the previous launch left them and
 // runs up to 6% faster than inside a step, enough to reorder close
 // candidates.)  The launches write only scratch buffers: face-point values,
-// source, face fluxes and K[0].
+// source and K[0].
 static void tune_rec(zfv_handle *h, const double *Ustate) {
   const Img m = stateless(h->dimg);
   constexpr int kTimed = 4;
@@ -1280,12 +1281,12 @@ int zfv_advance_noalloc(zfv_handle *h, double cfl_number, double t0, double t_en
   HIP_CHECK(hipGetDevice(&dev));
   if (dev != h->dev) throw ZfvError(ZFV_ERR_INVALID, "zfv_advance_noalloc: make the handle's device current first");
   const bool reject = drho_crit_rel > 0.0;
-  const size_t backup = sizeof(double) * size_t(h->img.s.nvars) * size_t(h->img.n);
-  if (reject && backup > kNoAllocScratchBytes - kNoAllocStateBytes)
-    throw ZfvError(ZFV_ERR_MEMORY, "zfv_advance_noalloc: step rejection backs up the state in " +
-                                       std::to_string((kNoAllocScratchBytes - kNoAllocStateBytes) >> 20) +
-                                       " MiB of scratch; this instance needs " + std::to_string(backup) +
-                                       " bytes (use zfv_advance)");
+  const size_t state_bytes = sizeof(double) * size_t(h->img.s.nvars) * size_t(h->img.n);
+  if (reject && state_bytes > kNoAllocScratchBytes - kNoAllocStateBytes)
+    throw ZfvError(ZFV_ERR_MEMORY, "zfv_advance_noalloc: step rejection is limited to states of at most the " +
+                                       std::to_string(kNoAllocScratchBytes >> 20) + " MiB of scratch less " +
+                                       std::to_string(kNoAllocStateBytes) + " bytes; this instance's has " +
+                                       std::to_string(state_bytes) + " (use zfv_advance)");
   unsigned char *sp = scratch_on(dev);
   AdvState *adv = reinterpret_cast<AdvState *>(sp);
   auto *slots = reinterpret_cast<unsigned long long *>(sp + kNoAllocStateBytes);
@@ -1451,7 +1452,7 @@ int zfv_estimate_device_bytes(const zfv_mesh *mesh, const zfv_params *params, in
   const double frame = s.dim == 2 ? frame_words<2>() : frame_words<3>();
   double per_cell = 8.0 * s.m + 4.0 * s.nrows + 1.0 * (s.nrows - s.rc) +
                     8.0 * ((s.dim == 2 ? 6 : 16) + s.dim + 3 + s.nmom) + 4.0 * (2 + 4) +
-                    8.0 * s.nfaces * frame +    // face frames
+                    8.0 * s.nfaces * frame +    // face normals and areas
                     8.0 * nv * (1 + 1 + 2);     // U, X, K[2]
   if (params->gravity != ZFV_GRAVITY_NONE) {
     per_cell += 8.0 * nv;                       // source

@@ -70,7 +70,7 @@ struct Img {
   const double *steady;  // as the state (ghost cells only are read)
   const double *phim;    // n pairs: cell mean of phi and of (phi - mean)^2 (one 16-byte load), or null
   const double *pot;     // potential tables of the cell's own points (pot_index), or null
-  const double *frm;     // face frames of the cells' local faces (load_face_frame)
+  const double *frm;     // normals and areas of the cells' local faces (load_face_frame)
   const double *ffr;     // per interior face its normal and area (face_table_frame)
   // 3D with an equilibrium: per cell its faces' outward normals times their
   // areas, n x (face 3 + d) (store_face_normals), or null
@@ -812,7 +812,8 @@ ZFV_HD void potential_points(const Img &m, int nqf, int64_t i, double *tab) {
 }
 
 // ---- polynomial evaluation (include/zisa/math/poly2d_impl.hpp:271-323) -------
-// a[alpha][v] for alpha < DOF, c = moments (0 for alpha < 3)
+// a[alpha][v] for alpha < DOF, c = moments (0 for alpha < 3).  (The basis
+// functions one by one, for setup and checks; the kernels use poly_nested.)
 template <int DIM, int DEG, int NV>
 ZFV_HD void poly_eval(const double (*a)[NV], const double *c, const double *X, double *px) {
   for (int v = 0; v < NV; ++v) px[v] = 0.0;
@@ -1049,19 +1050,19 @@ ZFV_HD void rusanov(const double *uL, const double *uR, const double *n, double 
 // Reads the cell's stencil, forms every stencil polynomial with the
 // precomputed pseudo-inverses, applies the CWENO correction and the WENO
 // weights, then evaluates the result at the quadrature points of the cell's
-// interior faces (rotated into each face's frame) and, with gravity, computes
-// the cell's source term.
+// interior faces (in the global frame) and, with gravity, computes the cell's
+// source term.
 //
 // A group of NV lanes shares one cell: lane g owns conserved variable g (rho,
 // momentum components, energy) and keeps only that variable's polynomial
 // coefficients, so a lane needs a fraction of the registers of a whole cell.
 // The lanes exchange values through X::bcast(v, k) / X::bcast_i(v, k) (value
-// v of lane k of the same group) and a per-group LDS slice X::lds() of
-// NV x (DOFC - 1) doubles ordered by X::sync():
+// v of lane k of the same group) and through LDS (X::wave_lds(), X::lds()),
+// ordered by X::sync():
 //   - the equilibrium averages of the stencil members are computed by lane
-//     (row mod NV) and broadcast to the density and energy lanes,
+//     (row mod NV) and read by the density and energy lanes,
 //   - the smoothness indicator of a stencil is the maximum over the variables,
-//   - the face-frame rotation and the gravity source mix momentum components.
+//   - the gravity source mixes momentum components.
 // Every call of bcast sits in control flow that is uniform over the group.
 //
 // U: state (state_at).  fpv: per cell-face slot (i * NF + f) its Q x NV
