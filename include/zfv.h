@@ -280,6 +280,8 @@ int zfv_batch_run(zfv_batch *b, int32_t n_steps);
  * of its members waits for steps in flight first. */
 int zfv_batch_launch(zfv_batch *b, int32_t n_steps);
 int zfv_batch_wait(zfv_batch *b);
+/* dt: the last step's; of a member that stopped because its state gives no
+ * positive step (a non-physical state), that dt, which is not positive. */
 int zfv_batch_query(zfv_batch *b, int32_t slot, double *t, double *dt, int32_t *steps_done, int32_t *active);
 /* Block-to-XCD mapping: 1 (default) gives each XCD a contiguous eighth of the
  * cells so stencil gathers share one L2; 0 is the hardware round robin. */

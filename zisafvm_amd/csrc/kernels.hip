@@ -1620,6 +1620,7 @@ static void member_settle(zfv_handle *h) {
 }
 
 // the members' cells, by slot; ZFV_ERR_MEMORY if their blocks exceed the capacity
+// (in faces too: the caller's limit, though no table is sized by it)
 static std::vector<int64_t> batch_cells(const zfv_batch *b) {
   std::vector<int64_t> cells(b->max_inst, 0);
   int64_t face_blocks = 0;
